@@ -77,15 +77,15 @@ static int upload(spx_plan* p, double** dst, const V& host) {
 // the boundary-plane buffers of mixed plans) and the advect additions
 static void work_sizes(const spx_plan* p, size_t* hd, size_t* bouss) {
   const size_t cb = p->nc * p->nb * p->csize, rb = p->nr * p->nb * p->rsize;
-  size_t h = 3 * (3 * cb + 2 * rb) + p->nr * p->nb * 8;
+  size_t h = 3 * (3 * cb + rb) + p->nr * p->nb * 8;
   if (p->fp32 && p->g.Cz > 0) {
     const size_t d2 = 2 * size_t(p->g.oz), nbm = size_t(p->nb);
     const size_t bc = size_t(p->nkx) * p->g.ny * d2 * nbm * 16;
     const size_t br = size_t(p->g.nx) * p->g.ny * d2 * nbm * 8;
-    h += 16 * bc + 7 * br;
+    h += 16 * bc + 3 * br;
   }
   *hd = h;
-  *bouss = 3 * cb + rb;
+  *bouss = 3 * cb;
 }
 
 // device bytes of one solver state (all members): 10 float64 spectral fields,
@@ -105,15 +105,14 @@ static int ensure_work(spx_plan* p, bool bouss) {
   if (!p->XV[0]) {
     for (int c = 0; c < 3; ++c) {
       if ((rc = alloc_dev(p, &p->XV[c], cb)) || (rc = alloc_dev(p, &p->XZ[c], cb)) ||
-          (rc = alloc_dev(p, &p->XY[c], cb)) || (rc = alloc_dev(p, &p->RV[c], rb)) ||
-          (rc = alloc_dev(p, &p->RO[c], rb)))
+          (rc = alloc_dev(p, &p->XY[c], cb)) || (rc = alloc_dev(p, &p->RV[c], rb)))
         return rc;
     }
     if ((rc = alloc_dev(p, &p->R0, p->nr * p->nb * 8))) return rc;
   }
   if (bouss && !p->work_bouss) {
     if ((rc = alloc_dev(p, &p->XV[3], cb)) || (rc = alloc_dev(p, &p->XZ[3], cb)) ||
-        (rc = alloc_dev(p, &p->XY[3], cb)) || (rc = alloc_dev(p, &p->RO[3], rb)))
+        (rc = alloc_dev(p, &p->XY[3], cb)))
       return rc;
     p->work_bouss = true;
   }
@@ -123,7 +122,7 @@ static int ensure_work(spx_plan* p, bool bouss) {
     const size_t br = size_t(p->g.nx) * p->g.ny * d2 * nbm * 8;
     if ((rc = alloc_dev(p, &p->XVb, 4 * bc)) || (rc = alloc_dev(p, &p->XZb, 4 * bc)) ||
         (rc = alloc_dev(p, &p->XYb, 4 * bc)) || (rc = alloc_dev(p, &p->RVb, 3 * br)) ||
-        (rc = alloc_dev(p, &p->ROb, 4 * br)) || (rc = alloc_dev(p, &p->XFb, 4 * bc)))
+        (rc = alloc_dev(p, &p->XFb, 4 * bc)))
       return rc;
   }
   return SPX_OK;
@@ -140,21 +139,21 @@ static inline void* bnd_r(const spx_plan* p, void* base, int c) {
 }
 
 // 3D transforms on internal buffers -------------------------------------------
-// lo: float32 buffers and kernels of a mixed plan (X holds float32 data then);
-// xb: float64 boundary planes for the continuation (mixed plans)
-static int r2c3(spx_plan* p, const void* in, void* out, bool lo = false,
-                const void* xb = nullptr) {
+// one field at a time through p->X
+static int r2c3(spx_plan* p, const void* in, void* out) {
   int rc;
-  if ((rc = xr2c(p, in, p->X, p->np, lo))) return rc;
-  if ((rc = yfft(p, p->X, 1, p->np, nullptr, nullptr, lo, p->Cy > 0))) return rc;
-  return zfft_x2s(p, p->X, out, 0, lo, xb);
+  if ((rc = xr2c(p, 1, &in, &p->X, p->np))) return rc;
+  const void* x = p->X;
+  if ((rc = yfft(p, 1, &x, &p->X, 1, p->np, nullptr, false, p->Cy > 0))) return rc;
+  return zfft_x2s(p, 1, &x, &out, 0);
 }
 
 static int c2r3(spx_plan* p, const void* in, void* out, int dirn, int nplanes) {
   int rc;
-  if ((rc = zfft_s2x(p, in, p->X, dirn, nplanes, 0))) return rc;
-  if ((rc = yfft(p, p->X, 0, nplanes))) return rc;
-  return xc2r(p, p->X, out, nplanes);
+  const void* x = p->X;
+  if ((rc = zfft_s2x(p, 1, &in, &p->X, dirn, nplanes, 0))) return rc;
+  if ((rc = yfft(p, 1, &x, &p->X, 0, nplanes))) return rc;
+  return xc2r(p, 1, &x, &out, nplanes);
 }
 
 // ---- MHD building blocks -----------------------------------------------------
@@ -166,6 +165,48 @@ static int ensure_mhd_work(spx_plan* p) {
   return SPX_OK;
 }
 
+// nf physical-plane transforms, as many fields per launch as there are
+// xy-stage buffers: the plan's X, and the work arrays of the nonlinear term
+// once a solver state has allocated them
+static int mhd_buffers(spx_plan* p, void** xs) {
+  if (!p->XV[0] || p->fp32) {
+    xs[0] = p->X;
+    return 1;
+  }
+  for (int c = 0; c < 3; ++c) {
+    xs[c] = p->XV[c];
+    xs[3 + c] = p->XZ[c];
+  }
+  return 6;
+}
+
+static int c2r3_n(spx_plan* p, int nf, const void* const* in, void* const* out) {
+  void* xs[6];
+  const int nbuf = mhd_buffers(p, xs);
+  int rc;
+  for (int c = 0; c < nf; c += nbuf) {
+    const int m = std::min(nbuf, nf - c);
+    if ((rc = zfft_s2x(p, m, in + c, xs, 0, p->np, 0)) ||
+        (rc = yfft(p, m, xs, xs, 0, p->np)) || (rc = xc2r(p, m, xs, out + c, p->np)))
+      return rc;
+  }
+  return SPX_OK;
+}
+
+static int r2c3_n(spx_plan* p, int nf, void* const* in, void* const* out) {
+  void* xs[6];
+  const int nbuf = mhd_buffers(p, xs);
+  int rc;
+  for (int c = 0; c < nf; c += nbuf) {
+    const int m = std::min(nbuf, nf - c);
+    if ((rc = xr2c(p, m, in + c, xs, p->np)) ||
+        (rc = yfft(p, m, xs, xs, 1, p->np, nullptr, false, p->Cy > 0)) ||
+        (rc = zfft_x2s(p, m, xs, out + c, 0)))
+      return rc;
+  }
+  return SPX_OK;
+}
+
 // real values (physical planes, members of the view packed) of A and B, then
 // out = A x B through real space (pseudospec_hd.f90:383-399, pseudospec_mhd.f90
 // vector).  RA / RB receive the real fields unless have_a / have_b say they
@@ -173,16 +214,21 @@ static int ensure_mhd_work(spx_plan* p) {
 static int cross_spec(spx_plan* p, const void* const* A, const void* const* B, void* const* out,
                       void* const* RA, void* const* RB, void* const* RO, bool have_a,
                       bool have_b) {
-  int rc;
-  for (int c = 0; c < 3 && !have_a; ++c)
-    if ((rc = c2r3(p, A[c], RA[c], 0, p->np))) return rc;
-  for (int c = 0; c < 3 && !have_b; ++c)
-    if ((rc = c2r3(p, B[c], RB[c], 0, p->np))) return rc;
+  int rc, nf = 0;
+  const void* in[6];
+  void* real[6];
+  for (int c = 0; c < 3 && !have_a; ++c, ++nf) {
+    in[nf] = A[c];
+    real[nf] = RA[c];
+  }
+  for (int c = 0; c < 3 && !have_b; ++c, ++nf) {
+    in[nf] = B[c];
+    real[nf] = RB[c];
+  }
+  if (nf && (rc = c2r3_n(p, nf, in, real))) return rc;
   const long n = long(p->g.nx) * p->g.ny * p->np * p->mem;
   if ((rc = op_cross_real(p, RA, RB, RO, n))) return rc;
-  for (int c = 0; c < 3; ++c)
-    if ((rc = r2c3(p, RO[c], out[c]))) return rc;
-  return SPX_OK;
+  return r2c3_n(p, 3, RO, out);
 }
 
 // sol_project with the condition on the potential (bctarget 0; wall kinds
@@ -632,9 +678,11 @@ int spx_fftp2d_real_to_complex_xy(spx_plan* p, const void* in, void* out) {
   MemberView mv(p, 1);
   int rc;
   for (int b = 0; b < p->nact; ++b) {
-    if ((rc = xr2c(p, roff(in, p->nr, b), p->X, p->g.nz))) return rc;
-    if ((rc = yfft(p, p->X, 1, p->g.nz))) return rc;
-    if ((rc = zfft_x2s(p, p->X, coff(out, p->nc, b), 1))) return rc;
+    const void *r = roff(in, p->nr, b), *x = p->X;
+    void* o = coff(out, p->nc, b);
+    if ((rc = xr2c(p, 1, &r, &p->X, p->g.nz))) return rc;
+    if ((rc = yfft(p, 1, &x, &p->X, 1, p->g.nz))) return rc;
+    if ((rc = zfft_x2s(p, 1, &x, &o, 1))) return rc;
   }
   return SPX_OK;
 }
@@ -644,9 +692,11 @@ int spx_fftp2d_complex_to_real_xy(spx_plan* p, void* in, void* out) {
   MemberView mv(p, 1);
   int rc;
   for (int b = 0; b < p->nact; ++b) {
-    if ((rc = zfft_s2x(p, coff(in, p->nc, b), p->X, 0, p->g.nz, 1))) return rc;
-    if ((rc = yfft(p, p->X, 0, p->g.nz))) return rc;
-    if ((rc = xc2r(p, p->X, roff(out, p->nr, b), p->g.nz))) return rc;
+    const void *c = coff(in, p->nc, b), *x = p->X;
+    void* o = roff(out, p->nr, b);
+    if ((rc = zfft_s2x(p, 1, &c, &p->X, 0, p->g.nz, 1))) return rc;
+    if ((rc = yfft(p, 1, &x, &p->X, 0, p->g.nz))) return rc;
+    if ((rc = xc2r(p, 1, &x, &o, p->g.nz))) return rc;
   }
   return SPX_OK;
 }
@@ -658,8 +708,10 @@ int spx_fftp1d_real_to_complex_x(spx_plan* p, const void* in, void* out) {
   MemberView mv(p, 1);
   int rc;
   for (int b = 0; b < p->nact; ++b) {
-    if ((rc = xr2c(p, roff(in, p->nr, b), p->X, p->g.nz))) return rc;
-    if ((rc = zfft_x2s(p, p->X, coff(out, p->nc, b), 1))) return rc;
+    const void *r = roff(in, p->nr, b), *x = p->X;
+    void* o = coff(out, p->nc, b);
+    if ((rc = xr2c(p, 1, &r, &p->X, p->g.nz))) return rc;
+    if ((rc = zfft_x2s(p, 1, &x, &o, 1))) return rc;
   }
   return SPX_OK;
 }
@@ -673,9 +725,10 @@ int spx_fftp2d_real_to_complex_yz(spx_plan* p, void* s) {
   // commute with each other
   for (int b = 0; b < p->nact; ++b) {
     void* sb = coff(s, p->nc, b);
-    if ((rc = zfft_s2x(p, sb, p->X, 0, p->np, 1))) return rc;
-    if ((rc = yfft(p, p->X, 1, p->np, nullptr, nullptr, false, p->Cy > 0))) return rc;
-    if ((rc = zfft_x2s(p, p->X, sb, 0))) return rc;
+    const void *cs = sb, *x = p->X;
+    if ((rc = zfft_s2x(p, 1, &cs, &p->X, 0, p->np, 1))) return rc;
+    if ((rc = yfft(p, 1, &x, &p->X, 1, p->np, nullptr, false, p->Cy > 0))) return rc;
+    if ((rc = zfft_x2s(p, 1, &x, &sb, 0))) return rc;
   }
   return SPX_OK;
 }
@@ -686,9 +739,10 @@ int spx_fftp2d_complex_to_real_yz(spx_plan* p, void* s) {
   int rc;
   for (int b = 0; b < p->nact; ++b) {
     void* sb = coff(s, p->nc, b);
-    if ((rc = zfft_s2x(p, sb, p->X, 0, p->g.nz, 0))) return rc;
-    if ((rc = yfft(p, p->X, 0, p->g.nz))) return rc;
-    if ((rc = zfft_x2s(p, p->X, sb, 1))) return rc;
+    const void *cs = sb, *x = p->X;
+    if ((rc = zfft_s2x(p, 1, &cs, &p->X, 0, p->g.nz, 0))) return rc;
+    if ((rc = yfft(p, 1, &x, &p->X, 0, p->g.nz))) return rc;
+    if ((rc = zfft_x2s(p, 1, &x, &sb, 1))) return rc;
   }
   return SPX_OK;
 }
@@ -698,8 +752,10 @@ int spx_fftp1d_complex_to_real_x(spx_plan* p, const void* in, void* out) {
   MemberView mv(p, 1);
   int rc;
   for (int b = 0; b < p->nact; ++b) {
-    if ((rc = zfft_s2x(p, coff(in, p->nc, b), p->X, 0, p->g.nz, 1))) return rc;
-    if ((rc = xc2r(p, p->X, roff(out, p->nr, b), p->g.nz))) return rc;
+    const void *c = coff(in, p->nc, b), *x = p->X;
+    void* o = roff(out, p->nr, b);
+    if ((rc = zfft_s2x(p, 1, &c, &p->X, 0, p->g.nz, 1))) return rc;
+    if ((rc = xc2r(p, 1, &x, &o, p->g.nz))) return rc;
   }
   return SPX_OK;
 }
@@ -746,102 +802,104 @@ int spx_fc_filter(spx_plan* p, void* a) {
 
 namespace spx {
 
-// (v.grad) v_c for c = x,y,z in advective form (pseudospec_hd.f90:209-319).
+// (v.grad) v_c for c = x,y,z in advective form (pseudospec_hd.f90:209-319)
+// and, with th, (v.grad) th (pseudospec_phd.f90:23-113).
 // The x and y derivatives commute with the z transform (kx, ky are constant
-// along a z line), so each component needs two z IFFTs (v and d_z v) instead
+// along a z line), so each field needs two z IFFTs (v and d_z v) instead
 // of four; the y pass yields v and d_y v from one load; the x pass forms the
-// three derivatives and accumulates the products in the reference's order.
+// three derivatives, accumulates the products in the reference's order and
+// takes their half spectra.  Every pass is one launch over the three or four
+// fields: z, y, x, y, z.
 // In mixed plans the whole pipeline runs in float32: the first z pass reads
 // the float64 state and the outputs are float32.
-int gradre_impl(spx_plan* p, const void* const v[3], void* const out[3], bool keep_rv) {
+int gradre_impl(spx_plan* p, const void* const v[3], const void* th, void* const* out) {
   int rc;
-  const int np = p->np;
+  const int np = p->np, nf = th ? 4 : 3;
   const bool lo = p->fp32;
-  for (int c = 0; c < 3; ++c)
-    if ((rc = zfft_s2x(p, v[c], p->XV[c], 0, np, 0, p->XZ[c], lo))) return rc;
-  for (int c = 0; c < 3; ++c) {
-    if ((rc = yfft(p, p->XV[c], 0, np, nullptr, p->XY[c], lo))) return rc;
-    if ((rc = yfft(p, p->XZ[c], 0, np, nullptr, nullptr, lo))) return rc;
+  const void* in[4] = {v[0], v[1], v[2], th};
+  if ((rc = zfft_s2x(p, nf, in, p->XV, 0, np, 0, p->XZ, lo))) return rc;
+  void* yf[8];
+  void* y2[8];
+  for (int c = 0; c < nf; ++c) {
+    yf[c] = p->XV[c];
+    y2[c] = p->XY[c];
+    yf[nf + c] = p->XZ[c];
+    y2[nf + c] = nullptr;
   }
-  rc = p->xfused ? xgrad_fused(p, p->XV, p->XY, p->XZ, keep_rv ? p->RV : nullptr, p->RO, lo)
+  if ((rc = yfft(p, 2 * nf, yf, yf, 0, np, y2, lo))) return rc;
+  rc = p->xfused ? xgrad_fused(p, nf, p->XV, p->XY, p->XZ, nullptr, p->XY, lo)
                  : SPX_ERR_UNSUPPORTED;
-  if (rc != SPX_OK && rc != SPX_ERR_UNSUPPORTED) return rc;
   if (rc == SPX_ERR_UNSUPPORTED) {
-    for (int c = 0; c < 3; ++c)
-      if ((rc = xc2r(p, p->XV[c], p->RV[c], np, 0, lo))) return rc;
-    for (int c = 0; c < 3; ++c)
-      if ((rc = xgrad_prod(p, p->XV[c], p->XY[c], p->XZ[c], p->RV[0], p->RV[1], p->RV[2],
-                           p->RO[c], lo)))
-        return rc;
+    if ((rc = xc2r(p, 3, p->XV, p->RV, np, 0, lo))) return rc;
+    rc = xgrad_prod(p, nf, p->XV, p->XY, p->XZ, p->RV, p->XY, lo);
   }
+  if (rc) return rc;
+  if ((rc = yfft(p, nf, p->XY, p->XY, 1, np, nullptr, lo, p->Cy > 0))) return rc;
   const bool bnd = lo && p->g.Cz > 0;
-  const int d2 = 2 * p->g.oz;
+  const void* xf[4] = {nullptr, nullptr, nullptr, nullptr};
   if (bnd) {
     // float64 boundary planes: z IFFT at the 2d planes, y and x passes and
-    // products there, forward x, y passes (three components per launch)
+    // products there, forward x, y passes (all components per launch)
+    const int d2 = 2 * p->g.oz;
     ProfTag tag(p->prof, "_bnd");
-    if ((rc = zfft_s2x_bnd(p, v, 3, p->XVb, p->XZb))) return rc;
-    if ((rc = yfft(p, p->XVb, 0, 3 * d2, nullptr, p->XYb))) return rc;
-    if ((rc = yfft(p, p->XZb, 0, 3 * d2))) return rc;
-    if ((rc = xc2r(p, p->XVb, p->RVb, 3 * d2, 0))) return rc;
-    if ((rc = xgrad_prod(p, p->XVb, p->XYb, p->XZb, bnd_r(p, p->RVb, 0), bnd_r(p, p->RVb, 1),
-                         bnd_r(p, p->RVb, 2), p->ROb, false, d2, 3)))
-      return rc;
-    if ((rc = xr2c(p, p->ROb, p->XFb, 3 * d2))) return rc;
-    if ((rc = yfft(p, p->XFb, 1, 3 * d2))) return rc;
+    if ((rc = zfft_s2x_bnd(p, in, nf, p->XVb, p->XZb))) return rc;
+    void* yb[2] = {p->XVb, p->XZb};
+    void* yb2[2] = {p->XYb, nullptr};
+    if ((rc = yfft(p, 2, yb, yb, 0, nf * d2, yb2))) return rc;
+    const void* xvb = p->XVb;
+    if ((rc = xc2r(p, 1, &xvb, &p->RVb, 3 * d2, 0))) return rc;
+    const void *bv[4], *by[4], *bz[4], *bu[3];
+    void* bo[4];
+    for (int c = 0; c < nf; ++c) {
+      bv[c] = bnd_c(p, p->XVb, c);
+      by[c] = bnd_c(p, p->XYb, c);
+      bz[c] = bnd_c(p, p->XZb, c);
+      xf[c] = bo[c] = bnd_c(p, p->XFb, c);
+      if (c < 3) bu[c] = bnd_r(p, p->RVb, c);
+    }
+    if ((rc = xgrad_prod(p, nf, bv, by, bz, bu, bo, false, d2))) return rc;
+    const void* xfb = p->XFb;
+    if ((rc = yfft(p, 1, &xfb, &p->XFb, 1, nf * d2))) return rc;
   }
-  for (int c = 0; c < 3; ++c)
-    if ((rc = r2c3(p, p->RO[c], out[c], lo, bnd ? bnd_c(p, p->XFb, c) : nullptr))) return rc;
-  return SPX_OK;
+  return zfft_x2s(p, nf, p->XY, out, 0, lo, bnd ? xf : nullptr);
 }
 
-// (v.grad) th (pseudospec_phd.f90:23-113); have_rv: RV already holds v in
-// real space (computed by gradre_impl on the same v).
-static int advect_impl(spx_plan* p, const void* const v[3], const void* th, void* out,
-                       bool have_rv) {
+// (v.grad) th (pseudospec_phd.f90:23-113) on its own
+static int advect_impl(spx_plan* p, const void* const v[3], const void* th, void* out) {
   int rc;
   const int np = p->np;
   const bool lo = p->fp32;
   const bool bnd = lo && p->g.Cz > 0;
   const int d2 = 2 * p->g.oz;
-  if (!have_rv) {
-    for (int c = 0; c < 3; ++c) {
-      if ((rc = zfft_s2x(p, v[c], p->XV[c], 0, np, 0, nullptr, lo))) return rc;
-      if ((rc = yfft(p, p->XV[c], 0, np, nullptr, nullptr, lo))) return rc;
-      if ((rc = xc2r(p, p->XV[c], p->RV[c], np, 0, lo))) return rc;
-    }
-    if (bnd) {
-      ProfTag tag(p->prof, "_bnd");
-      if ((rc = zfft_s2x_bnd(p, v, 3, p->XVb, p->XZb))) return rc;
-      if ((rc = yfft(p, p->XVb, 0, 3 * d2))) return rc;
-      if ((rc = xc2r(p, p->XVb, p->RVb, 3 * d2, 0))) return rc;
-    }
-  }
+  if ((rc = zfft_s2x(p, 3, v, p->XV, 0, np, 0, nullptr, lo))) return rc;
+  if ((rc = zfft_s2x(p, 1, &th, p->XV + 3, 0, np, 0, p->XZ + 3, lo))) return rc;
+  void* yf[5] = {p->XV[0], p->XV[1], p->XV[2], p->XV[3], p->XZ[3]};
+  void* y2[5] = {nullptr, nullptr, nullptr, p->XY[3], nullptr};
+  if ((rc = yfft(p, 5, yf, yf, 0, np, y2, lo))) return rc;
+  if ((rc = xc2r(p, 3, p->XV, p->RV, np, 0, lo))) return rc;
+  if ((rc = xgrad_prod(p, 1, p->XV + 3, p->XY + 3, p->XZ + 3, p->RV, p->XY + 3, lo))) return rc;
+  if ((rc = yfft(p, 1, p->XY + 3, p->XY + 3, 1, np, nullptr, lo, p->Cy > 0))) return rc;
+  const void* xf = nullptr;
   if (bnd) {
-    // the scalar's float64 boundary planes (component slot 3)
     ProfTag tag(p->prof, "_bnd");
-    const void* ths[1] = {th};
-    void* xv3 = bnd_c(p, p->XVb, 3);
+    const void* in[4] = {v[0], v[1], v[2], th};
+    if ((rc = zfft_s2x_bnd(p, in, 4, p->XVb, p->XZb))) return rc;
     void* xz3 = bnd_c(p, p->XZb, 3);
-    void* xy3 = bnd_c(p, p->XYb, 3);
-    if ((rc = zfft_s2x_bnd(p, ths, 1, xv3, xz3))) return rc;
-    if ((rc = yfft(p, xv3, 0, d2, nullptr, xy3))) return rc;
-    if ((rc = yfft(p, xz3, 0, d2))) return rc;
-    if ((rc = xgrad_prod(p, xv3, xy3, xz3, bnd_r(p, p->RVb, 0), bnd_r(p, p->RVb, 1),
-                         bnd_r(p, p->RVb, 2), bnd_r(p, p->ROb, 3), false, d2)))
-      return rc;
-    if ((rc = xr2c(p, bnd_r(p, p->ROb, 3), bnd_c(p, p->XFb, 3), d2))) return rc;
-    if ((rc = yfft(p, bnd_c(p, p->XFb, 3), 1, d2))) return rc;
+    void* yb[3] = {p->XVb, bnd_c(p, p->XVb, 3), xz3};
+    void* yb2[3] = {nullptr, bnd_c(p, p->XYb, 3), nullptr};
+    if ((rc = yfft(p, 1, yb, yb, 0, 3 * d2))) return rc;
+    if ((rc = yfft(p, 2, yb + 1, yb + 1, 0, d2, yb2 + 1))) return rc;
+    const void* xvb = p->XVb;
+    if ((rc = xc2r(p, 1, &xvb, &p->RVb, 3 * d2, 0))) return rc;
+    const void *bv = yb[1], *by = yb2[1], *bz = xz3;
+    const void* bu[3] = {bnd_r(p, p->RVb, 0), bnd_r(p, p->RVb, 1), bnd_r(p, p->RVb, 2)};
+    void* bo = bnd_c(p, p->XFb, 3);
+    if ((rc = xgrad_prod(p, 1, &bv, &by, &bz, bu, &bo, false, d2))) return rc;
+    xf = bo;
+    if ((rc = yfft(p, 1, &xf, &bo, 1, d2))) return rc;
   }
-  if ((rc = zfft_s2x(p, th, p->XV[3], 0, np, 0, p->XZ[3], lo))) return rc;
-  if ((rc = yfft(p, p->XV[3], 0, np, nullptr, p->XY[3], lo))) return rc;
-  if ((rc = yfft(p, p->XZ[3], 0, np, nullptr, nullptr, lo))) return rc;
-  if ((rc = xgrad_prod(p, p->XV[3], p->XY[3], p->XZ[3], p->RV[0], p->RV[1], p->RV[2],
-                       p->RO[3], lo)))
-    return rc;
-  return r2c3(p, p->RO[3], out, lo, bnd ? bnd_c(p, p->XFb, 3) : nullptr);
+  return zfft_x2s(p, 1, p->XY + 3, &out, 0, lo, bnd ? &xf : nullptr);
 }
-
 }  // namespace spx
 
 extern "C" {
@@ -854,7 +912,7 @@ int spx_gradre(spx_plan* p, const void* a, const void* b, const void* c, void* d
   MemberView mv(p, p->nact);
   const void* v[3] = {a, b, c};
   void* o[3] = {d, e, f};
-  return gradre_impl(p, v, o, false);
+  return gradre_impl(p, v, nullptr, o);
 }
 
 int spx_advect(spx_plan* p, const void* a, const void* b, const void* c, const void* dd,
@@ -864,7 +922,7 @@ int spx_advect(spx_plan* p, const void* a, const void* b, const void* c, const v
   if ((rc = ensure_work(p, true))) return rc;
   MemberView mv(p, p->nact);
   const void* v[3] = {a, b, c};
-  return advect_impl(p, v, dd, e, false);
+  return advect_impl(p, v, dd, e);
 }
 
 // ---- boundary conditions --------------------------------------------------------
@@ -1422,9 +1480,8 @@ static int substep_impl(spx_plan* p, spx_state* s, int o, bool full_pressure) {
   int rc;
   MemberView mv(p, p->nact);
   const void* vel[3] = {s->vx, s->vy, s->vz};
-  void* nlo[3] = {s->N[0], s->N[1], s->N[2]};
-  if ((rc = gradre_impl(p, vel, nlo, bouss))) return rc;
-  if (bouss && (rc = advect_impl(p, vel, s->th, s->N[3], true))) return rc;
+  void* nlo[4] = {s->N[0], s->N[1], s->N[2], s->N[3]};
+  if ((rc = gradre_impl(p, vel, bouss ? s->th : nullptr, nlo))) return rc;
   // rotating frame: 2 Omega x v joins the nonlinear term before the buoyancy
   // and the filter (include/rotbouss/rotbouss_rkstep2.f90:13-21)
   if (rot && (rc = op_coriolis(p, nlo, vel, q.omega, p->fp32))) return rc;

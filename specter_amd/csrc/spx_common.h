@@ -179,13 +179,12 @@ struct spx_plan {
   // scratch
   void* X = nullptr;        // xy-stage buffer, nc float64 complex
   // gradre / advect work arrays (allocated on first use, csize / rsize elements):
-  //   XV[c]: z+y inverse transform of v_c, XZ[c]: of d_z v_c, XY[c]: y-derivative stage
-  //   RV[c]: v_c in real space, RO[0..3]: nonlinear products (x,y,z, scalar)
+  //   XV[c]: z+y inverse transform of v_c, XZ[c]: of d_z v_c, XY[c]: y-derivative stage,
+  //   then the x half spectra of the nonlinear products; RV[c]: v_c in real space
   void* XV[4] = {nullptr};
   void* XZ[4] = {nullptr};
   void* XY[4] = {nullptr};
   void* RV[3] = {nullptr};
-  void* RO[4] = {nullptr};
   void* R0 = nullptr;       // general real scratch (Boussinesq round trip)
   // MHD: real work fields (physical planes of every member), allocated on
   // first use by prodre / vector / the MHD stage; Neumann vectors neu
@@ -200,8 +199,7 @@ struct spx_plan {
   void* XZb = nullptr;      // of d_z v_c
   void* XYb = nullptr;      // of d_y v_c
   void* RVb = nullptr;      // v_c in real space (3 components)
-  void* ROb = nullptr;      // products (4 components)
-  void* XFb = nullptr;      // forward x, y transforms of the products (4 components)
+  void* XFb = nullptr;      // forward x, then y transforms of the products (4 components)
   void* d_wbnd = nullptr;   // exp(+2 pi i k / nz), then exp(+2 pi i k (np-d) / nz)
   void* d_wtop = nullptr;   // exp(+2 pi i k (np-1) / nz): the top wall of sol_project
   void* DS = nullptr;       // diagnostics scratch: spectral (nb members), allocated on use
@@ -320,39 +318,43 @@ void free_line_fft(LineFFTHost& f);
 int zfft_inplace(spx_plan* p, void* S, int forward, int cont, double scale);
 // the continuation loop alone (fftp.fpp:755-773), in place on S
 int fc_continue_only(spx_plan* p, void* S);
+// The x, y and z passes take up to eight fields per launch (arrays of pointers).
 // forward 3D last pass: X (planes k < np) -> continuation -> z FFT -> S.
 // nofft = 1: transpose only (all nz planes), for fftp2d_real_to_complex_xy.
 // Xb (mixed plans, float32 X): float64 boundary planes [member][q][ky][kx], q < 2d,
 // that replace X's planes z = 0..d-1, np-d..np-1 and feed the continuation.
-int zfft_x2s(spx_plan* p, const void* X, void* S, int nofft, bool lo = false,
-             const void* Xb = nullptr);
+int zfft_x2s(spx_plan* p, int nf, const void* const* X, void* const* S, int nofft,
+             bool lo = false, const void* const* Xb = nullptr);
 // float64 z IFFT of S (and of (i kz) S) at the 2d boundary planes of every
 // line, for ncomp float64 spectral inputs: XVb / XZb planes [comp][member][q][ky][kx].
 int zfft_s2x_bnd(spx_plan* p, const void* const* S, int ncomp, void* XVb, void* XZb);
 // backward 3D first pass: S * (i k_dir) (dir 0 = none) -> z IFFT -> X, planes < nzout.
 // X2 != nullptr: also X2 <- z IFFT of (i kz) S from the same load (dual).
-int zfft_s2x(spx_plan* p, const void* S, void* X, int dir, int nzout, int nofft,
-             void* X2 = nullptr, bool lo = false);
-// y transform of X planes < nplanes: Xout <- y FFT(Xin) (in place when equal);
-// Y2 != nullptr: also Y2 <- y FFT of (i ky) Xin (dual, backward only).
+int zfft_s2x(spx_plan* p, int nf, const void* const* S, void* const* X, int dir, int nzout,
+             int nofft, void* const* X2 = nullptr, bool lo = false);
+// y transform of planes < nplanes: out <- y FFT(in) (in place when equal);
+// Y2 != nullptr (backward only): also Y2[c] <- y FFT of (i ky) in[c] for the
+// fields with Y2[c] != nullptr.
 // cont (forward, plans with Cy > 0): FC-Gram continuation of every y line
 // before the FFT (rows ny-Cy.. from the first and last oy physical rows).
-int yfft(spx_plan* p, void* X, int forward, int nplanes, const void* Xin = nullptr,
-         void* Y2 = nullptr, bool lo = false, bool cont = false);
-int xr2c(spx_plan* p, const void* R, void* X, int nplanes, bool lo = false);
+int yfft(spx_plan* p, int nf, const void* const* in, void* const* out, int forward, int nplanes,
+         void* const* Y2 = nullptr, bool lo = false, bool cont = false);
+int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
+         bool lo = false);
 // x half complex -> real of planes < nplanes; dirx = 1 multiplies by i kx first.
-int xc2r(spx_plan* p, const void* X, void* R, int nplanes, int dirx = 0, bool lo = false);
-// gradient products of one component: out = ((u*Dx + v*Dy) + w*Dz)*tmp with
-// Dx = c2r(i kx YV), Dy = c2r(YY), Dz = c2r(XZ) (pseudospec_hd.f90:254-312 order)
-// ncomp > 1: components stored back to back (YV/YY/XZ blocks of nkx*ny*nplanes*mem
-// complex, out blocks of nx*ny*nplanes*mem real), one launch
-int xgrad_prod(spx_plan* p, const void* YV, const void* YY, const void* XZ, const void* u,
-               const void* v, const void* w, void* out, bool lo = false, int nplanes = -1,
-               int ncomp = 1);
-// the three components' x stage in one launch on the np planes: RV = c2r(YV)
-// (stored only when RV is given) and out_c as xgrad_prod, bit for bit
-int xgrad_fused(spx_plan* p, void* const* YV, void* const* YY, void* const* XZ, void* const* RV,
-                void* const* out, bool lo);
+int xc2r(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes, int dirx = 0,
+         bool lo = false);
+// x stage of up to four fields: out[c] <- r2c(((u*Dx + v*Dy) + w*Dz)*tmp) with
+// vel = (u, v, w) real, Dx = c2r(i kx YV[c]), Dy = c2r(YY[c]), Dz = c2r(XZ[c])
+// (pseudospec_hd.f90:254-312 order); out[c] may be YY[c]
+int xgrad_prod(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
+               const void* const* XZ, const void* const* vel, void* const* out, bool lo = false,
+               int nplanes = -1);
+// the same on the np planes of three velocity components (and a scalar,
+// nf = 4) with vel = c2r(YV[0..2]) formed in the same launch and stored to RV
+// when given; x lengths of a power of two, SPX_ERR_UNSUPPORTED otherwise
+int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
+                void* const* RV, void* const* out, bool lo);
 // fused v_imposebc: goto_domain_w_boundaries + noslip_z + goto_3d_fourier on vx,vy
 // rk: the RK update of vx, vy (c[0], c[1]) is applied on load (null: none)
 // Launch-shape overrides set by an autotuner (spx_tune_*), consulted when a
@@ -406,9 +408,9 @@ struct LinComb {
   int sgn[3];    // +1 / -1 for terms 1,2 (term 0 always +1); 0 = term absent
 };
 // gradre (pseudospec_hd.f90:209-319) through the plan's current work arrays
-// XV, XZ, XY, RV, RO (and the boundary-plane buffers of mixed plans); keep_rv:
-// leave v in real space in RV (advect on the same v reuses it)
-int gradre_impl(spx_plan* p, const void* const v[3], void* const out[3], bool keep_rv = true);
+// XV, XZ, XY, RV (and the boundary-plane buffers of mixed plans); th given:
+// also advect (pseudospec_phd.f90:23-113) of th into out[3]
+int gradre_impl(spx_plan* p, const void* const v[3], const void* th, void* const* out);
 
 int zline_sumsq(spx_plan* p, const LinComb& lc, double* line_out);
 int zline_dot(spx_plan* p, const void* a, const void* b, double* line_out);

@@ -113,22 +113,26 @@ __device__ __forceinline__ void lds_to_global(int first, int step, int count, Rd
   }
 }
 
-// XCD-aware tile order of a 2D grid.  Workgroups are handed to the 8 XCDs
-// (each with its own L2) round-robin by linear id; the kx tiles of the
-// transposing kernels are narrower than a cache line, so neighbouring tiles
-// must meet in one L2.  Each XCD gets a contiguous range of logical tiles
-// (a bijection on [0, gx*gy)): returns the logical (x, y) of this workgroup.
-__device__ __forceinline__ void xcd_tile(int& bx, int& by) {
-  constexpr int X = 8;
-  const int gx = gridDim.x;
-  const int n = gx * gridDim.y;
-  const int pid = blockIdx.x + gx * blockIdx.y;
-  const int q = n / X, r = n % X;
-  const int x = pid % X, slot = pid / X;
-  const int l = x * q + (x < r ? x : r) + slot;
-  by = l / gx;
-  bx = l - by * gx;
+// XCD-aware order of the tiles along gridDim.x.  Workgroups are handed to the
+// 8 XCDs (each with its own L2) round-robin by linear id; the tiles of the
+// transposing kernels are about as wide as a cache line and not aligned to
+// one, so neighbouring tiles must meet in one L2.  Each XCD gets a contiguous
+// range of logical tiles (a bijection on [0, gridDim.x)).
+__device__ __forceinline__ unsigned xcd_tile() {
+  constexpr unsigned X = 8;
+  const unsigned n = gridDim.x, pid = blockIdx.x;
+  const unsigned q = n / X, r = n % X;
+  const unsigned x = pid % X, slot = pid / X;
+  return x * q + (x < r ? x : r) + slot;
 }
+
+// Up to kMaxComp fields of one launch (blockIdx.y selects): the components
+// of a vector field go through one launch, so a small grid fills the GPU and
+// a stage has a third of the launches.  With the products' half spectra taken
+// in the x stage (24 launches per HD stage before, 9 now) an RK2 step of 32^3
+// takes 318 us instead of 529, Boussinesq 128^3 RK4 4.01 ms instead of 4.98,
+// MHD 128^3 RK2 3.42 ms instead of 4.21, HD 256^3 RK4 14.6 ms instead of 15.4.
+constexpr int kMaxComp = 8;
 
 // ---------------------------------------------------------------------------
 // z transforms in place on S (contiguous lines)
@@ -195,38 +199,46 @@ __global__ void k_fc_continue(cpx<T>* __restrict__ S, long nlines, int n, int np
 // ---------------------------------------------------------------------------
 // forward 3D last pass: X(kx,y,z) planes < np -> continuation -> z FFT -> S(z,y,kx)
 // blockIdx.z = member: S advances by n*ny*nkx, X by xstride elements per member.
+// The lines of a workgroup are nl consecutive (kx, y) points e = kx + nkx*y of
+// a plane, whatever nkx is: tiles over kx alone left 15 of 32 lines of a
+// 17-point row (nx = 32) empty, 3 of 36 of a 33-point one.
 // ---------------------------------------------------------------------------
+template <typename T>
+struct ZX2S {
+  const cpx<T>* x[kMaxComp];
+  cpx<T>* s[kMaxComp];
+  const cpx<double>* xb[kMaxComp];
+};
+
 // BND (mixed plans): the 2d boundary planes z = 0..d-1, np-d..np-1 come in
-// float64 from Xb (planes [member][q][ky][kx], q < 2d) and the continuation
+// float64 from xb (planes [member][q][ky][kx], q < 2d) and the continuation
 // is evaluated from them, so the float32 roundoff of the other planes is not
 // amplified by the continuation.
 template <typename T, int RS, bool BND>
-__global__ void __launch_bounds__(kMaxBlock) k_z_x2s(const cpx<T>* __restrict__ X, cpx<T>* __restrict__ S,
-                                               LineFFT<cpx<T>> f, int nkx, int ny, int np,
-                                               int nofft, const double* __restrict__ dir, int C,
-                                               int d, long xstride,
-                                               const cpx<double>* __restrict__ Xb) {
+__global__ void __launch_bounds__(kMaxBlock) k_z_x2s(ZX2S<T> a, LineFFT<cpx<T>> f, int nkx,
+                                               int ny, int np, int nofft,
+                                               const double* __restrict__ dir, int C, int d,
+                                               long xstride) {
   using Cp = cpx<T>;
   SPX_PROLOGUE(Cp, f);
   const int n = f.n;
-  X += blockIdx.z * xstride;
-  S += blockIdx.z * (long(n) * ny * nkx);
-  int bx, j;
-  xcd_tile(bx, j);
-  const int i0 = bx * f.nl;
-  const int nload = nofft ? n : np;
   const long pl = long(nkx) * ny;
+  const Cp* __restrict__ X = a.x[blockIdx.y] + blockIdx.z * xstride;
+  Cp* __restrict__ S = a.s[blockIdx.y] + blockIdx.z * (pl * n);
+  const int e0 = int(xcd_tile()) * f.nl;
+  const int nlines = int(pl);
+  const int nload = nofft ? n : np;
   {
-    const int l = tid & (f.nl - 1), i = i0 + l;
+    const int l = tid & (f.nl - 1), e = e0 + l;
     if constexpr (RS >= RS_WAVE) {
-      // compiled plans (tpl 64, n <= KN*tpl): the thread's loads in flight together
+      // compiled plans (n <= KN*tpl): the thread's loads in flight together
       constexpr int KN = keep_n<RS>();
       Cp v[KN];
 #pragma unroll
       for (int q = 0; q < KN; ++q) {
         const int k = (tid >> f.lgnl) + q * f.tpl;
         v[q] = mkc<T>(0, 0);
-        if (i < nkx && k < nload) v[q] = X[i + long(nkx) * j + pl * k];
+        if (e < nlines && k < nload) v[q] = X[e + pl * k];
       }
 #pragma unroll
       for (int q = 0; q < KN; ++q) {
@@ -236,7 +248,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_x2s(const cpx<T>* __restrict__ 
     } else {
       for (int k = tid >> f.lgnl; k < nload; k += f.tpl) {
         Cp v = mkc<T>(0, 0);
-        if (i < nkx) v = X[i + long(nkx) * j + pl * k];
+        if (e < nlines) v = X[e + pl * k];
         lds[l * f.ldl + k] = v;
       }
     }
@@ -246,39 +258,35 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_x2s(const cpx<T>* __restrict__ 
     if constexpr (BND) {
 #pragma clang fp contract(off)
       const int d2 = 2 * d;
-      const long pb = long(nkx) * ny;
-      const cpx<double>* xb = Xb + blockIdx.z * (pb * d2) + long(nkx) * j;
+      const cpx<double>* xb = a.xb[blockIdx.y] + blockIdx.z * (pl * d2);
       // the tile's float64 boundary values, staged once behind the line
       // buffers (16-byte aligned; bnd_stage_bytes at launch): bl[l * d2 + q]
       cpx<double>* const bl = reinterpret_cast<cpx<double>*>(
           (reinterpret_cast<uintptr_t>(lds + f.nl * f.ldl) + 15) & ~uintptr_t(15));
-      for (int e = tid; e < f.nl * d2; e += blockDim.x) {
-        const int l = e / d2, q = e - l * d2, i = i0 + l;
+      for (int t = tid; t < f.nl * d2; t += blockDim.x) {
+        const int q = t >> f.lgnl, l = t & (f.nl - 1), e = e0 + l;
         const int z = q < d ? q : np - d2 + q;
-        const cpx<double> v = i < nkx ? xb[i + pb * q] : mkc<double>(0, 0);
+        const cpx<double> v = e < nlines ? xb[e + pl * q] : mkc<double>(0, 0);
         lds[l * f.ldl + z] = mkc<T>(T(v.x), T(v.y));
-        bl[e] = v;
+        bl[l * d2 + q] = v;
       }
       __syncthreads();
       // continuation (fftp.fpp:755-773 order): x[top+jj] is plane q = d+jj,
       // x[d-1-jj] is plane q = d-1-jj
-      for (int e = tid; e < f.nl * C; e += blockDim.x) {
-        const int l = e / C, ii = e - l * C, i = i0 + l;
-        double ar = 0.0, ai = 0.0;
-        if (i < nkx) {
-          const cpx<double>* bq = bl + l * d2;
-          const double* D0 = dir + ii * d;
-          const double* D1 = dir + (C - 1 - ii) * d;
-          const cpx<double> t0 = bq[d], b0 = bq[d - 1];
-          ar = D0[0] * t0.x + D1[0] * b0.x;
-          ai = D0[0] * t0.y + D1[0] * b0.y;
-          for (int jj = 1; jj < d; ++jj) {
-            const cpx<double> ut = bq[d + jj], ub = bq[d - 1 - jj];
-            ar = ar + D0[jj] * ut.x;
-            ar = ar + D1[jj] * ub.x;
-            ai = ai + D0[jj] * ut.y;
-            ai = ai + D1[jj] * ub.y;
-          }
+      for (int t = tid; t < f.nl * C; t += blockDim.x) {
+        const int l = t / C, ii = t - l * C;
+        const cpx<double>* bq = bl + l * d2;
+        const double* D0 = dir + ii * d;
+        const double* D1 = dir + (C - 1 - ii) * d;
+        const cpx<double> t0 = bq[d], b0 = bq[d - 1];
+        double ar = D0[0] * t0.x + D1[0] * b0.x;
+        double ai = D0[0] * t0.y + D1[0] * b0.y;
+        for (int jj = 1; jj < d; ++jj) {
+          const cpx<double> ut = bq[d + jj], ub = bq[d - 1 - jj];
+          ar = ar + D0[jj] * ut.x;
+          ar = ar + D1[jj] * ub.x;
+          ai = ai + D0[jj] * ut.y;
+          ai = ai + D1[jj] * ub.y;
         }
         lds[l * f.ldl + np + ii] = mkc<T>(T(ar), T(ai));
       }
@@ -289,8 +297,9 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_x2s(const cpx<T>* __restrict__ 
     }
     zline_dft<T, RS>(xl, f, tws, lane);
   }
-  const int i = i0 + line;
-  if (i < nkx) {
+  const int e = e0 + line;
+  if (e < nlines) {
+    const int j = e / nkx, i = e - j * nkx;
     Cp* so = S + long(n) * (j + long(ny) * i);
     lds_to_global<0, Cp>(lane, f.tpl, n, [&](int k) { return xl[k]; },
                          [&](int k, Cp v) { so[k] = v; });
@@ -398,29 +407,31 @@ __global__ void __launch_bounds__(256) k_z_s2x_bnd(BndSrc src, cpx<double>* __re
 // backward 3D first pass: S * (i k_dir) -> z IFFT -> X planes < nzout.
 // DUAL: the same load also gives X2 <- z IFFT of (i kz) S.
 // blockIdx.z = member: S advances by n*ny*nkx, X and X2 by nkx*ny*nzout.
+// Lines as in k_z_x2s.
 // ---------------------------------------------------------------------------
+template <typename T, typename TI>
+struct ZS2X {
+  const cpx<TI>* s[kMaxComp];
+  cpx<T>* x[kMaxComp];
+  cpx<T>* x2[kMaxComp];
+};
+
 template <typename T, int RS, bool DUAL, typename TI>
-__global__ void __launch_bounds__(kMaxBlock) k_z_s2x(const cpx<TI>* __restrict__ S, cpx<T>* __restrict__ X,
-                                               cpx<T>* __restrict__ X2, LineFFT<cpx<T>> f,
-                                               int nkx, int ny, int nzout, int dirn, int nofft,
+__global__ void __launch_bounds__(kMaxBlock) k_z_s2x(ZS2X<T, TI> a, LineFFT<cpx<T>> f, int nkx,
+                                               int ny, int nzout, int dirn, int nofft,
                                                const double* __restrict__ kx,
                                                const double* __restrict__ ky,
                                                const double* __restrict__ kz) {
   using Cp = cpx<T>;
   SPX_PROLOGUE(Cp, f);
   const int n = f.n;
-  {
-    const long xs = blockIdx.z * (long(nkx) * ny * nzout);
-    S += blockIdx.z * (long(n) * ny * nkx);
-    X += xs;
-    if constexpr (DUAL) X2 += xs;
-  }
-  int bx, j;
-  xcd_tile(bx, j);
-  const int i0 = bx * f.nl;
-  const int i = i0 + line;
-  const bool ok = i < nkx;
-  const long base = long(n) * (j + long(ny) * (ok ? i : 0));
+  const long pl = long(nkx) * ny;
+  const cpx<TI>* __restrict__ S = a.s[blockIdx.y] + blockIdx.z * (pl * n);
+  const int e0 = int(xcd_tile()) * f.nl;
+  const int nlines = int(pl);
+  const bool ok = e0 + line < nlines;
+  const int j = ok ? (e0 + line) / nkx : 0, i = ok ? e0 + line - j * nkx : 0;
+  const long base = long(n) * (j + long(ny) * i);
   // the line (times i k_dirn).  The dual transform needs it again: float
   // kernels and the wave plans (whose occupancy LDS bounds) keep it in
   // registers, the other float64 kernels read it again (the second read hits
@@ -477,12 +488,11 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_s2x(const cpx<TI>* __restrict__
   }
   __syncthreads();
   if (!nofft) zline_dft<T, RS>(xl, f, tws, lane);
-  const long pl = long(nkx) * ny;
-  const int l = tid & (f.nl - 1), ii = i0 + l;
+  const int l = tid & (f.nl - 1), e = e0 + l;
   // (batched stores measured slower here: the z line kernels are VALU-bound)
   constexpr int KB = 0;
-  if (ii < nkx) {
-    Cp* xo = X + ii + long(nkx) * j;
+  if (e < nlines) {
+    Cp* __restrict__ xo = a.x[blockIdx.y] + blockIdx.z * (pl * nzout) + e;
     lds_to_global<KB, Cp>(
         tid >> f.lgnl, f.tpl, nzout, [&](int k) { return cconj(lds[l * f.ldl + k]); },
         [&](int k, Cp v) { xo[pl * k] = v; });
@@ -499,8 +509,8 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_s2x(const cpx<TI>* __restrict__
     }
     __syncthreads();
     zline_dft<T, RS>(xl, f, tws, lane);
-    if (ii < nkx) {
-      Cp* xo = X2 + ii + long(nkx) * j;
+    if (e < nlines) {
+      Cp* __restrict__ xo = a.x2[blockIdx.y] + blockIdx.z * (pl * nzout) + e;
       lds_to_global<KB, Cp>(
           tid >> f.lgnl, f.tpl, nzout, [&](int k) { return cconj(lds[l * f.ldl + k]); },
           [&](int k, Cp v) { xo[pl * k] = v; });
@@ -509,24 +519,34 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_s2x(const cpx<TI>* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// y transform of X (lines along y, stride nkx), one plane per blockIdx.y.
-// DUAL (backward): Y2 <- y IFFT of (i ky) Xin from the same load.
+// y transform of X (lines along y, stride nkx).  The lines of all planes are
+// counted through, e = kx + nkx*plane, and a workgroup takes nl consecutive
+// ones, so only the last workgroup of a field has empty lines.  blockIdx.y:
+// field.  y2 of a field (DUAL kernels, backward): also y2 <- y IFFT of
+// (i ky) in from the same load; null: not for this field.
 // Cy > 0 (forward): FC-Gram continuation of each line before the FFT
 // (fftp.fpp:565-581): rows npy..ny-1 from rows 0..oy-1 and npy-oy..npy-1.
 // ---------------------------------------------------------------------------
+template <typename T>
+struct YFields {
+  const cpx<T>* in[kMaxComp];
+  cpx<T>* out[kMaxComp];
+  cpx<T>* y2[kMaxComp];
+};
+
 template <typename T, int RS, bool DUAL>
-__global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout,
-                                           cpx<T>* __restrict__ Y2, LineFFT<cpx<T>> f, int nkx,
-                                           int ny, int forward, const double* __restrict__ ky,
-                                           int npy, int Cy, int oy,
+__global__ void __launch_bounds__(kMaxBlock) k_y(YFields<T> a, LineFFT<cpx<T>> f, int nkx,
+                                           int ny, long nlines, int forward,
+                                           const double* __restrict__ ky, int npy, int Cy, int oy,
                                            const double* __restrict__ diry) {
   using Cp = cpx<T>;
   SPX_PROLOGUE(Cp, f);
-  int bx, by;
-  xcd_tile(bx, by);
-  const int i0 = bx * f.nl;
-  const long base = long(by) * nkx * ny;
-  const int l = tid & (f.nl - 1), ii = i0 + l;
+  const int l = tid & (f.nl - 1);
+  const long e = long(xcd_tile()) * f.nl + l;
+  const bool in = e < nlines;
+  const long plane = in ? e / nkx : 0;
+  const long base = plane * nkx * ny + (in ? e - plane * nkx : 0);
+  const Cp* const Xin = a.in[blockIdx.y];
   const bool cont = forward && Cy > 0;
   const int nload = cont ? npy : ny;
   if constexpr (RS >= RS_WAVE) {
@@ -538,7 +558,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout
     for (int q = 0; q < KN; ++q) {
       const int jy = (tid >> f.lgnl) + q * f.tpl;
       v[q] = mkc<T>(0, 0);
-      if (ii < nkx && jy < nload) v[q] = Xin[base + ii + long(nkx) * jy];
+      if (in && jy < nload) v[q] = Xin[base + long(nkx) * jy];
     }
 #pragma unroll
     for (int q = 0; q < KN; ++q) {
@@ -549,7 +569,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout
   } else {
     for (int jy = tid >> f.lgnl; jy < nload; jy += f.tpl) {
       Cp v = mkc<T>(0, 0);
-      if (ii < nkx) v = Xin[base + ii + long(nkx) * jy];
+      if (in) v = Xin[base + long(nkx) * jy];
       if (!forward) v.y = -v.y;
       lds[l * f.ldl + jy] = v;
     }
@@ -569,8 +589,8 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout
   }
   zline_dft<T, RS>(xl, f, tws, lane);
   constexpr int KB = RS >= RS_WAVE ? keep_n<RS>() : 0;
-  if (ii < nkx) {
-    Cp* xo = Xout + base + ii;
+  if (in) {
+    Cp* xo = a.out[blockIdx.y] + base;
     lds_to_global<KB, Cp>(
         tid >> f.lgnl, f.tpl, ny,
         [&](int jy) {
@@ -581,6 +601,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout
         [&](int jy, Cp v) { xo[long(nkx) * jy] = v; });
   }
   if constexpr (DUAL) {
+    if (!a.y2[blockIdx.y]) return;  // uniform per workgroup
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < KEEP; ++q) {
@@ -589,8 +610,8 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout
     }
     __syncthreads();
     zline_dft<T, RS>(xl, f, tws, lane);
-    if (ii < nkx) {
-      Cp* yo = Y2 + base + ii;
+    if (in) {
+      Cp* yo = a.y2[blockIdx.y] + base;
       lds_to_global<KB, Cp>(
           tid >> f.lgnl, f.tpl, ny, [&](int jy) { return cconj(lds[l * f.ldl + jy]); },
           [&](int jy, Cp v) { yo[long(nkx) * jy] = v; });
@@ -598,14 +619,36 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(const cpx<T>* Xin, cpx<T>* Xout
   }
 }
 
+// The half spectra of a row pair from the transform xl of A + iB.
+template <typename T>
+__device__ __forceinline__ void store_r2c_pair(const cpx<T>* xl, cpx<T>* o0, int nkx, int nx,
+                                               int lane, int tpl) {
+  const T h = T(0.5);
+  for (int k = lane; k < nkx; k += tpl) {
+    const cpx<T> Z = xl[k];
+    const cpx<T> Zc = xl[k == 0 ? 0 : nx - k];
+    o0[k] = mkc<T>((Z.x + Zc.x) * h, (Z.y - Zc.y) * h);
+    o0[k + nkx] = mkc<T>((Z.y + Zc.y) * h, -(Z.x - Zc.x) * h);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // x real -> half complex: rows 2p, 2p+1 packed as one complex line
 // ---------------------------------------------------------------------------
+// (blockIdx.y: field)
+template <typename T>
+struct XFields {
+  const void* in[kMaxComp];
+  void* out[kMaxComp];
+};
+
 template <typename T, int RS>
-__global__ void __launch_bounds__(kMaxBlock) k_xr2c(const T* __restrict__ R, cpx<T>* __restrict__ X,
-                                              LineFFT<cpx<T>> f, int nkx, long npairs) {
+__global__ void __launch_bounds__(kMaxBlock) k_xr2c(XFields<T> a, LineFFT<cpx<T>> f, int nkx,
+                                              long npairs) {
   using Cp = cpx<T>;
   SPX_PROLOGUE(Cp, f);
+  const T* __restrict__ R = static_cast<const T*>(a.in[blockIdx.y]);
+  Cp* __restrict__ X = static_cast<Cp*>(a.out[blockIdx.y]);
   const int nx = f.n;
   const long p = long(blockIdx.x) * f.nl + line;
   const bool ok = p < npairs;
@@ -634,16 +677,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_xr2c(const T* __restrict__ R, cpx
   }
   __syncthreads();
   zline_dft<T, RS>(xl, f, tws, lane);
-  if (ok) {
-    Cp* o0 = X + long(nkx) * (2 * p);
-    const T h = T(0.5);
-    for (int k = lane; k < nkx; k += f.tpl) {
-      const Cp Z = xl[k];
-      const Cp Zc = xl[k == 0 ? 0 : nx - k];
-      o0[k] = mkc<T>((Z.x + Zc.x) * h, (Z.y - Zc.y) * h);
-      o0[k + nkx] = mkc<T>((Z.y + Zc.y) * h, -(Z.x - Zc.x) * h);
-    }
-  }
+  if (ok) store_r2c_pair(xl, X + long(nkx) * (2 * p), nkx, nx, lane, f.tpl);
 }
 
 // Load of an x c2r row pair into LDS: Z = A + iB from the two half spectra
@@ -742,11 +776,13 @@ constexpr int xg_chunk() {
 }
 
 template <typename T, int RS>
-__global__ void __launch_bounds__(kMaxBlock) k_xc2r(const cpx<T>* __restrict__ X, T* __restrict__ R,
-                                              LineFFT<cpx<T>> f, int nkx, long npairs, int dirx,
+__global__ void __launch_bounds__(kMaxBlock) k_xc2r(XFields<T> a, LineFFT<cpx<T>> f, int nkx,
+                                              long npairs, int dirx,
                                               const double* __restrict__ kx) {
   using Cp = cpx<T>;
   SPX_PROLOGUE(Cp, f);
+  const Cp* __restrict__ X = static_cast<const Cp*>(a.in[blockIdx.y]);
+  T* __restrict__ R = static_cast<T*>(a.out[blockIdx.y]);
   const int nx = f.n;
   const long p = long(blockIdx.x) * f.nl + line;
   const bool ok = p < npairs;
@@ -765,25 +801,26 @@ __global__ void __launch_bounds__(kMaxBlock) k_xc2r(const cpx<T>* __restrict__ X
 
 // ((u*Dx + v*Dy) + w*Dz)*tmp on a row pair, the three derivatives c2r'd in
 // LDS one after the other and accumulated in registers
-// (pseudospec_hd.f90:254-312, pseudospec_phd.f90:63-108).
+// (pseudospec_hd.f90:254-312, pseudospec_phd.f90:63-108), then the r2c of the
+// product: the real product never goes to memory.  blockIdx.y: field.  The
+// half spectra may go over YY: the line that writes a row pair is the one
+// that read it.
+template <typename T>
+struct XProd {
+  const cpx<T>* yv[4];
+  const cpx<T>* yy[4];
+  const cpx<T>* xz[4];
+  cpx<T>* out[4];
+  const T* vel[3];
+};
+
 template <typename T, int RS>
-__global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(const cpx<T>* __restrict__ YV,
-                                                    const cpx<T>* __restrict__ YY,
-                                                    const cpx<T>* __restrict__ XZ,
-                                                    const T* __restrict__ u,
-                                                    const T* __restrict__ v,
-                                                    const T* __restrict__ w, T* __restrict__ out,
-                                                    LineFFT<cpx<T>> f, int nkx, long npairs,
-                                                    double tmpd, const double* __restrict__ kx,
-                                                    long cstride, long rstride) {
+__global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cpx<T>> f, int nkx,
+                                                    long npairs, double tmpd,
+                                                    const double* __restrict__ kx) {
 #pragma clang fp contract(off)
   using Cp = cpx<T>;
   SPX_PROLOGUE(Cp, f);
-  // blockIdx.y: component (YV, YY, XZ advance by cstride, out by rstride)
-  YV += blockIdx.y * cstride;
-  YY += blockIdx.y * cstride;
-  XZ += blockIdx.y * cstride;
-  out += blockIdx.y * rstride;
   const int nx = f.n;
   const T tmp = T(tmpd);
   const long p = long(blockIdx.x) * f.nl + line;
@@ -791,13 +828,12 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(const cpx<T>* __restri
   const long ro = long(nx) * (2 * (ok ? p : 0));
   const long co = long(nkx) * (2 * (ok ? p : 0));
   T accA[KEEP], accB[KEEP];
-  const Cp* srcs[3] = {YV, YY, XZ};
-  const T* mult[3] = {u, v, w};
+  const Cp* srcs[3] = {a.yv[blockIdx.y], a.yy[blockIdx.y], a.xz[blockIdx.y]};
   for (int r = 0; r < 3; ++r) {
     load_c2r_pair<T, batch_n<RS>()>(xl, srcs[r] + co, nkx, nx, lane, f.tpl, ok, r == 0 ? 1 : 0, kx);
     // the velocity values this thread multiplies with, loaded before the
     // transform so that their latency overlaps it
-    const T* m = mult[r] + ro;
+    const T* m = a.vel[r] + ro;
     T ma[KEEP], mb[KEEP];
 #pragma unroll
     for (int q = 0; q < KEEP; ++q) {
@@ -811,55 +847,53 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(const cpx<T>* __restri
 #pragma unroll
     for (int q = 0; q < KEEP; ++q) {
       const int x = lane + q * f.tpl;
-      if (x < nx && ok) {
+      if (x < nx) {
         const Cp z = xl[x];
-        const T a = z.x, b = -z.y;
+        const T va = z.x, vb = -z.y;
         if (r == 0) {
-          accA[q] = ma[q] * a;
-          accB[q] = mb[q] * b;
+          accA[q] = ma[q] * va;
+          accB[q] = mb[q] * vb;
         } else if (r == 1) {
-          accA[q] = accA[q] + ma[q] * a;
-          accB[q] = accB[q] + mb[q] * b;
+          accA[q] = accA[q] + ma[q] * va;
+          accB[q] = accB[q] + mb[q] * vb;
         } else {
-          accA[q] = (accA[q] + ma[q] * a) * tmp;
-          accB[q] = (accB[q] + mb[q] * b) * tmp;
+          accA[q] = (accA[q] + ma[q] * va) * tmp;
+          accB[q] = (accB[q] + mb[q] * vb) * tmp;
         }
       }
     }
     __syncthreads();
   }
-  if (ok) {
 #pragma unroll
-    for (int q = 0; q < KEEP; ++q) {
-      const int x = lane + q * f.tpl;
-      if (x < nx) {
-        out[ro + x] = accA[q];
-        out[ro + x + nx] = accB[q];
-      }
-    }
+  for (int q = 0; q < KEEP; ++q) {
+    const int x = lane + q * f.tpl;
+    if (x < nx) xl[x] = mkc<T>(accA[q], accB[q]);
   }
+  __syncthreads();
+  zline_dft<T, RS>(xl, f, tws, lane);
+  if (ok) store_r2c_pair(xl, a.out[blockIdx.y] + co, nkx, nx, lane, f.tpl);
 }
 
 // gradre's whole x stage on a row pair (pseudospec_hd.f90:254-312): the
 // velocity components u, v, w = c2r(YV_c) are formed first and kept in
 // registers (and stored to rv[c] when given: advect reuses them), then for
-// each component c ((u Dx v_c + v Dy v_c) + w Dz v_c) tmp from the c2r of
-// i kx YV_c, YY_c and XZ_c, in k_xgrad_prod's operation order.  It saves the
-// traffic of the real velocity (written once and read nine times per stage
-// by xc2r x 3 + xgrad_prod x 3).  A line is owned by its tpl threads, so
-// the twelve transforms of a row pair synchronise with line_sync.
+// each field c (the three components, and a scalar when nf = 4)
+// ((u Dx v_c + v Dy v_c) + w Dz v_c) tmp from the c2r of i kx YV_c, YY_c and
+// XZ_c, in k_xgrad_prod's operation order, and its r2c.  Neither the real
+// velocity nor the products go to memory.  A line is owned by its tpl threads, so
+// the transforms of a row pair synchronise with line_sync.
 template <typename T>
 struct XGradArgs {
-  const cpx<T>* yv[3];
-  const cpx<T>* yy[3];
-  const cpx<T>* xz[3];
+  const cpx<T>* yv[4];
+  const cpx<T>* yy[4];
+  const cpx<T>* xz[4];
   T* rv[3];   // may be null
-  T* out[3];
+  cpx<T>* out[4];
 };
 
 template <typename T, int RS>
 __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fused(
-    XGradArgs<T> a, LineFFT<cpx<T>> f, int nkx, long npairs, double tmpd,
+    XGradArgs<T> a, LineFFT<cpx<T>> f, int nkx, long npairs, int nf, double tmpd,
     const double* __restrict__ kx) {
 #pragma clang fp contract(off)
   using Cp = cpx<T>;
@@ -896,7 +930,7 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
     line_sync(f.tpl);
   }
 #pragma unroll 1
-  for (int c = 0; c < 3; ++c) {
+  for (int c = 0; c < nf; ++c) {
     T accA[KEEP], accB[KEEP];
     const Cp* srcs[3] = {a.yv[c], a.yy[c], a.xz[c]};
 #pragma unroll
@@ -918,23 +952,18 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
             accA[q] = accA[q] + vel[1][0][q] * va;
             accB[q] = accB[q] + vel[1][1][q] * vb;
           } else {
-            accA[q] = (accA[q] + vel[2][0][q] * va) * tmp;
-            accB[q] = (accB[q] + vel[2][1][q] * vb) * tmp;
+            // the element's own thread read it: the product replaces it
+            xl[x] = mkc<T>((accA[q] + vel[2][0][q] * va) * tmp,
+                           (accB[q] + vel[2][1][q] * vb) * tmp);
           }
         }
       }
       line_sync(f.tpl);
     }
-    if (ok) {
-#pragma unroll
-      for (int q = 0; q < KEEP; ++q) {
-        const int x = lane + q * f.tpl;
-        if (x < nx) {
-          a.out[c][ro + x] = accA[q];
-          a.out[c][ro + x + nx] = accB[q];
-        }
-      }
-    }
+    line_fft_nosync<T, RS>(xl, f, tws, lane);
+    line_sync(f.tpl);
+    if (ok) store_r2c_pair(xl, a.out[c] + co, nkx, nx, lane, f.tpl);
+    line_sync(f.tpl);
   }
 }
 
@@ -2100,34 +2129,43 @@ int fc_continue_only(spx_plan* p, void* S) {
 }
 
 template <typename T>
-static int zfft_x2s_t(spx_plan* p, const void* X, void* S, int nofft, const LineFFTHost& f,
-                      const void* Xb) {
+static int zfft_x2s_t(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft,
+                      const LineFFTHost& f, const void* const* Xb) {
   // members: grid.z; X holds np planes per member (all nz with nofft)
-  dim3 grid(unsigned((p->nkx + f.nl - 1) / f.nl), unsigned(p->g.ny), unsigned(p->mem));
-  const long xstride = long(p->nkx) * p->g.ny * (nofft ? p->g.nz : p->np);
-  ProfScope ps_(p, "z_x2s", double(p->wkx()) * p->g.ny * sizeof(cpx<T>) *
+  const long pl = long(p->nkx) * p->g.ny;
+  dim3 grid(unsigned((pl + f.nl - 1) / f.nl), unsigned(ncomp), unsigned(p->mem));
+  const long xstride = pl * (nofft ? p->g.nz : p->np);
+  ZX2S<T> a;
+  for (int c = 0; c < kMaxComp; ++c) {
+    a.x[c] = c < ncomp ? C_<T>(X[c]) : nullptr;
+    a.s[c] = c < ncomp ? C_<T>(S[c]) : nullptr;
+    a.xb[c] = c < ncomp && Xb ? C_<double>(Xb[c]) : nullptr;
+  }
+  ProfScope ps_(p, "z_x2s", double(p->wkx()) * p->g.ny * sizeof(cpx<T>) * ncomp *
                                 ((nofft ? p->g.nz : p->np) + p->g.nz));
   if (Xb) {
     // plus the staged float64 boundary values of the tile (nl * 2d, aligned)
     const size_t bnd_stage_bytes = size_t(f.nl) * 2 * p->g.oz * sizeof(Cd) + 16;
     SPX_LAUNCH_Z(f, k_z_x2s, T, SPX_COMMA true, grid, blk(f),
-                  f.lds_bytes(sizeof(cpx<T>)) + bnd_stage_bytes, p->stream, C_<T>(X), C_<T>(S),
+                  f.lds_bytes(sizeof(cpx<T>)) + bnd_stage_bytes, p->stream, a,
                   f.dev<cpx<T>>(), p->nkx, p->g.ny, p->np, nofft, p->d_dir, p->g.Cz, p->g.oz,
-                  xstride, C_<double>(Xb));
+                  xstride);
     SPX_CHECK_LAUNCH();
     return SPX_OK;
   }
   SPX_LAUNCH_Z(f, k_z_x2s, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
-                p->stream, C_<T>(X), C_<T>(S), f.dev<cpx<T>>(), p->nkx, p->g.ny, p->np, nofft, p->d_dir,
-                p->g.Cz, p->g.oz, xstride, static_cast<const Cd*>(nullptr));
+                p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, p->np, nofft, p->d_dir,
+                p->g.Cz, p->g.oz, xstride);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
-int zfft_x2s(spx_plan* p, const void* X, void* S, int nofft, bool lo, const void* Xb) {
+int zfft_x2s(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft, bool lo,
+             const void* const* Xb) {
   if (int rc = check_lo(p, lo)) return rc;
+  if (ncomp < 1 || ncomp > kMaxComp) return fail(SPX_ERR_ARG, "zfft_x2s: bad field count");
   if (Xb && (nofft || p->g.Cz <= 0)) return fail(SPX_ERR_ARG, "boundary planes need a continuation");
-  return lo ? zfft_x2s_t<float>(p, X, S, nofft, fzt(p, true), Xb)
-            : zfft_x2s_t<double>(p, X, S, nofft, fzt(p, false), Xb);
+  return lo ? zfft_x2s_t<float>(p, ncomp, X, S, nofft, fzt(p, true), Xb)
+            : zfft_x2s_t<double>(p, ncomp, X, S, nofft, fzt(p, false), Xb);
 }
 
 int zfft_s2x_bnd(spx_plan* p, const void* const* S, int ncomp, void* XVb, void* XZb) {
@@ -2167,168 +2205,204 @@ int zfft_s2x_bnd(spx_plan* p, const void* const* S, int ncomp, void* XVb, void* 
 
 // S is float64 in both precisions; X (and X2) are T
 template <typename T>
-static int zfft_s2x_t(spx_plan* p, const void* S, void* X, int dirn, int nzout, int nofft,
-                      void* X2, const LineFFTHost& f) {
+static int zfft_s2x_t(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn,
+                      int nzout, int nofft, void* const* X2, const LineFFTHost& f) {
   // members: grid.z; X holds nzout planes per member
-  dim3 grid(unsigned((p->nkx + f.nl - 1) / f.nl), unsigned(p->g.ny), unsigned(p->mem));
-  const double line = double(p->wkx()) * p->g.ny;
-  const Cd* in = C_<double>(S);
+  const long pl = long(p->nkx) * p->g.ny;
+  dim3 grid(unsigned((pl + f.nl - 1) / f.nl), unsigned(ncomp), unsigned(p->mem));
+  const double line = double(p->wkx()) * p->g.ny * ncomp;
+  ZS2X<T, double> a;
+  for (int c = 0; c < kMaxComp; ++c) {
+    a.s[c] = c < ncomp ? C_<double>(S[c]) : nullptr;
+    a.x[c] = c < ncomp ? C_<T>(X[c]) : nullptr;
+    a.x2[c] = c < ncomp && X2 ? C_<T>(X2[c]) : nullptr;
+  }
   if (X2) {
     ProfScope ps_(p, "z_s2x_dual", line * (16.0 * p->g.nz + 2.0 * sizeof(cpx<T>) * nzout));
     SPX_LAUNCH_Z(f, k_z_s2x, T, SPX_COMMA true SPX_COMMA double, grid, blk(f),
-                  f.lds_bytes(sizeof(cpx<T>)), p->stream, in, C_<T>(X), C_<T>(X2),
-                  f.dev<cpx<T>>(), p->nkx, p->g.ny, nzout, dirn, nofft, p->d_kx, p->d_ky,
-                  p->d_kz);
+                  f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny,
+                  nzout, dirn, nofft, p->d_kx, p->d_ky, p->d_kz);
   } else {
     ProfScope ps_(p, "z_s2x", line * (16.0 * p->g.nz + sizeof(cpx<T>) * nzout));
     SPX_LAUNCH_Z(f, k_z_s2x, T, SPX_COMMA false SPX_COMMA double, grid, blk(f),
-                  f.lds_bytes(sizeof(cpx<T>)), p->stream, in, C_<T>(X),
-                  static_cast<cpx<T>*>(nullptr), f.dev<cpx<T>>(), p->nkx, p->g.ny, nzout, dirn,
-                  nofft, p->d_kx, p->d_ky, p->d_kz);
+                  f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny,
+                  nzout, dirn, nofft, p->d_kx, p->d_ky, p->d_kz);
   }
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
-int zfft_s2x(spx_plan* p, const void* S, void* X, int dirn, int nzout, int nofft, void* X2,
-             bool lo) {
+int zfft_s2x(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn, int nzout,
+             int nofft, void* const* X2, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
-  return lo ? zfft_s2x_t<float>(p, S, X, dirn, nzout, nofft, X2, fzt(p, true))
-            : zfft_s2x_t<double>(p, S, X, dirn, nzout, nofft, X2, fzt(p, false));
+  if (ncomp < 1 || ncomp > kMaxComp) return fail(SPX_ERR_ARG, "zfft_s2x: bad field count");
+  return lo ? zfft_s2x_t<float>(p, ncomp, S, X, dirn, nzout, nofft, X2, fzt(p, true))
+            : zfft_s2x_t<double>(p, ncomp, S, X, dirn, nzout, nofft, X2, fzt(p, false));
 }
 #endif  // SPX_PART 1 (z transforms)
 
 #if !defined(SPX_PART) || SPX_PART == 2
 template <typename T>
-static int yfft_t(spx_plan* p, void* X, int forward, int nplanes, const void* Xin, void* Y2,
-                  const LineFFTHost& f, bool cont) {
+static int yfft_t(spx_plan* p, int nf, const void* const* in, void* const* out, int forward,
+                  int nplanes, void* const* Y2, const LineFFTHost& f, bool cont) {
   // members are consecutive blocks of nplanes planes
-  const int npl = nplanes * p->mem;
-  dim3 grid(unsigned((p->nkx + f.nl - 1) / f.nl), unsigned(npl));
-  const cpx<T>* in = C_<T>(Xin ? Xin : static_cast<const void*>(X));
-  const double io = double(p->nkx) * p->g.ny * npl * sizeof(cpx<T>);
-  if (Y2) {
+  const long nlines = long(p->nkx) * nplanes * p->mem;
+  dim3 grid(unsigned((nlines + f.nl - 1) / f.nl), unsigned(nf));
+  YFields<T> a;
+  int nd = 0;
+  for (int c = 0; c < kMaxComp; ++c) {
+    a.in[c] = c < nf ? C_<T>(in[c]) : nullptr;
+    a.out[c] = c < nf ? C_<T>(out[c]) : nullptr;
+    a.y2[c] = c < nf && Y2 ? C_<T>(Y2[c]) : nullptr;
+    nd += a.y2[c] != nullptr;
+  }
+  const double io = double(nlines) * p->g.ny * sizeof(cpx<T>);
+  if (nd > 0) {
     if (forward) return fail(SPX_ERR_ARG, "dual y transform is backward only");
-    ProfScope ps_(p, "y_dual", io * 3.0);
+    ProfScope ps_(p, "y_dual", io * (2.0 * nf + nd));
     SPX_LAUNCH_XY(f, k_y, T, SPX_COMMA true, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
-                  p->stream, in, C_<T>(X), C_<T>(Y2), f.dev<cpx<T>>(), p->nkx, p->g.ny, forward,
-                  p->d_ky, p->npy, 0, 0, static_cast<const double*>(nullptr));
+                  p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, nlines, forward, p->d_ky,
+                  p->npy, 0, 0, static_cast<const double*>(nullptr));
   } else {
-    ProfScope ps_(p, "y", io * 2.0);
+    ProfScope ps_(p, "y", io * 2.0 * nf);
     SPX_LAUNCH_XY(f, k_y, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
-                  p->stream, in, C_<T>(X), static_cast<cpx<T>*>(nullptr), f.dev<cpx<T>>(),
-                  p->nkx, p->g.ny, forward, p->d_ky, p->npy, cont ? p->Cy : 0, p->oy,
-                  p->d_diry);
+                  p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, nlines, forward, p->d_ky,
+                  p->npy, cont ? p->Cy : 0, p->oy, p->d_diry);
   }
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
-int yfft(spx_plan* p, void* X, int forward, int nplanes, const void* Xin, void* Y2, bool lo,
-         bool cont) {
+int yfft(spx_plan* p, int nf, const void* const* in, void* const* out, int forward, int nplanes,
+         void* const* Y2, bool lo, bool cont) {
   if (int rc = check_lo(p, lo)) return rc;
+  if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "yfft: bad field count");
   if (cont && (!forward || p->Cy <= 0 || Y2))
     return fail(SPX_ERR_ARG, "y continuation: forward transforms of plans with Cy > 0 only");
-  return lo ? yfft_t<float>(p, X, forward, nplanes, Xin, Y2, p->fy32, cont)
-            : yfft_t<double>(p, X, forward, nplanes, Xin, Y2, p->fy, cont);
+  return lo ? yfft_t<float>(p, nf, in, out, forward, nplanes, Y2, p->fy32, cont)
+            : yfft_t<double>(p, nf, in, out, forward, nplanes, Y2, p->fy, cont);
 }
 
 template <typename T>
-static int xr2c_t(spx_plan* p, const void* R, void* X, int nplanes, const LineFFTHost& f) {
-  const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
-  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl));
-  ProfScope ps_(p, "xr2c", double(p->g.ny) * nplanes * p->mem *
-                               (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
-  SPX_LAUNCH_XY(f, k_xr2c, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream,
-                static_cast<const T*>(R), C_<T>(X), f.dev<cpx<T>>(), p->nkx, npairs);
-  SPX_CHECK_LAUNCH();
-  return SPX_OK;
-}
-int xr2c(spx_plan* p, const void* R, void* X, int nplanes, bool lo) {
-  if (int rc = check_lo(p, lo)) return rc;
-  return lo ? xr2c_t<float>(p, R, X, nplanes, p->fx32) : xr2c_t<double>(p, R, X, nplanes, p->fx);
+static XFields<T> x_fields(int nf, const void* const* in, void* const* out) {
+  XFields<T> a;
+  for (int c = 0; c < kMaxComp; ++c) {
+    a.in[c] = c < nf ? in[c] : nullptr;
+    a.out[c] = c < nf ? out[c] : nullptr;
+  }
+  return a;
 }
 
 template <typename T>
-static int xc2r_t(spx_plan* p, const void* X, void* R, int nplanes, int dirx,
+static int xr2c_t(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
                   const LineFFTHost& f) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
-  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl));
-  ProfScope ps_(p, "xc2r", double(p->g.ny) * nplanes * p->mem *
+  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
+  const XFields<T> a = x_fields<T>(nf, R, X);
+  ProfScope ps_(p, "xr2c", double(p->g.ny) * nplanes * p->mem * nf *
                                (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
-  SPX_LAUNCH_XY(f, k_xc2r, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream,
-                C_<T>(X), static_cast<T*>(R), f.dev<cpx<T>>(), p->nkx, npairs, dirx, p->d_kx);
+  SPX_LAUNCH_XY(f, k_xr2c, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+                f.dev<cpx<T>>(), p->nkx, npairs);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
-int xc2r(spx_plan* p, const void* X, void* R, int nplanes, int dirx, bool lo) {
+int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
-  return lo ? xc2r_t<float>(p, X, R, nplanes, dirx, p->fx32)
-            : xc2r_t<double>(p, X, R, nplanes, dirx, p->fx);
+  if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xr2c: bad field count");
+  return lo ? xr2c_t<float>(p, nf, R, X, nplanes, p->fx32)
+            : xr2c_t<double>(p, nf, R, X, nplanes, p->fx);
 }
 
 template <typename T>
-static int xgrad_prod_t(spx_plan* p, const void* YV, const void* YY, const void* XZ,
-                        const void* u, const void* v, const void* w, void* out,
-                        const LineFFTHost& f, int nplanes, int ncomp) {
+static int xc2r_t(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes,
+                  int dirx, const LineFFTHost& f) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
-  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(ncomp));
-  const long cstride = long(p->nkx) * p->g.ny * nplanes * p->mem;
-  const long rstride = long(p->g.nx) * p->g.ny * nplanes * p->mem;
+  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
+  const XFields<T> a = x_fields<T>(nf, X, R);
+  ProfScope ps_(p, "xc2r", double(p->g.ny) * nplanes * p->mem * nf *
+                               (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
+  SPX_LAUNCH_XY(f, k_xc2r, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+                f.dev<cpx<T>>(), p->nkx, npairs, dirx, p->d_kx);
+  SPX_CHECK_LAUNCH();
+  return SPX_OK;
+}
+int xc2r(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes, int dirx,
+         bool lo) {
+  if (int rc = check_lo(p, lo)) return rc;
+  if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xc2r: bad field count");
+  return lo ? xc2r_t<float>(p, nf, X, R, nplanes, dirx, p->fx32)
+            : xc2r_t<double>(p, nf, X, R, nplanes, dirx, p->fx);
+}
+
+template <typename T>
+static int xgrad_prod_t(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
+                        const void* const* XZ, const void* const* vel, void* const* out,
+                        const LineFFTHost& f, int nplanes) {
+  const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
+  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
   const double t = double(p->g.nx) * double(p->g.ny) * double(p->g.nz);
-  const double rows = double(p->g.ny) * nplanes * p->mem * ncomp;
-  ProfScope ps_(p, "xgrad_prod", rows * (3.0 * sizeof(cpx<T>) * p->nkx +
-                                         4.0 * sizeof(T) * p->g.nx));
-  SPX_LAUNCH_XY(f, k_xgrad_prod, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream,
-                C_<T>(YV), C_<T>(YY), C_<T>(XZ), static_cast<const T*>(u),
-                static_cast<const T*>(v), static_cast<const T*>(w), static_cast<T*>(out),
-                f.dev<cpx<T>>(), p->nkx, npairs, 1.0 / (t * t), p->d_kx, cstride, rstride);
+  const double rows = double(p->g.ny) * nplanes * p->mem * nf;
+  XProd<T> a;
+  for (int c = 0; c < 4; ++c) {
+    a.yv[c] = c < nf ? C_<T>(YV[c]) : nullptr;
+    a.yy[c] = c < nf ? C_<T>(YY[c]) : nullptr;
+    a.xz[c] = c < nf ? C_<T>(XZ[c]) : nullptr;
+    a.out[c] = c < nf ? C_<T>(out[c]) : nullptr;
+  }
+  for (int c = 0; c < 3; ++c) a.vel[c] = static_cast<const T*>(vel[c]);
+  ProfScope ps_(p, "xgrad_prod", rows * (4.0 * sizeof(cpx<T>) * p->nkx +
+                                         3.0 * sizeof(T) * p->g.nx));
+  SPX_LAUNCH_XY(f, k_xgrad_prod, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+                f.dev<cpx<T>>(), p->nkx, npairs, 1.0 / (t * t), p->d_kx);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
 template <typename T>
-static int xgrad_fused_t(spx_plan* p, void* const* YV, void* const* YY, void* const* XZ,
+static int xgrad_fused_t(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
                          void* const* RV, void* const* out, const LineFFTHost& f) {
   const int nplanes = p->np;
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
   const double t = double(p->g.nx) * double(p->g.ny) * double(p->g.nz);
   const double rows = double(p->g.ny) * nplanes * p->mem;
   XGradArgs<T> a;
-  for (int c = 0; c < 3; ++c) {
-    a.yv[c] = C_<T>(static_cast<const void*>(YV[c]));
-    a.yy[c] = C_<T>(static_cast<const void*>(YY[c]));
-    a.xz[c] = C_<T>(static_cast<const void*>(XZ[c]));
-    a.rv[c] = RV ? static_cast<T*>(RV[c]) : nullptr;
-    a.out[c] = static_cast<T*>(out[c]);
+  for (int c = 0; c < 4; ++c) {
+    a.yv[c] = c < nf ? C_<T>(static_cast<const void*>(YV[c])) : nullptr;
+    a.yy[c] = c < nf ? C_<T>(static_cast<const void*>(YY[c])) : nullptr;
+    a.xz[c] = c < nf ? C_<T>(static_cast<const void*>(XZ[c])) : nullptr;
+    a.out[c] = c < nf ? C_<T>(out[c]) : nullptr;
+    if (c < 3) a.rv[c] = RV ? static_cast<T*>(RV[c]) : nullptr;
   }
-  ProfScope ps_(p, "xgrad_fused", rows * (9.0 * sizeof(cpx<T>) * p->nkx +
-                                          (RV ? 6.0 : 3.0) * sizeof(T) * p->g.nx));
+  ProfScope ps_(p, "xgrad_fused", rows * (4.0 * nf * sizeof(cpx<T>) * p->nkx +
+                                          (RV ? 3.0 : 0.0) * sizeof(T) * p->g.nx));
   if (f.wave == 3)
     hipLaunchKernelGGL((k_xgrad_fused<T, RS_WAVE + 3>), dim3(unsigned((npairs + f.nl - 1) / f.nl)),
                        blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(),
-                       p->nkx, npairs, 1.0 / (t * t), p->d_kx);
+                       p->nkx, npairs, nf, 1.0 / (t * t), p->d_kx);
   else
     hipLaunchKernelGGL((k_xgrad_fused<T, RS_POW2>), dim3(unsigned((npairs + f.nl - 1) / f.nl)),
                        blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(),
-                       p->nkx, npairs, 1.0 / (t * t), p->d_kx);
+                       p->nkx, npairs, nf, 1.0 / (t * t), p->d_kx);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
-int xgrad_fused(spx_plan* p, void* const* YV, void* const* YY, void* const* XZ, void* const* RV,
-                void* const* out, bool lo) {
+int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
+                void* const* RV, void* const* out, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
+  if (nf < 3 || nf > 4) return fail(SPX_ERR_ARG, "xgrad_fused: 3 or 4 fields");
   // power-of-two x lines only: the other radix families spill the velocity
   // registers
   const int rs = rset_of(lo ? p->fx32 : p->fx);
   if (rs != RS_POW2 && rs != RS_WAVE + 3) return SPX_ERR_UNSUPPORTED;
-  return lo ? xgrad_fused_t<float>(p, YV, YY, XZ, RV, out, p->fx32)
-            : xgrad_fused_t<double>(p, YV, YY, XZ, RV, out, p->fx);
+  return lo ? xgrad_fused_t<float>(p, nf, YV, YY, XZ, RV, out, p->fx32)
+            : xgrad_fused_t<double>(p, nf, YV, YY, XZ, RV, out, p->fx);
 }
 
-int xgrad_prod(spx_plan* p, const void* YV, const void* YY, const void* XZ, const void* u,
-               const void* v, const void* w, void* out, bool lo, int nplanes, int ncomp) {
+int xgrad_prod(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
+               const void* const* XZ, const void* const* vel, void* const* out, bool lo,
+               int nplanes) {
   if (int rc = check_lo(p, lo)) return rc;
+  if (nf < 1 || nf > 4) return fail(SPX_ERR_ARG, "xgrad_prod: 1..4 fields");
   if (nplanes < 0) nplanes = p->np;
-  return lo ? xgrad_prod_t<float>(p, YV, YY, XZ, u, v, w, out, p->fx32, nplanes, ncomp)
-            : xgrad_prod_t<double>(p, YV, YY, XZ, u, v, w, out, p->fx, nplanes, ncomp);
+  return lo ? xgrad_prod_t<float>(p, nf, YV, YY, XZ, vel, out, p->fx32, nplanes)
+            : xgrad_prod_t<double>(p, nf, YV, YY, XZ, vel, out, p->fx, nplanes);
 }
 #endif  // SPX_PART 2 (y and x transforms)
 

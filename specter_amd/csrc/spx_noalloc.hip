@@ -46,8 +46,10 @@ static int scratch_address(int dev, unsigned char** out) {
 }
 
 // the gradre work set carved out of the scratch, each array on a 256-byte
-// boundary: XV, XZ, XY (3 each), RV, RO (3 each), and in mixed plans with
-// walls the six float64 boundary-plane buffers
+// boundary: XV, XZ, XY, RV (3 each), and in mixed plans with walls the float64
+// boundary-plane buffers.  The reserve also counts real products of the size
+// of RV and of the boundary planes, which the x stage no longer stores: the
+// limit on the grid stays where callers know it
 // (in the order of the pointer slots of spx_gradre_noalloc); returns the count
 static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 static int noalloc_sizes(const spx_plan* p, size_t sz[21]) {
@@ -98,10 +100,11 @@ int spx_gradre_noalloc(spx_plan* p, const void* a, const void* b, const void* c,
   // carve the work set out of the scratch (every array is written before it
   // is read, as with the allocated set, so nothing is cleared); the plan's
   // own work pointers are swapped for the call and restored after it
+  void* unused = nullptr;
   void** slots[21] = {&p->XV[0], &p->XV[1], &p->XV[2], &p->XZ[0], &p->XZ[1], &p->XZ[2],
                       &p->XY[0], &p->XY[1], &p->XY[2], &p->RV[0], &p->RV[1], &p->RV[2],
-                      &p->RO[0], &p->RO[1], &p->RO[2], &p->XVb, &p->XZb, &p->XYb,
-                      &p->RVb,   &p->ROb,   &p->XFb};
+                      &unused,   &unused,   &unused,   &p->XVb, &p->XZb, &p->XYb,
+                      &p->RVb,   &unused,   &p->XFb};
   void* sv[21];
   for (int i = 0; i < 21; ++i) sv[i] = *slots[i];
   size_t sz[21];
@@ -115,7 +118,7 @@ int spx_gradre_noalloc(spx_plan* p, const void* a, const void* b, const void* c,
     MemberView mv(p, p->nact);
     const void* v[3] = {a, b, c};
     void* o[3] = {d, e, f};
-    rc = gradre_impl(p, v, o, false);
+    rc = gradre_impl(p, v, nullptr, o);
   }
   for (int i = 0; i < 21; ++i) *slots[i] = sv[i];
   return rc;
