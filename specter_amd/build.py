@@ -12,10 +12,9 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libspx.so")
-# (source, defines): spx_fft.hip is compiled in three parts (see its header)
-SOURCES = [("spx_fft.hip", ["-DSPX_PART=1"]), ("spx_fft.hip", ["-DSPX_PART=2"]),
-           ("spx_fft.hip", ["-DSPX_PART=3"]), ("spx_ops.hip", []), ("spx_api.hip", []),
-           ("spx_noalloc.hip", []), ("spx_wall.hip", [])]
+# (source, defines): spx_fft.hip is compiled in parts (see its header), the longest first
+SOURCES = [("spx_fft.hip", [f"-DSPX_PART={n}"]) for n in (6, 16, 8, 3, 12, 2, 7, 5, 13, 9, 4, 10, 1, 14, 15, 11)] + [
+    ("spx_ops.hip", []), ("spx_api.hip", []), ("spx_noalloc.hip", []), ("spx_wall.hip", [])]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -303,13 +303,14 @@ struct ProfScope {
 // csize: bytes per complex element (16: float64 tables, 8: float32 tables)
 // want_lines: lines per workgroup at most (0: as many as max_block threads
 // hold); the tables plus line buffers stay within lds_budget bytes
+// force_m > 0: Bluestein on that length, whatever n is
 int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_block = 256,
-                   size_t lds_budget = 64 * 1024);
-// the one-wavefront-per-line plan of length n (f.wave < 0 if none is compiled)
-int build_wave_fft(LineFFTHost& f, int n, int csize);
-// mark an x / y line plan of 512 points (one wavefront per line) for the
-// compiled 512-point wave plan
-void attach_xy_wave(LineFFTHost& f, int csize);
+                   size_t lds_budget = 64 * 1024, int force_m = 0);
+// the compiled plan of z lines of length n (f.wave < 0 if there is none);
+// same_bits: only those that give the engine's results to the bit
+int build_wave_fft(LineFFTHost& f, int n, int csize, bool same_bits);
+// run an x / y line plan by the compiled plan of its length, where there is one
+int attach_xy_wave(LineFFTHost& f, int csize);
 void free_line_fft(LineFFTHost& f);
 
 // z transforms in place on S (contiguous lines).

@@ -485,8 +485,13 @@ __device__ __forceinline__ void conv_passes(cpx<T>* a, cpx<T>* b, const LineFFT<
 // __syncthreads publishes them): twiddles at [0, M); Bluestein: filter at
 // [M, 2M), chirp at [2M, 2M+n); Rader: filter at [M, 2M), then the 2M
 // permutation indices as ints.
-template <typename T>
+// Compiled plans (RS >= RS_GTAB + 1): their own table of f.tab entries.
+template <int RS, typename T>
 __device__ __forceinline__ void stage_twiddles(cpx<T>* tws, const LineFFT<cpx<T>>& f) {
+  if constexpr (RS > RS_GTAB) {
+    for (int m = threadIdx.x; m < f.tab; m += blockDim.x) tws[m] = f.tw[m];
+    return;
+  }
   for (int m = threadIdx.x; m < f.M; m += blockDim.x) tws[m] = f.tw[m];
   if (f.mode == 0 || f.tab == f.M) return;  // RS_GTAB plans read them from global memory
   for (int m = threadIdx.x; m < f.M; m += blockDim.x) tws[f.M + m] = f.bfil[m];

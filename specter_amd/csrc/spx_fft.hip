@@ -3,10 +3,12 @@
 // gradient-product x pass of gradre/advect, and the z-line kernels of the
 // boundary / projection / diagnostics stages.
 //
-// Build: the host part of this file is compiled in three parts so that the
-// kernel instantiations build in parallel (SPX_PART = 1: plan tables and z
-// transforms, 2: y and x transforms, 3: boundary, projection and diagnostics
-// launchers); without SPX_PART everything is compiled in one unit.
+// Build: the host part of this file is compiled in parts so that the kernel
+// instantiations build in parallel (SPX_PART = 1: plan tables, in-place z
+// transforms and the entry points of the passes, 3: boundary and projection
+// launchers, 16: magnetic walls and pressure, 8: diagnostics; in float64 / float32 4 / 5: forward z pass, 6 / 7:
+// backward z pass, 2 / 9: y pass, 10 / 11: x passes, 12 / 13 and 14 / 15:
+// gradient products); without SPX_PART everything is compiled in one unit.
 //
 // Precision: the transform kernels are templated on their arithmetic / buffer
 // type T (double; float for the nonlinear pipeline of mixed-precision plans,
@@ -41,7 +43,7 @@ __device__ __forceinline__ cpx<TO> ccast(cpx<TI> v) { return mkc<TO>(TO(v.x), TO
   extern __shared__ unsigned char smem[];                        \
   CT* const tws = reinterpret_cast<CT*>(smem);                   \
   CT* const lds = tws + (f).tab;                                 \
-  stage_twiddles(tws, (f));                                      \
+  stage_twiddles<RS>(tws, (f));                                   \
   const int tid = threadIdx.x;                                   \
   const int line = tid >> (f).lgtpl, lane = tid & ((f).tpl - 1); \
   CT* const xl = lds + line * (f).ldl;                           \
@@ -60,9 +62,7 @@ __device__ __forceinline__ void zline_dft(cpx<T>* x, const LineFFT<cpx<T>>& f, c
                                           int lane) {
   if constexpr (RS >= RS_WAVE) {
     using P = typename WavePlanOf<RS>::type;
-    // float32-only plans are never built for float64 lines (wave_plan_for):
-    // their float64 instances are not compiled
-    if constexpr (sizeof(T) == 4 || P::f64) P::template dft<T>(x, lane, tw, f.bfil, f.chirp);
+    P::template dft<T>(x, lane, tw, f.n, f.bfil, f.chirp, f.perm);
     __syncthreads();
   } else {
     line_dft<T, RS>(x, f, tw, lane);
@@ -78,7 +78,7 @@ __device__ __forceinline__ void line_fft_nosync(cpx<T>* x, const LineFFT<cpx<T>>
   if constexpr (RS >= RS_WAVE) {
     using P = typename WavePlanOf<RS>::type;
     static_assert(P::mode == 0, "direct plans only");
-    P::template dft<T>(x, lane, tw, nullptr, nullptr);
+    P::template dft<T>(x, lane, tw, f.n, nullptr, nullptr, nullptr);
   } else {
     fft_lds<T, RS>(x, f, tw, lane);
   }
@@ -87,8 +87,20 @@ __device__ __forceinline__ void line_fft_nosync(cpx<T>* x, const LineFFT<cpx<T>>
 // line elements a thread holds in registers in the z kernels (n <= KN * tpl)
 template <int RS>
 constexpr int keep_n() {
-  if constexpr (RS >= RS_WAVE) return (WavePlanOf<RS>::type::n + 63) / 64;
-  else return KEEP;
+  if constexpr (RS >= RS_WAVE) {
+    using P = typename WavePlanOf<RS>::type;
+    return (P::nmax + P::lanes - 1) / P::lanes;
+  } else {
+    return KEEP;
+  }
+}
+
+// waves per SIMD of a line kernel's register budget (compiled plans: what
+// their LDS leaves room for)
+template <typename T, int RS>
+constexpr int min_waves() {
+  if constexpr (RS >= RS_WAVE) return WavePlanOf<RS>::type::waves(2 * sizeof(T));
+  else return 1;
 }
 
 // idx = first, first + step, ... < count: wr(idx, rd(idx)).  KN > 0 (the
@@ -215,7 +227,7 @@ struct ZX2S {
 // is evaluated from them, so the float32 roundoff of the other planes is not
 // amplified by the continuation.
 template <typename T, int RS, bool BND>
-__global__ void __launch_bounds__(kMaxBlock) k_z_x2s(ZX2S<T> a, LineFFT<cpx<T>> f, int nkx,
+__global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_z_x2s(ZX2S<T> a, LineFFT<cpx<T>> f, int nkx,
                                                int ny, int np, int nofft,
                                                const double* __restrict__ dir, int C, int d,
                                                long xstride) {
@@ -267,7 +279,8 @@ __global__ void __launch_bounds__(kMaxBlock) k_z_x2s(ZX2S<T> a, LineFFT<cpx<T>> 
         const int q = t >> f.lgnl, l = t & (f.nl - 1), e = e0 + l;
         const int z = q < d ? q : np - d2 + q;
         const cpx<double> v = e < nlines ? xb[e + pl * q] : mkc<double>(0, 0);
-        lds[l * f.ldl + z] = mkc<T>(T(v.x), T(v.y));
+        // (a point of both blocks, np < 2d, is the top one's)
+        if (q >= d || z < np - d) lds[l * f.ldl + z] = mkc<T>(T(v.x), T(v.y));
         bl[l * d2 + q] = v;
       }
       __syncthreads();
@@ -417,7 +430,7 @@ struct ZS2X {
 };
 
 template <typename T, int RS, bool DUAL, typename TI>
-__global__ void __launch_bounds__(kMaxBlock) k_z_s2x(ZS2X<T, TI> a, LineFFT<cpx<T>> f, int nkx,
+__global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_z_s2x(ZS2X<T, TI> a, LineFFT<cpx<T>> f, int nkx,
                                                int ny, int nzout, int dirn, int nofft,
                                                const double* __restrict__ kx,
                                                const double* __restrict__ ky,
@@ -535,7 +548,7 @@ struct YFields {
 };
 
 template <typename T, int RS, bool DUAL>
-__global__ void __launch_bounds__(kMaxBlock) k_y(YFields<T> a, LineFFT<cpx<T>> f, int nkx,
+__global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_y(YFields<T> a, LineFFT<cpx<T>> f, int nkx,
                                            int ny, long nlines, int forward,
                                            const double* __restrict__ ky, int npy, int Cy, int oy,
                                            const double* __restrict__ diry) {
@@ -579,10 +592,11 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(YFields<T> a, LineFFT<cpx<T>> f
     fc_continue_lds(lds, f.nl, f.ldl, npy, Cy, oy, diry);
     __syncthreads();
   }
-  Cp keep[DUAL ? KEEP : 1];
+  constexpr int KN = keep_n<RS>();
+  Cp keep[DUAL ? KN : 1];
   if constexpr (DUAL) {
 #pragma unroll
-    for (int q = 0; q < KEEP; ++q) {
+    for (int q = 0; q < KN; ++q) {
       const int k = lane + q * f.tpl;
       if (k < ny) keep[q] = xl[k];
     }
@@ -604,7 +618,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_y(YFields<T> a, LineFFT<cpx<T>> f
     if (!a.y2[blockIdx.y]) return;  // uniform per workgroup
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < KEEP; ++q) {
+    for (int q = 0; q < KN; ++q) {
       const int k = lane + q * f.tpl;
       if (k < ny) xl[k] = cconj(ikmul(T(ky[k]), cconj(keep[q])));
     }
@@ -701,7 +715,27 @@ __device__ __forceinline__ cpx<T> c2r_pair_value(cpx<T> A, cpx<T> B, int m, int 
   return v;
 }
 
-template <typename T, int KN = 0, int CH = KN>
+// (the same operations without fused multiply-adds)
+template <typename T>
+__device__ __forceinline__ cpx<T> c2r_pair_value_nofma(cpx<T> A, cpx<T> B, int m, int k, int h,
+                                                       double kxk) {
+#pragma clang fp contract(off)
+  const T q = T(kxk);
+  A = mkc<T>(-(q * A.y), q * A.x);
+  B = mkc<T>(-(q * B.y), q * B.x);
+  if (k == 0 || k == h) {
+    A.y = 0;
+    B.y = 0;
+  }
+  cpx<T> v = m > h ? mkc<T>(A.x + B.y, -A.y + B.x) : mkc<T>(A.x - B.y, A.y + B.x);
+  v.y = -v.y;
+  return v;
+}
+
+// FMA: the derivative's products may be fused into the combination (dirx
+// known at compile time); else they are rounded first, whatever the compiler
+// does with the branch.
+template <typename T, int KN = 0, int CH = KN, bool FMA = true>
 __device__ __forceinline__ void load_c2r_pair(cpx<T>* xl, const cpx<T>* __restrict__ a0, int nkx,
                                               int nx, int lane, int tpl, bool ok, int dirx,
                                               const double* __restrict__ kx) {
@@ -729,7 +763,12 @@ __device__ __forceinline__ void load_c2r_pair(cpx<T>* xl, const cpx<T>* __restri
       for (int q = 0; q < CH; ++q) {
         const int m = lane + (c0 + q) * tpl;
         const int k = m > h ? nx - m : m;
-        if (m < nx) xl[m] = ok ? c2r_pair_value(A[q], B[q], m, k, h, dirx, kk[q]) : mkc<T>(0, 0);
+        if (m < nx) {
+          cpx<T> v;
+          if (!FMA && dirx) v = c2r_pair_value_nofma(A[q], B[q], m, k, h, kk[q]);
+          else v = c2r_pair_value(A[q], B[q], m, k, h, FMA ? dirx : 0, kk[q]);
+          xl[m] = ok ? v : mkc<T>(0, 0);
+        }
       }
     }
   } else {
@@ -766,6 +805,25 @@ constexpr int batch_n() {
 template <typename T, int RS>
 constexpr int xg_batch() {
   return batch_n<RS>();
+}
+// x lines of a plan whose fused x stage keeps its row pair's velocity in
+// registers: powers of two of the general engine (its other radix families
+// spill), compiled plans with few points per lane
+template <typename T, int RS>
+constexpr bool xfused_ok() {
+  if constexpr (RS >= RS_WAVE) return keep_n<RS>() <= (sizeof(T) == 4 ? 16 : 10);
+  else return RS == RS_POW2;
+}
+template <int RS>
+constexpr bool xline_pow2() {
+  if constexpr (RS >= RS_WAVE) return (WavePlanOf<RS>::type::m & (WavePlanOf<RS>::type::m - 1)) == 0;
+  else return RS == RS_POW2;
+}
+// whether d/dx in k_xgrad_prod fuses the derivative's product (load_c2r_pair)
+template <int RS>
+constexpr bool xprod_fma() {
+  if constexpr (RS >= RS_WAVE) return WavePlanOf<RS>::type::natural;
+  else return false;
 }
 template <typename T, int RS>
 constexpr int xg_chunk() {
@@ -827,16 +885,21 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cp
   const bool ok = p < npairs;
   const long ro = long(nx) * (2 * (ok ? p : 0));
   const long co = long(nkx) * (2 * (ok ? p : 0));
-  T accA[KEEP], accB[KEEP];
+  constexpr int KX = keep_n<RS>();
+  T accA[KX], accB[KX];
   const Cp* srcs[3] = {a.yv[blockIdx.y], a.yy[blockIdx.y], a.xz[blockIdx.y]};
   for (int r = 0; r < 3; ++r) {
-    load_c2r_pair<T, batch_n<RS>()>(xl, srcs[r] + co, nkx, nx, lane, f.tpl, ok, r == 0 ? 1 : 0, kx);
+    if (xprod_fma<RS>() && r == 0)
+      load_c2r_pair<T, batch_n<RS>()>(xl, srcs[0] + co, nkx, nx, lane, f.tpl, ok, 1, kx);
+    else
+      load_c2r_pair<T, batch_n<RS>(), batch_n<RS>(), false>(xl, srcs[r] + co, nkx, nx, lane,
+                                                            f.tpl, ok, r == 0 ? 1 : 0, kx);
     // the velocity values this thread multiplies with, loaded before the
     // transform so that their latency overlaps it
     const T* m = a.vel[r] + ro;
-    T ma[KEEP], mb[KEEP];
+    T ma[KX], mb[KX];
 #pragma unroll
-    for (int q = 0; q < KEEP; ++q) {
+    for (int q = 0; q < KX; ++q) {
       const int x = lane + q * f.tpl;
       const bool in = x < nx && ok;
       ma[q] = in ? m[x] : T(0);
@@ -845,7 +908,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cp
     __syncthreads();
     zline_dft<T, RS>(xl, f, tws, lane);
 #pragma unroll
-    for (int q = 0; q < KEEP; ++q) {
+    for (int q = 0; q < KX; ++q) {
       const int x = lane + q * f.tpl;
       if (x < nx) {
         const Cp z = xl[x];
@@ -865,7 +928,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cp
     __syncthreads();
   }
 #pragma unroll
-  for (int q = 0; q < KEEP; ++q) {
+  for (int q = 0; q < KX; ++q) {
     const int x = lane + q * f.tpl;
     if (x < nx) xl[x] = mkc<T>(accA[q], accB[q]);
   }
@@ -904,7 +967,9 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
   const bool ok = p < npairs;
   const long ro = long(nx) * (2 * (ok ? p : 0));
   const long co = long(nkx) * (2 * (ok ? p : 0));
-  T vel[3][2][KEEP];
+  constexpr int KX = keep_n<RS>();
+  constexpr bool pow2 = xline_pow2<RS>();
+  T vel[3][2][KX];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>()>(xl, a.yv[c] + co, nkx, nx, lane, f.tpl, ok, 0, kx);
@@ -914,7 +979,7 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
     line_fft_nosync<T, RS>(xl, f, tws, lane);
     line_sync(f.tpl);
 #pragma unroll
-    for (int q = 0; q < KEEP; ++q) {
+    for (int q = 0; q < KX; ++q) {
       const int x = lane + q * f.tpl;
       vel[c][0][q] = vel[c][1][q] = T(0);
       if (x < nx) {
@@ -931,16 +996,22 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
   }
 #pragma unroll 1
   for (int c = 0; c < nf; ++c) {
-    T accA[KEEP], accB[KEEP];
+    T accA[KX], accB[KX];
     const Cp* srcs[3] = {a.yv[c], a.yy[c], a.xz[c]};
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
-      load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>()>(xl, srcs[r] + co, nkx, nx, lane, f.tpl, ok, r == 0 ? 1 : 0, kx);
+      // (the scalar's and other lengths' d/dx are k_xgrad_prod's to the bit)
+      if (r == 0 && (!pow2 || c == 3))
+        load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>(), false>(
+            xl, srcs[r] + co, nkx, nx, lane, f.tpl, ok, 1, kx);
+      else
+        load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>()>(xl, srcs[r] + co, nkx, nx, lane,
+                                                              f.tpl, ok, r == 0 ? 1 : 0, kx);
       line_sync(f.tpl);
       line_fft_nosync<T, RS>(xl, f, tws, lane);
       line_sync(f.tpl);
 #pragma unroll
-      for (int q = 0; q < KEEP; ++q) {
+      for (int q = 0; q < KX; ++q) {
         const int x = lane + q * f.tpl;
         if (x < nx) {
           const Cp z = xl[x];
@@ -1043,7 +1114,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_bwall(Cd* __restrict__ a0, Cd* __
   const bool ok = ln < nlines;
   for (int k = lane; k < n; k += f.tpl) xl[k] = ok ? cconj(V[ln * n + k]) : mkc<double>(0, 0);
   __syncthreads();
-  line_dft<double, RS>(xl, f, tws, lane);
+  zline_dft<double, RS>(xl, f, tws, lane);
   for (int k = lane; k < np; k += f.tpl) xl[k] = cscale(cconj(xl[k]), invn);
   __syncthreads();
   // lane 0: the wall at z = 0, lane 1: z = Lz (their stencils do not overlap
@@ -1069,7 +1140,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_bwall(Cd* __restrict__ a0, Cd* __
   __syncthreads();
   fc_continue_lds(lds, f.nl, f.ldl, np, C, d, dir);
   __syncthreads();
-  line_dft<double, RS>(xl, f, tws, lane);
+  zline_dft<double, RS>(xl, f, tws, lane);
   if (ok)
     for (int k = lane; k < n; k += f.tpl) V[ln * n + k] = xl[k];
 }
@@ -1570,8 +1641,8 @@ __global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(LinCombDev<TS> lc,
     if (mode == 1) xb[k] = cconj(w);
   }
   __syncthreads();
-  line_dft<double, RS>(xl, f, tws, lane);
-  if (mode == 1) line_dft<double, RS>(xb, f, tws, lane);
+  zline_dft<double, RS>(xl, f, tws, lane);
+  if (mode == 1) zline_dft<double, RS>(xb, f, tws, lane);
   if (mode == 2) {
     if (lane == 0 && ok) {
       const Cd b = xl[0], t = xl[np - 1];
@@ -1651,6 +1722,13 @@ static bool smooth7(int m) {
   return m == 1;
 }
 
+// Bluestein length of the engine: the smallest M >= 2n - 1 of primes <= 7
+static int bluestein_m(int n) {
+  int M = 2 * n - 1;
+  while (!smooth7(M)) ++M;
+  return M;
+}
+
 static bool is_prime(int n) {
   if (n < 2) return false;
   for (int d = 2; d * d <= n; ++d)
@@ -1726,9 +1804,9 @@ static void dft_ld(const std::vector<long double>& xr, const std::vector<long do
   out.assign(2 * size_t(M), 0.0);
   for (int k = 0; k < M; ++k) {
     long double sr = 0, si = 0;
-    for (int m = 0; m < M; ++m) {
+    // idx = m k mod M, counted up: the 64-bit remainder took most of the time
+    for (int m = 0, idx = 0; m < M; ++m, idx += idx + k < M ? k : k - M) {
       if (xr[m] == 0.0L && xi[m] == 0.0L) continue;
-      const int idx = int((long long)m * k % M);
       sr += xr[m] * wr[idx] - xi[m] * wi[idx];
       si += xr[m] * wi[idx] + xi[m] * wr[idx];
     }
@@ -1771,10 +1849,14 @@ void clear_tunes() {
 }
 
 int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_block,
-                   size_t lds_budget) {
+                   size_t lds_budget, int force_m) {
   std::vector<int> fac;
   f.n = n;
-  if (factor_small(n, fac)) {
+  if (force_m > 0) {
+    f.mode = 1;
+    f.M = force_m;
+    factor_small(f.M, fac);
+  } else if (factor_small(n, fac)) {
     f.mode = 0;
     f.M = n;
   } else if (is_prime(n) && factor_small(n - 1, fac)) {
@@ -1782,10 +1864,8 @@ int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_blo
     f.M = n - 1;
   } else {
     f.mode = 1;
-    int M = 2 * n - 1;
-    while (!smooth7(M)) ++M;
-    f.M = M;
-    factor_small(M, fac);
+    f.M = bluestein_m(n);
+    factor_small(f.M, fac);
   }
   if (int(fac.size()) > kMaxStages) return fail(SPX_ERR_UNSUPPORTED, "FFT length has too many factors");
   f.nstage = int(fac.size());
@@ -1860,7 +1940,7 @@ int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_blo
     // chirp w[m] = exp(-pi i (m^2 mod 2n)/n)
     const long double PI = PI2 / 2;
     std::vector<long double> cr(n), ci(n);
-    std::vector<double> ch(2 * size_t(n));
+    std::vector<double> ch(2 * size_t(M), 0.0);  // zeros from n on (the wave plans read M entries)
     for (int m = 0; m < n; ++m) {
       const long long r = (long long)m * m % (2LL * n);
       cr[m] = cosl(PI * (long double)r / (long double)n);
@@ -1906,43 +1986,129 @@ int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_blo
   return SPX_OK;
 }
 
-int build_wave_fft(LineFFTHost& f, int n, int csize) {
+// sizes of the compiled plans, indexed by plan number
+struct WaveInfo {
+  int n, m, lanes, mode, nmax, ldl, tab, twm, lines16, lines8, npass;
+  const int* radix;
+  bool natural;
+  int lines(int csize) const { return csize == 16 ? lines16 : lines8; }
+};
+template <int W = 0>
+static void wave_infos(WaveInfo* o) {
+  using P = typename WavePlanN<W>::type;
+  o[W] = WaveInfo{P::n,   P::m,   P::lanes,          P::mode,          P::nmax,  P::ldl,
+                  P::tab, P::twm, wave_lines<W>(16), wave_lines<W>(8), P::npass, P::radix,
+                  P::natural};
+  if constexpr (W + 1 < kWavePlans) wave_infos<W + 1>(o);
+}
+static const WaveInfo* wave_info() {
+  static const struct Tab {
+    WaveInfo t[kWavePlans];
+    Tab() { wave_infos<>(t); }
+  } tab;
+  return tab.t;
+}
+// shape of a line plan run by compiled plan w, with the plan's table (the
+// engine's W_M in the order of the passes, stage_twiddle, then W_9^0..4) in the
+// place of the engine's
+static int set_wave(LineFFTHost& h, int w, int csize) {
+  const WaveInfo& i = wave_info()[w];
+  h.wave = w;
+  h.tpl = i.lanes;
+  h.nl = i.lines(csize);
+  for (h.lgtpl = 0; (1 << h.lgtpl) < h.tpl;) ++h.lgtpl;
+  for (h.lgnl = 0; (1 << h.lgnl) < h.nl;) ++h.lgnl;
+  h.ldl = i.ldl;
+  h.tab = i.tab;  // staged in LDS; filter, chirp and indices in global memory
+  if (i.natural) return SPX_OK;  // the engine's own table
+  const long double PI2 = 6.283185307179586476925286766559005768L;
+  const int M = h.M;
+  std::vector<double> tw(2 * size_t(i.tab), 0.0);
+  auto put = [&](int at, int m) {  // entry at <- W_M^m
+    tw[2 * at] = double(cosl(PI2 * (long double)m / (long double)M));
+    tw[2 * at + 1] = double(-sinl(PI2 * (long double)m / (long double)M));
+  };
+  int Ns = 1;
+  for (int p = 0; p < i.npass; ++p) {
+    const int R = i.radix[p];
+    for (int r = 1; r < R; ++r)
+      for (int jm = 0; jm < Ns; ++jm) put(r * Ns + jm - 1, r * jm * (M / (Ns * R)));
+    Ns *= R;
+  }
+  if (M % 9 == 0)
+    for (int q = 0; q < 5; ++q) put(M + q, q * (M / 9));
+  if (h.tw) (void)hipFree(h.tw);
+  h.tw = nullptr;
+  h.bytes -= size_t(M) * csize;
+  return upload_table(&h.tw, tw, csize, &h.bytes);
+}
+
+// The compiled plan of a z line: the direct or Rader plan of exactly this
+// length; for the other lengths with a prime factor above 13 the smallest
+// Bluestein M >= 2n - 1.  Rader lengths without a plan stay on the engine: its
+// two (n-1)-point FFTs are more accurate in float32 (gradre's error at 89 and
+// 281 1.53e-7 and 1.74e-7 through Bluestein, 1.26e-7 and 1.49e-7 through
+// Rader), and smooth lengths without a plan because one FFT beats two.
+// same_bits (mixed plans): only plans that run the engine's own arithmetic
+// (its radices, table twiddles and Bluestein M), and those the lines always
+// had.  The float32 nonlinear term's rounding is amplified by the pressure of
+// the next stages, and a last-bit change anywhere redraws all of it (192^3,
+// two steps: pressure 5e-6 in the norm, up to 1e-3 of its rms in single
+// modes), so a mixed run keeps its bits instead.
+int build_wave_fft(LineFFTHost& f, int n, int csize, bool same_bits) {
   f = LineFFTHost();
   if (const char* e = std::getenv("SPX_WAVE"))
     if (e[0] == '0') return SPX_OK;
   LineFFTHost h;
-  if (int rc = build_line_fft(h, n, csize, 0)) {
+  std::vector<int> fac;
+  const bool direct = factor_small(n, fac);
+  const bool rader = !direct && is_prime(n) && factor_small(n - 1, fac);
+  constexpr int kFixedZ = 3;  // plans 0 .. 2: z lines of 537, 539, 1049
+  int w = -1;
+  for (int q = 0; q < kWavePlans; ++q) {
+    const WaveInfo& i = wave_info()[q];
+    if (!i.lines(csize) || (same_bits && i.twm != 0 && i.n == 0)) continue;
+    if (i.n == n && q < kFixedZ) {  // a plan of this length alone
+      w = q;
+      break;
+    }
+    if (i.n != 0) continue;
+    if (direct) {
+      if (i.mode == 0 && i.m == n) w = q;
+    } else if (rader) {
+      if (i.mode == 2 && i.m == n - 1) w = q;
+    } else if (i.mode == 1 && n <= i.nmax && (w < 0 || i.m < wave_info()[w].m) &&
+               (!same_bits || i.m == bluestein_m(n))) {
+      w = q;
+    }
+  }
+  if (w < 0) return SPX_OK;
+  const int blu = wave_info()[w].mode == 1 ? wave_info()[w].m : 0;
+  if (int rc = build_line_fft(h, n, csize, 0, 256, 64 * 1024, blu)) {
     free_line_fft(h);
     return rc;
   }
-  // the z launch macro lists plans 0..2 (plan 3 is the x / y lines' plan)
-  const int w = wave_plan_for(h.n, h.M, h.mode, csize);
-  if (w < 0 || w > 2) {
+  if (int rc = set_wave(h, w, csize)) {
     free_line_fft(h);
-    return SPX_OK;
-  }
-  // one wavefront per line, 8 lines per workgroup; twiddles staged in LDS,
-  // the Bluestein filter and chirp read from global memory
-  h.wave = w;
-  h.tpl = 64;
-  h.lgtpl = 6;
-  h.nl = 8;
-  h.lgnl = 3;
-  h.ldl = h.M + 1;
-  h.tab = h.M;
-  if (h.lds_bytes(size_t(csize)) > 160 * 1024) {
-    free_line_fft(h);
-    return SPX_OK;
+    return rc;
   }
   f = h;
   return SPX_OK;
 }
 
-void attach_xy_wave(LineFFTHost& f, int csize) {
+int attach_xy_wave(LineFFTHost& f, int csize) {
   for (const char* v : {"SPX_WAVE", "SPX_WAVE_XY"})
     if (const char* e = std::getenv(v))
-      if (e[0] == '0') return;
-  if (f.mode == 0 && f.tpl == 64 && wave_plan_for(f.n, f.M, 0, csize) == 3) f.wave = 3;
+      if (e[0] == '0') return SPX_OK;
+  if (f.mode != 0) return SPX_OK;
+  for (int q = 0; q < kWavePlans; ++q) {
+    const WaveInfo& i = wave_info()[q];
+    if (i.mode != 0 || i.m != f.n || !i.lines(csize)) continue;
+    if (!i.natural) return set_wave(f, q, csize);
+    if (f.n == 512 && f.tpl == 64) f.wave = q;  // the engine's launch shape
+    return SPX_OK;
+  }
+  return SPX_OK;
 }
 
 void free_line_fft(LineFFTHost& f) {
@@ -1983,104 +2149,56 @@ static int lds_limit(K kernel, size_t bytes) {
   return rs;
 }
 
+// fn(std::integral_constant<int, RS>) for the radix set of a general plan
+template <typename F>
+static int with_general(const LineFFTHost& f, F&& fn) {
+  switch (rset_of(f)) {
+    case RS_POW2: return fn(std::integral_constant<int, RS_POW2>{});
+    case RS_SMOOTH: return fn(std::integral_constant<int, RS_SMOOTH>{});
+    case RS_ALL: return fn(std::integral_constant<int, RS_ALL>{});
+    case RS_GTAB: return fn(std::integral_constant<int, RS_GTAB>{});
+    default: return fail(SPX_ERR_STATE, "wave line plan passed to a general kernel");
+  }
+}
+// the same for any plan, compiled ones included, with csize-byte elements
+template <int CS, bool DIRECT, int W = 0, int END = kWavePlans, typename F>
+static int with_wave(int w, F&& fn) {
+  if constexpr (W < END) {
+    if constexpr (wave_lines<W>(CS) > 0 && (!DIRECT || WavePlanN<W>::type::mode == 0)) {
+      if (w == W) return fn(std::integral_constant<int, RS_WAVE + W>{});
+    }
+    return with_wave<CS, DIRECT, W + 1, END>(w, fn);
+  } else {
+    return fail(SPX_ERR_STATE, "line plan without a compiled kernel family");
+  }
+}
+template <int CS, typename F>
+static int with_z(const LineFFTHost& f, F&& fn) {
+  return f.wave >= 0 ? with_wave<CS, false>(f.wave, fn) : with_general(f, fn);
+}
+constexpr int kInplacePlans = 2;  // 1080 and 539
+template <typename F>
+[[maybe_unused]] static int with_inplace(const LineFFTHost& f, F&& fn) {
+  return f.wave >= 0 ? with_wave<16, false, 0, kInplacePlans>(f.wave, fn) : with_general(f, fn);
+}
+// x / y lines: compiled plans of direct lengths
+template <int CS, typename F>
+static int with_xy(const LineFFTHost& f, F&& fn) {
+  return f.wave >= 0 ? with_wave<CS, true>(f.wave, fn) : with_general(f, fn);
+}
 #define SPX_COMMA ,
-// launch the instance KER<TY, RS TARGS> compiled for the plan's radix set
-#define SPX_LAUNCH_RS(F, KER, TY, TARGS, GRID, BLOCK, LDS, STREAM, ...)                      \
+// launch the instance KER<TY, RS TARGS> of the dispatcher DISP(F, ...)
+#define SPX_LAUNCH(DISP, F, KER, TY, TARGS, GRID, BLOCK, LDS, STREAM, ...)                   \
   do {                                                                                       \
-    const int rs_ = rset_of(F);                                                              \
-    if (rs_ == RS_POW2) {                                                                    \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_POW2 TARGS>, (LDS))) return rc_;           \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_POW2 TARGS>), GRID, BLOCK, LDS, STREAM,        \
+    const int lrc_ = DISP(F, [&](auto rs_) -> int {                                          \
+      constexpr int RS_ = decltype(rs_)::value;                                              \
+      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_ TARGS>, (LDS))) return rc_;               \
+      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_ TARGS>), GRID, BLOCK, LDS, STREAM,            \
                          __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_SMOOTH) {                                                           \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_SMOOTH TARGS>, (LDS))) return rc_;         \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_SMOOTH TARGS>), GRID, BLOCK, LDS, STREAM,      \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_ALL) {                                                              \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_ALL TARGS>, (LDS))) return rc_;            \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_ALL TARGS>), GRID, BLOCK, LDS, STREAM,         \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_GTAB) {                                                             \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_GTAB TARGS>, (LDS))) return rc_;           \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_GTAB TARGS>), GRID, BLOCK, LDS, STREAM,        \
-                         __VA_ARGS__);                                                       \
-    } else {                                                                                 \
-      return fail(SPX_ERR_STATE, "wave line plan passed to a general kernel");               \
-    }                                                                                        \
+      return SPX_OK;                                                                         \
+    });                                                                                      \
+    if (lrc_) return lrc_;                                                                   \
   } while (0)
-
-// x / y transform launch: the 512-point wave plan (RS_WAVE + 3) or the
-// general families (spelled out: TARGS cannot be forwarded to another macro)
-#define SPX_LAUNCH_XY(F, KER, TY, TARGS, GRID, BLOCK, LDS, STREAM, ...)                      \
-  do {                                                                                       \
-    const int rs_ = rset_of(F);                                                              \
-    if (rs_ == RS_WAVE + 3) {                                                                \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_WAVE + 3 TARGS>, (LDS))) return rc_;       \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_WAVE + 3 TARGS>), GRID, BLOCK, LDS, STREAM,    \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_POW2) {                                                             \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_POW2 TARGS>, (LDS))) return rc_;           \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_POW2 TARGS>), GRID, BLOCK, LDS, STREAM,        \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_SMOOTH) {                                                           \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_SMOOTH TARGS>, (LDS))) return rc_;         \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_SMOOTH TARGS>), GRID, BLOCK, LDS, STREAM,      \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_ALL) {                                                              \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_ALL TARGS>, (LDS))) return rc_;            \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_ALL TARGS>), GRID, BLOCK, LDS, STREAM,         \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_GTAB) {                                                             \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_GTAB TARGS>, (LDS))) return rc_;           \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_GTAB TARGS>), GRID, BLOCK, LDS, STREAM,        \
-                         __VA_ARGS__);                                                       \
-    } else {                                                                                 \
-      return fail(SPX_ERR_STATE, "x/y line plan without a compiled kernel family");          \
-    }                                                                                        \
-  } while (0)
-
-// z-transform launch: the wave-plan instance when the plan has one, else as
-// SPX_LAUNCH_RS (spelled out: TARGS cannot be forwarded to another macro)
-#define SPX_LAUNCH_Z(F, KER, TY, TARGS, GRID, BLOCK, LDS, STREAM, ...)                       \
-  do {                                                                                       \
-    const int rs_ = rset_of(F);                                                              \
-    if (rs_ == RS_WAVE + 0) {                                                                \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_WAVE + 0 TARGS>, (LDS))) return rc_;       \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_WAVE + 0 TARGS>), GRID, BLOCK, LDS, STREAM,    \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_WAVE + 1) {                                                         \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_WAVE + 1 TARGS>, (LDS))) return rc_;       \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_WAVE + 1 TARGS>), GRID, BLOCK, LDS, STREAM,    \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_WAVE + 2) {                                                         \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_WAVE + 2 TARGS>, (LDS))) return rc_;       \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_WAVE + 2 TARGS>), GRID, BLOCK, LDS, STREAM,    \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_WAVE + 3) {                                                         \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_WAVE + 3 TARGS>, (LDS))) return rc_;       \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_WAVE + 3 TARGS>), GRID, BLOCK, LDS, STREAM,    \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_POW2) {                                                             \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_POW2 TARGS>, (LDS))) return rc_;           \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_POW2 TARGS>), GRID, BLOCK, LDS, STREAM,        \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_SMOOTH) {                                                           \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_SMOOTH TARGS>, (LDS))) return rc_;         \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_SMOOTH TARGS>), GRID, BLOCK, LDS, STREAM,      \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_ALL) {                                                              \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_ALL TARGS>, (LDS))) return rc_;            \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_ALL TARGS>), GRID, BLOCK, LDS, STREAM,         \
-                         __VA_ARGS__);                                                       \
-    } else if (rs_ == RS_GTAB) {                                                             \
-      if (int rc_ = lds_limit(KER<TY SPX_COMMA RS_GTAB TARGS>, (LDS))) return rc_;           \
-      hipLaunchKernelGGL((KER<TY SPX_COMMA RS_GTAB TARGS>), GRID, BLOCK, LDS, STREAM,        \
-                         __VA_ARGS__);                                                       \
-    } else {                                                                                 \
-      return fail(SPX_ERR_STATE, "z line plan without a compiled kernel family");            \
-    }                                                                                        \
-  } while (0)
-
 template <typename T>
 static inline cpx<T>* C_(void* p) { return static_cast<cpx<T>*>(p); }
 template <typename T>
@@ -2104,12 +2222,13 @@ static inline const LineFFTHost& fzt(const spx_plan* p, bool lo) {
 
 #if !defined(SPX_PART) || SPX_PART == 1
 int zfft_inplace(spx_plan* p, void* S, int forward, int cont, double scale) {
-  const LineFFTHost& f = fzt(p, false);
+  // the public one-dimensional transforms: compiled plans of the long lines only
+  const LineFFTHost& f = p->fzw.wave >= 0 && p->fzw.wave < kInplacePlans ? p->fzw : p->fz;
   const long nlines = p->wlines();
   const unsigned nb = unsigned((nlines + f.nl - 1) / f.nl);
   const int C = p->g.Cz, d = p->g.oz;
   ProfScope ps_(p, "z_inplace", double(p->wnc()) * 2.0 * 16.0);
-  SPX_LAUNCH_Z(f, k_z_inplace, double, , dim3(nb), blk(f), f.lds_bytes(16), p->stream,
+  SPX_LAUNCH(with_inplace, f, k_z_inplace, double, , dim3(nb), blk(f), f.lds_bytes(16), p->stream,
                 C_<double>(S), nlines, f.dev<Cd>(), p->np, forward, (cont && C > 0) ? 1 : 0,
                 scale, p->d_dir, C, d);
   SPX_CHECK_LAUNCH();
@@ -2128,8 +2247,15 @@ int fc_continue_only(spx_plan* p, void* S) {
   return SPX_OK;
 }
 
+#endif  // SPX_PART 1 (z transforms in place)
+
 template <typename T>
-static int zfft_x2s_t(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft,
+struct ZForward {
+  static int run(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft, const
+                 LineFFTHost& f, const void* const* Xb);
+};
+template <typename T>
+int ZForward<T>::run(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft,
                       const LineFFTHost& f, const void* const* Xb) {
   // members: grid.z; X holds np planes per member (all nz with nofft)
   const long pl = long(p->nkx) * p->g.ny;
@@ -2143,29 +2269,41 @@ static int zfft_x2s_t(spx_plan* p, int ncomp, const void* const* X, void* const*
   }
   ProfScope ps_(p, "z_x2s", double(p->wkx()) * p->g.ny * sizeof(cpx<T>) * ncomp *
                                 ((nofft ? p->g.nz : p->np) + p->g.nz));
-  if (Xb) {
+  if constexpr (sizeof(T) == 4) if (Xb) {
     // plus the staged float64 boundary values of the tile (nl * 2d, aligned)
     const size_t bnd_stage_bytes = size_t(f.nl) * 2 * p->g.oz * sizeof(Cd) + 16;
-    SPX_LAUNCH_Z(f, k_z_x2s, T, SPX_COMMA true, grid, blk(f),
+    SPX_LAUNCH(with_z<sizeof(cpx<T>)>, f, k_z_x2s, T, SPX_COMMA true, grid, blk(f),
                   f.lds_bytes(sizeof(cpx<T>)) + bnd_stage_bytes, p->stream, a,
                   f.dev<cpx<T>>(), p->nkx, p->g.ny, p->np, nofft, p->d_dir, p->g.Cz, p->g.oz,
                   xstride);
     SPX_CHECK_LAUNCH();
     return SPX_OK;
   }
-  SPX_LAUNCH_Z(f, k_z_x2s, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
+  SPX_LAUNCH(with_z<sizeof(cpx<T>)>, f, k_z_x2s, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
                 p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, p->np, nofft, p->d_dir,
                 p->g.Cz, p->g.oz, xstride);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 4
+template struct ZForward<double>;
+#else
+extern template struct ZForward<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 5
+template struct ZForward<float>;
+#else
+extern template struct ZForward<float>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 1
 int zfft_x2s(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft, bool lo,
              const void* const* Xb) {
   if (int rc = check_lo(p, lo)) return rc;
   if (ncomp < 1 || ncomp > kMaxComp) return fail(SPX_ERR_ARG, "zfft_x2s: bad field count");
   if (Xb && (nofft || p->g.Cz <= 0)) return fail(SPX_ERR_ARG, "boundary planes need a continuation");
-  return lo ? zfft_x2s_t<float>(p, ncomp, X, S, nofft, fzt(p, true), Xb)
-            : zfft_x2s_t<double>(p, ncomp, X, S, nofft, fzt(p, false), Xb);
+  if (!lo && Xb) return fail(SPX_ERR_ARG, "boundary planes: float32 transforms only");
+  return lo ? ZForward<float>::run(p, ncomp, X, S, nofft, fzt(p, true), Xb)
+            : ZForward<double>::run(p, ncomp, X, S, nofft, fzt(p, false), Xb);
 }
 
 int zfft_s2x_bnd(spx_plan* p, const void* const* S, int ncomp, void* XVb, void* XZb) {
@@ -2203,9 +2341,16 @@ int zfft_s2x_bnd(spx_plan* p, const void* const* S, int ncomp, void* XVb, void* 
   return SPX_OK;
 }
 
+#endif  // SPX_PART 1
+
 // S is float64 in both precisions; X (and X2) are T
 template <typename T>
-static int zfft_s2x_t(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn,
+struct ZBackward {
+  static int run(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn, int
+                 nzout, int nofft, void* const* X2, const LineFFTHost& f);
+};
+template <typename T>
+int ZBackward<T>::run(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn,
                       int nzout, int nofft, void* const* X2, const LineFFTHost& f) {
   // members: grid.z; X holds nzout planes per member
   const long pl = long(p->nkx) * p->g.ny;
@@ -2219,30 +2364,45 @@ static int zfft_s2x_t(spx_plan* p, int ncomp, const void* const* S, void* const*
   }
   if (X2) {
     ProfScope ps_(p, "z_s2x_dual", line * (16.0 * p->g.nz + 2.0 * sizeof(cpx<T>) * nzout));
-    SPX_LAUNCH_Z(f, k_z_s2x, T, SPX_COMMA true SPX_COMMA double, grid, blk(f),
+    SPX_LAUNCH(with_z<sizeof(cpx<T>)>, f, k_z_s2x, T, SPX_COMMA true SPX_COMMA double, grid, blk(f),
                   f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny,
                   nzout, dirn, nofft, p->d_kx, p->d_ky, p->d_kz);
   } else {
     ProfScope ps_(p, "z_s2x", line * (16.0 * p->g.nz + sizeof(cpx<T>) * nzout));
-    SPX_LAUNCH_Z(f, k_z_s2x, T, SPX_COMMA false SPX_COMMA double, grid, blk(f),
+    SPX_LAUNCH(with_z<sizeof(cpx<T>)>, f, k_z_s2x, T, SPX_COMMA false SPX_COMMA double, grid, blk(f),
                   f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny,
                   nzout, dirn, nofft, p->d_kx, p->d_ky, p->d_kz);
   }
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 6
+template struct ZBackward<double>;
+#else
+extern template struct ZBackward<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 7
+template struct ZBackward<float>;
+#else
+extern template struct ZBackward<float>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 1
 int zfft_s2x(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn, int nzout,
              int nofft, void* const* X2, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
   if (ncomp < 1 || ncomp > kMaxComp) return fail(SPX_ERR_ARG, "zfft_s2x: bad field count");
-  return lo ? zfft_s2x_t<float>(p, ncomp, S, X, dirn, nzout, nofft, X2, fzt(p, true))
-            : zfft_s2x_t<double>(p, ncomp, S, X, dirn, nzout, nofft, X2, fzt(p, false));
+  return lo ? ZBackward<float>::run(p, ncomp, S, X, dirn, nzout, nofft, X2, fzt(p, true))
+            : ZBackward<double>::run(p, ncomp, S, X, dirn, nzout, nofft, X2, fzt(p, false));
 }
 #endif  // SPX_PART 1 (z transforms)
 
-#if !defined(SPX_PART) || SPX_PART == 2
 template <typename T>
-static int yfft_t(spx_plan* p, int nf, const void* const* in, void* const* out, int forward,
+struct YPass {
+  static int run(spx_plan* p, int nf, const void* const* in, void* const* out, int forward, int
+                 nplanes, void* const* Y2, const LineFFTHost& f, bool cont);
+};
+template <typename T>
+int YPass<T>::run(spx_plan* p, int nf, const void* const* in, void* const* out, int forward,
                   int nplanes, void* const* Y2, const LineFFTHost& f, bool cont) {
   // members are consecutive blocks of nplanes planes
   const long nlines = long(p->nkx) * nplanes * p->mem;
@@ -2259,27 +2419,40 @@ static int yfft_t(spx_plan* p, int nf, const void* const* in, void* const* out, 
   if (nd > 0) {
     if (forward) return fail(SPX_ERR_ARG, "dual y transform is backward only");
     ProfScope ps_(p, "y_dual", io * (2.0 * nf + nd));
-    SPX_LAUNCH_XY(f, k_y, T, SPX_COMMA true, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
+    SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_y, T, SPX_COMMA true, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
                   p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, nlines, forward, p->d_ky,
                   p->npy, 0, 0, static_cast<const double*>(nullptr));
   } else {
     ProfScope ps_(p, "y", io * 2.0 * nf);
-    SPX_LAUNCH_XY(f, k_y, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
+    SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_y, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
                   p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, nlines, forward, p->d_ky,
                   p->npy, cont ? p->Cy : 0, p->oy, p->d_diry);
   }
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 2
+template struct YPass<double>;
+#else
+extern template struct YPass<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 9
+template struct YPass<float>;
+#else
+extern template struct YPass<float>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 1
 int yfft(spx_plan* p, int nf, const void* const* in, void* const* out, int forward, int nplanes,
          void* const* Y2, bool lo, bool cont) {
   if (int rc = check_lo(p, lo)) return rc;
   if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "yfft: bad field count");
   if (cont && (!forward || p->Cy <= 0 || Y2))
     return fail(SPX_ERR_ARG, "y continuation: forward transforms of plans with Cy > 0 only");
-  return lo ? yfft_t<float>(p, nf, in, out, forward, nplanes, Y2, p->fy32, cont)
-            : yfft_t<double>(p, nf, in, out, forward, nplanes, Y2, p->fy, cont);
+  return lo ? YPass<float>::run(p, nf, in, out, forward, nplanes, Y2, p->fy32, cont)
+            : YPass<double>::run(p, nf, in, out, forward, nplanes, Y2, p->fy, cont);
 }
+
+#endif  // SPX_PART 1
 
 template <typename T>
 static XFields<T> x_fields(int nf, const void* const* in, void* const* out) {
@@ -2292,48 +2465,88 @@ static XFields<T> x_fields(int nf, const void* const* in, void* const* out) {
 }
 
 template <typename T>
-static int xr2c_t(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
+struct XForward {
+  static int run(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes, const
+                 LineFFTHost& f);
+};
+template <typename T>
+int XForward<T>::run(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
                   const LineFFTHost& f) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
   dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
   const XFields<T> a = x_fields<T>(nf, R, X);
   ProfScope ps_(p, "xr2c", double(p->g.ny) * nplanes * p->mem * nf *
                                (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
-  SPX_LAUNCH_XY(f, k_xr2c, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+  SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_xr2c, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
                 f.dev<cpx<T>>(), p->nkx, npairs);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 10
+template struct XForward<double>;
+#else
+extern template struct XForward<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 11
+template struct XForward<float>;
+#else
+extern template struct XForward<float>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 1
 int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
   if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xr2c: bad field count");
-  return lo ? xr2c_t<float>(p, nf, R, X, nplanes, p->fx32)
-            : xr2c_t<double>(p, nf, R, X, nplanes, p->fx);
+  return lo ? XForward<float>::run(p, nf, R, X, nplanes, p->fx32)
+            : XForward<double>::run(p, nf, R, X, nplanes, p->fx);
 }
+#endif
 
 template <typename T>
-static int xc2r_t(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes,
+struct XBackward {
+  static int run(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes, int
+                 dirx, const LineFFTHost& f);
+};
+template <typename T>
+int XBackward<T>::run(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes,
                   int dirx, const LineFFTHost& f) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
   dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
   const XFields<T> a = x_fields<T>(nf, X, R);
   ProfScope ps_(p, "xc2r", double(p->g.ny) * nplanes * p->mem * nf *
                                (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
-  SPX_LAUNCH_XY(f, k_xc2r, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+  SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_xc2r, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
                 f.dev<cpx<T>>(), p->nkx, npairs, dirx, p->d_kx);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 10
+template struct XBackward<double>;
+#else
+extern template struct XBackward<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 11
+template struct XBackward<float>;
+#else
+extern template struct XBackward<float>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 1
 int xc2r(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes, int dirx,
          bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
   if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xc2r: bad field count");
-  return lo ? xc2r_t<float>(p, nf, X, R, nplanes, dirx, p->fx32)
-            : xc2r_t<double>(p, nf, X, R, nplanes, dirx, p->fx);
+  return lo ? XBackward<float>::run(p, nf, X, R, nplanes, dirx, p->fx32)
+            : XBackward<double>::run(p, nf, X, R, nplanes, dirx, p->fx);
 }
+#endif
 
 template <typename T>
-static int xgrad_prod_t(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
+struct XGradProd {
+  static int run(spx_plan* p, int nf, const void* const* YV, const void* const* YY, const void*
+                 const* XZ, const void* const* vel, void* const* out, const LineFFTHost& f, int
+                 nplanes);
+};
+template <typename T>
+int XGradProd<T>::run(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
                         const void* const* XZ, const void* const* vel, void* const* out,
                         const LineFFTHost& f, int nplanes) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
@@ -2350,13 +2563,28 @@ static int xgrad_prod_t(spx_plan* p, int nf, const void* const* YV, const void* 
   for (int c = 0; c < 3; ++c) a.vel[c] = static_cast<const T*>(vel[c]);
   ProfScope ps_(p, "xgrad_prod", rows * (4.0 * sizeof(cpx<T>) * p->nkx +
                                          3.0 * sizeof(T) * p->g.nx));
-  SPX_LAUNCH_XY(f, k_xgrad_prod, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+  SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_xgrad_prod, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
                 f.dev<cpx<T>>(), p->nkx, npairs, 1.0 / (t * t), p->d_kx);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 12
+template struct XGradProd<double>;
+#else
+extern template struct XGradProd<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 13
+template struct XGradProd<float>;
+#else
+extern template struct XGradProd<float>;
+#endif
 template <typename T>
-static int xgrad_fused_t(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
+struct XGradFused {
+  static int run(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ, void*
+                 const* RV, void* const* out, const LineFFTHost& f);
+};
+template <typename T>
+int XGradFused<T>::run(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
                          void* const* RV, void* const* out, const LineFFTHost& f) {
   const int nplanes = p->np;
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
@@ -2372,39 +2600,54 @@ static int xgrad_fused_t(spx_plan* p, int nf, void* const* YV, void* const* YY, 
   }
   ProfScope ps_(p, "xgrad_fused", rows * (4.0 * nf * sizeof(cpx<T>) * p->nkx +
                                           (RV ? 3.0 : 0.0) * sizeof(T) * p->g.nx));
-  if (f.wave == 3)
-    hipLaunchKernelGGL((k_xgrad_fused<T, RS_WAVE + 3>), dim3(unsigned((npairs + f.nl - 1) / f.nl)),
-                       blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(),
-                       p->nkx, npairs, nf, 1.0 / (t * t), p->d_kx);
-  else
-    hipLaunchKernelGGL((k_xgrad_fused<T, RS_POW2>), dim3(unsigned((npairs + f.nl - 1) / f.nl)),
-                       blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a, f.dev<cpx<T>>(),
-                       p->nkx, npairs, nf, 1.0 / (t * t), p->d_kx);
+  const int rc = with_xy<sizeof(cpx<T>)>(f, [&](auto rs) -> int {
+    constexpr int RS = decltype(rs)::value;
+    if constexpr (xfused_ok<T, RS>()) {
+      const size_t lds = f.lds_bytes(sizeof(cpx<T>));
+      if (int lrc = lds_limit(k_xgrad_fused<T, RS>, lds)) return lrc;
+      hipLaunchKernelGGL((k_xgrad_fused<T, RS>), dim3(unsigned((npairs + f.nl - 1) / f.nl)),
+                         blk(f), lds, p->stream, a, f.dev<cpx<T>>(), p->nkx, npairs, nf,
+                         1.0 / (t * t), p->d_kx);
+      return SPX_OK;
+    } else {
+      return SPX_ERR_UNSUPPORTED;
+    }
+  });
+  if (rc) return rc;
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
+#if !defined(SPX_PART) || SPX_PART == 14
+template struct XGradFused<double>;
+#else
+extern template struct XGradFused<double>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 15
+template struct XGradFused<float>;
+#else
+extern template struct XGradFused<float>;
+#endif
+#if !defined(SPX_PART) || SPX_PART == 1
 int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
                 void* const* RV, void* const* out, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
   if (nf < 3 || nf > 4) return fail(SPX_ERR_ARG, "xgrad_fused: 3 or 4 fields");
-  // power-of-two x lines only: the other radix families spill the velocity
-  // registers
-  const int rs = rset_of(lo ? p->fx32 : p->fx);
-  if (rs != RS_POW2 && rs != RS_WAVE + 3) return SPX_ERR_UNSUPPORTED;
-  return lo ? xgrad_fused_t<float>(p, nf, YV, YY, XZ, RV, out, p->fx32)
-            : xgrad_fused_t<double>(p, nf, YV, YY, XZ, RV, out, p->fx);
+  return lo ? XGradFused<float>::run(p, nf, YV, YY, XZ, RV, out, p->fx32)
+            : XGradFused<double>::run(p, nf, YV, YY, XZ, RV, out, p->fx);
 }
+#endif
 
+#if !defined(SPX_PART) || SPX_PART == 1
 int xgrad_prod(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
                const void* const* XZ, const void* const* vel, void* const* out, bool lo,
                int nplanes) {
   if (int rc = check_lo(p, lo)) return rc;
   if (nf < 1 || nf > 4) return fail(SPX_ERR_ARG, "xgrad_prod: 1..4 fields");
   if (nplanes < 0) nplanes = p->np;
-  return lo ? xgrad_prod_t<float>(p, nf, YV, YY, XZ, vel, out, p->fx32, nplanes)
-            : xgrad_prod_t<double>(p, nf, YV, YY, XZ, vel, out, p->fx, nplanes);
+  return lo ? XGradProd<float>::run(p, nf, YV, YY, XZ, vel, out, p->fx32, nplanes)
+            : XGradProd<double>::run(p, nf, YV, YY, XZ, vel, out, p->fx, nplanes);
 }
-#endif  // SPX_PART 2 (y and x transforms)
+#endif
 
 #if !defined(SPX_PART) || SPX_PART == 3
 // ---- float64 boundary / projection / diagnostics kernels ----
@@ -2420,7 +2663,7 @@ static int noslip_launch(spx_plan* p, void* vx, void* vy, const void* pr, const 
   const double extra = rk ? (rk->nl32 ? 8.0 : 16.0) + 32.0 : 0.0;  // nl, c0, f reads
   ProfScope ps_(p, rk ? "noslip_rk" : name,
                 ncomp * double(p->wnc()) * (2.0 * 16.0 + extra));
-  SPX_LAUNCH_RS(f, k_noslip, double, , grid, blk(f), f.lds_bytes(16), p->stream, C_<double>(vx),
+  SPX_LAUNCH(with_general, f, k_noslip, double, , grid, blk(f), f.lds_bytes(16), p->stream, C_<double>(vx),
                 C_<double>(vy), C_<double>(pr), f.dev<Cd>(), nlines, p->g.ny, p->np,
                 1.0 / double(p->g.nz), wp, p->d_kx, p->d_ky, p->d_dir, p->g.Cz, p->g.oz, r,
                 rk ? 1 : 0);
@@ -2441,18 +2684,6 @@ int noslip_fused(spx_plan* p, void* vx, void* vy, const void* pr, double tau,
   return noslip_launch(p, vx, vy, pr, wp, 2, "noslip", rk);
 }
 
-int bwall_fused(spx_plan* p, void* a0, void* a1, void* a2, int ncomp, const BWallParams& bp) {
-  if (p->g.oz > 16) return fail(SPX_ERR_UNSUPPORTED, "magnetic walls: matching order above 16");
-  const LineFFTHost& f = p->fz;
-  const long nlines = p->wlines();
-  dim3 grid(unsigned((nlines + f.nl - 1) / f.nl), unsigned(ncomp));
-  ProfScope ps_(p, "bwall", ncomp * double(p->wnc()) * 2.0 * 16.0);
-  SPX_LAUNCH_RS(f, k_bwall, double, , grid, blk(f), f.lds_bytes(16), p->stream, C_<double>(a0),
-                C_<double>(a1), C_<double>(a2), f.dev<Cd>(), nlines, p->np,
-                1.0 / double(p->g.nz), bp, p->d_khom, p->d_dir, p->g.Cz, p->g.oz);
-  SPX_CHECK_LAUNCH();
-  return SPX_OK;
-}
 
 int sconst_fused(spx_plan* p, void* th) {
   WallParams wp;
@@ -2461,18 +2692,6 @@ int sconst_fused(spx_plan* p, void* th) {
   return noslip_launch(p, th, th, nullptr, wp, 1, "sconst", nullptr);
 }
 
-int proj_pressure(spx_plan* p, void* d, int k0, int k1) {
-  const LineFFTHost& f = fzt(p, false);
-  const long nlines = p->wlines();
-  ProfScope ps_(p, "proj_pressure", 2.0 * double(p->wnc()) * 16.0);
-  const dim3 grid(unsigned((nlines + f.nl - 1) / f.nl));
-  const size_t lds = f.lds_bytes(16);
-  SPX_LAUNCH_Z(f, k_proj_pressure, double, , grid, blk(f), lds, p->stream, C_<double>(d),
-               C_<double>(p->bc), f.dev<Cd>(), nlines, p->g.ny, 1.0 / double(p->g.nz), p->g.Lz,
-               p->d_khom, p->d_z, k0, k1);
-  SPX_CHECK_LAUNCH();
-  return SPX_OK;
-}
 
 int pressure_walls(spx_plan* p, void* d) {
   const long nlines = p->wlines();
@@ -2611,7 +2830,7 @@ int build_harmonic_table(spx_plan* p) {
     // continuation + forward z FFT of the 2U profile rows
     const LineFFTHost& f = p->fz;
     const long rows = 2L * U;
-    SPX_LAUNCH_RS(f, k_z_inplace, double, , dim3(unsigned((rows + f.nl - 1) / f.nl)), blk(f),
+    SPX_LAUNCH(with_general, f, k_z_inplace, double, , dim3(unsigned((rows + f.nl - 1) / f.nl)), blk(f),
                   f.lds_bytes(16), p->stream, static_cast<Cd*>(tab), rows, f.dev<Cd>(), np, 1,
                   1, 1.0, p->d_dir, p->g.Cz, p->g.oz);
     SPX_CHECK_LAUNCH();
@@ -2685,7 +2904,7 @@ int proj_harmonic(spx_plan* p, void* a, void* b, void* c, int k0, int k1) {
   const LineFFTHost& f = p->fz2;
   const size_t lds = f.lds_bytes(16, 2);
   ProfScope ps_(p, "proj_harmonic", 6.0 * double(p->wnc()) * 16.0);
-  SPX_LAUNCH_RS(f, k_proj_harmonic, double, , dim3(unsigned((nlines + f.nl - 1) / f.nl)), blk(f),
+  SPX_LAUNCH(with_general, f, k_proj_harmonic, double, , dim3(unsigned((nlines + f.nl - 1) / f.nl)), blk(f),
                 lds, p->stream, C_<double>(a), C_<double>(b), C_<double>(c), C_<double>(p->bc),
                 f.dev<Cd>(), nlines, p->g.ny, p->np, p->g.Lz, p->d_khom, p->d_z, p->d_kx,
                 p->d_ky, p->d_dir, p->g.Cz, p->g.oz, k0, k1);
@@ -2693,8 +2912,40 @@ int proj_harmonic(spx_plan* p, void* a, void* b, void* c, int k0, int k1) {
   return SPX_OK;
 }
 
+#endif  // SPX_PART 3 (boundary, projection)
+
+#if !defined(SPX_PART) || SPX_PART == 16
+int bwall_fused(spx_plan* p, void* a0, void* a1, void* a2, int ncomp, const BWallParams& bp) {
+  if (p->g.oz > 16) return fail(SPX_ERR_UNSUPPORTED, "magnetic walls: matching order above 16");
+  const LineFFTHost& f = fzt(p, false);
+  const long nlines = p->wlines();
+  dim3 grid(unsigned((nlines + f.nl - 1) / f.nl), unsigned(ncomp));
+  ProfScope ps_(p, "bwall", ncomp * double(p->wnc()) * 2.0 * 16.0);
+  SPX_LAUNCH(with_z<16>, f, k_bwall, double, , grid, blk(f), f.lds_bytes(16), p->stream, C_<double>(a0),
+                C_<double>(a1), C_<double>(a2), f.dev<Cd>(), nlines, p->np,
+                1.0 / double(p->g.nz), bp, p->d_khom, p->d_dir, p->g.Cz, p->g.oz);
+  SPX_CHECK_LAUNCH();
+  return SPX_OK;
+}
+
+int proj_pressure(spx_plan* p, void* d, int k0, int k1) {
+  const LineFFTHost& f = fzt(p, false);
+  const long nlines = p->wlines();
+  ProfScope ps_(p, "proj_pressure", 2.0 * double(p->wnc()) * 16.0);
+  const dim3 grid(unsigned((nlines + f.nl - 1) / f.nl));
+  const size_t lds = f.lds_bytes(16);
+  SPX_LAUNCH(with_z<16>, f, k_proj_pressure, double, , grid, blk(f), lds, p->stream, C_<double>(d),
+               C_<double>(p->bc), f.dev<Cd>(), nlines, p->g.ny, 1.0 / double(p->g.nz), p->g.Lz,
+               p->d_khom, p->d_z, k0, k1);
+  SPX_CHECK_LAUNCH();
+  return SPX_OK;
+}
+#endif  // SPX_PART 16 (magnetic walls, pressure)
+
+#if !defined(SPX_PART) || SPX_PART == 8
 static int zline_launch(spx_plan* p, const LinComb& lc, const void* b, int mode, double* out) {
-  const LineFFTHost& f = mode == 1 ? p->fz2 : p->fz;
+  const LineFFTHost& fw = fzt(p, false);
+  const LineFFTHost f = mode == 1 ? fw.with_lines(fw.nl / 2) : fw;
   const long nlines = p->wlines();
   LinCombDev<double> d;
   for (int t = 0; t < 3; ++t) {
@@ -2704,7 +2955,7 @@ static int zline_launch(spx_plan* p, const LinComb& lc, const void* b, int mode,
   }
   const size_t lds = f.lds_bytes(16, mode == 1 ? 2 : 1) + size_t(f.nl) * f.tpl * sizeof(double);
   ProfScope ps_(p, "zline_reduce", double(p->wnc()) * 16.0 * (mode == 1 ? 2 : 1));
-  SPX_LAUNCH_RS(f, k_zline_reduce, double, , dim3(unsigned((nlines + f.nl - 1) / f.nl)), blk(f),
+  SPX_LAUNCH(with_z<16>, f, k_zline_reduce, double, , dim3(unsigned((nlines + f.nl - 1) / f.nl)), blk(f),
                 lds, p->stream, d, C_<double>(b), mode, out, f.dev<Cd>(), nlines, p->g.ny, p->np,
                 p->d_kx, p->d_ky, p->d_kz);
   SPX_CHECK_LAUNCH();
@@ -2742,6 +2993,6 @@ int zline_walls(spx_plan* p, const void* a, double* line_out) {
   lc.sgn[1] = lc.sgn[2] = 0;
   return zline_launch(p, lc, nullptr, 2, line_out);
 }
-#endif  // SPX_PART 3 (boundary, projection, diagnostics)
+#endif  // SPX_PART 8 (diagnostics)
 
 }  // namespace spx
