@@ -107,6 +107,7 @@ struct WallMfmaHost {
   int nbk = 0;   // 16-row blocks of the 2 nz real line values
   int kbw = 0;   // blocks per wave
   int nw = 0;    // waves per workgroup
+  int ns = 0;    // LDS slots of the waves' partial sums
   int mt = 0;    // 16-row tiles of the partial inverse DFT (2 (2d + C) rows)
   int kt = 0;    // 4-column steps of the correction (2 (2 + C) columns)
   int wpe = 0;   // waves per SIMD the kernel's register budget is sized for

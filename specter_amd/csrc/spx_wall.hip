@@ -63,7 +63,7 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c) {
 
 // GEMM A rows [M0, M1) (16-row tiles) of the wave's kappa blocks, then the
 // waves' partial sums into the ns LDS slots in a fixed order: waves < ns
-// store, waves >= ns add onto slot wave - ns (one barrier between).
+// store, then ns waves at a time add onto slot wave mod ns (a barrier between).
 // Point z of partial-IDFT index qi (0..d-1, np-d..np-1, np..n-1) and of
 // correction index p (0, np-1, np..n-1).
 __device__ __forceinline__ int qpoint(int qi, int d, int np, int nq) {
@@ -87,7 +87,7 @@ __device__ __forceinline__ int modn(unsigned x, int n, unsigned magic) {
 template <int MT, int M0, int M1, int KBW, int TAB>
 __device__ __forceinline__ void gemm_a_rows(const double* __restrict__ winv, const Cd* rl,
                                             const v4d (&vr)[KBW], int b0, int nbk, int lane,
-                                            int wave, int ns, double* red, int n, int np,
+                                            int wave, int nw, int ns, double* red, int n, int np,
                                             int d, int nq) {
   v4d acc[M1 - M0];
 #pragma unroll
@@ -146,15 +146,18 @@ __device__ __forceinline__ void gemm_a_rows(const double* __restrict__ winv, con
       for (int r = 0; r < 4; ++r) red[((wave * MT + m) * 4 + r) * 64 + lane] = acc[m - M0][r];
   }
   __syncthreads();
-  if (wave >= ns) {
-    double* slot = red + (wave - ns) * MT * 256;
+  for (int w0 = ns; w0 < nw; w0 += ns) {
+    if (w0 > ns) __syncthreads();
+    if (wave >= w0 && wave < w0 + ns) {
+      double* slot = red + (wave - w0) * MT * 256;
 #pragma unroll
-    for (int m = M0; m < M1; ++m)
+      for (int m = M0; m < M1; ++m)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int e = (m * 4 + r) * 64 + lane;
-        slot[e] = slot[e] + acc[m - M0][r];
-      }
+        for (int r = 0; r < 4; ++r) {
+          const int e = (m * 4 + r) * 64 + lane;
+          slot[e] = slot[e] + acc[m - M0][r];
+        }
+    }
   }
 }
 
@@ -216,12 +219,12 @@ __device__ __forceinline__ void wall_load_rk(v4d (&vr)[KBW], const Cd* __restric
 template <int MT, int M0, int G, int KBW, int TAB>
 __device__ __forceinline__ void gemm_a_groups(const double* __restrict__ winv, const Cd* rl,
                                               const v4d (&vr)[KBW], int b0, int nbk, int lane,
-                                              int wave, int ns, double* red, int n, int np,
+                                              int wave, int nw, int ns, double* red, int n, int np,
                                               int d, int nq) {
   constexpr int M1 = M0 + G < MT ? M0 + G : MT;
-  gemm_a_rows<MT, M0, M1, KBW, TAB>(winv, rl, vr, b0, nbk, lane, wave, ns, red, n, np, d, nq);
+  gemm_a_rows<MT, M0, M1, KBW, TAB>(winv, rl, vr, b0, nbk, lane, wave, nw, ns, red, n, np, d, nq);
   if constexpr (M1 < MT)
-    gemm_a_groups<MT, M1, G, KBW, TAB>(winv, rl, vr, b0, nbk, lane, wave, ns, red, n, np, d, nq);
+    gemm_a_groups<MT, M1, G, KBW, TAB>(winv, rl, vr, b0, nbk, lane, wave, nw, ns, red, n, np, d, nq);
 }
 
 // MT: 16-row tiles of the 2(2d+C) real partial-IDFT outputs; KT: 4-column
@@ -233,11 +236,10 @@ __global__ void __launch_bounds__(512, WPE) k_wall_mfma(
     int ny, int n, int np, int nbk, double invn, WallParams wp, const double* __restrict__ kx,
     const double* __restrict__ ky, const double* __restrict__ dir, int C, int d,
     const double* __restrict__ winv, const double* __restrict__ wfwd,
-    const Cd* __restrict__ roots, unsigned magic, RkLoad rk, int rk_on) {
+    const Cd* __restrict__ roots, unsigned magic, int ns, RkLoad rk, int rk_on) {
 #pragma clang fp contract(off)
   extern __shared__ double sm[];
   const int nw = blockDim.x >> 6;
-  const int ns = nw < 4 ? nw : 4;               // partial-sum slots
   Cd* const rl = reinterpret_cast<Cd*>(sm);     // [n] roots of unity (TAB 1)
   double* const red = sm + (TAB ? 2 * n : 0);   // [ns][MT][4][64] partial X
   double* const xs = red;                       // slot 0 ends up holding X
@@ -289,19 +291,18 @@ __global__ void __launch_bounds__(512, WPE) k_wall_mfma(
     w[3] = wt.y;
   }
 
-  // ---- GEMM A: partial inverse DFT at the 2d + C points, one row tile at a
-  // time, summed over the waves in a fixed order; then slot 0 += slots
-  // 1..ns-1
+  // ---- GEMM A: partial inverse DFT at the 2d + C points, summed over the
+  // waves in a fixed order; then slot 0 += slots 1..ns-1
   const int nq = 2 * d + C;
   if constexpr (TAB == 1) {
     for (int e = threadIdx.x; e < n; e += blockDim.x) rl[e] = roots[e];
     __syncthreads();
   }
-  // one 16-row tile at a time: 8 accumulator registers beside the wave's
-  // line blocks (three at a time spilled 26 registers per lane at 4 waves per
+  // every row tile in one sweep while the wave's line blocks leave registers for
+  // their accumulators, else one 16-row tile at a time (three at a time spilled 26 registers per lane at 4 waves per
   // SIMD; HD 512^3: 3.43 -> 3.19 ms per launch with the batched loads)
-  constexpr int G = 1;
-  gemm_a_groups<MT, 0, G, KBW, TAB>(winv, rl, vr, b0, nbk, lane, wave, ns, red, n, np, d, nq);
+  constexpr int G = KBW <= 5 ? MT : 1;
+  gemm_a_groups<MT, 0, G, KBW, TAB>(winv, rl, vr, b0, nbk, lane, wave, nw, ns, red, n, np, d, nq);
   __syncthreads();
   for (int e = threadIdx.x; e < MT * 256; e += blockDim.x) {
     double s = red[e];
@@ -413,6 +414,39 @@ __global__ void __launch_bounds__(512, WPE) k_wall_mfma(
 
 constexpr int kMaxWaves = 8;
 
+// Calls launch with the kernel of the plan's launch shape.
+template <int MT, int KT, typename F>
+void wall_kernel(const WallMfmaHost& w, F&& launch) {
+  auto both = [&](auto roots, auto table) { w.tab ? launch(roots) : launch(table); };
+  switch (w.kbw) {
+    case 1: return launch(k_wall_mfma<MT, KT, 1, 4, 1>);
+    case 2: return launch(k_wall_mfma<MT, KT, 2, 4, 1>);
+    case 3: return launch(k_wall_mfma<MT, KT, 3, 4, 1>);
+    case 4: return launch(k_wall_mfma<MT, KT, 4, 4, 1>);
+    case 5: return launch(k_wall_mfma<MT, KT, 5, 4, 1>);
+    case 6: return launch(k_wall_mfma<MT, KT, 6, 4, 1>);
+    case 7: return launch(k_wall_mfma<MT, KT, 7, 4, 1>);
+    case 8: return launch(k_wall_mfma<MT, KT, 8, 4, 1>);
+    case 9:
+      if (w.wpe == 3) return both(k_wall_mfma<MT, KT, 9, 3, 1>, k_wall_mfma<MT, KT, 9, 3, 0>);
+      return both(k_wall_mfma<MT, KT, 9, 4, 1>, k_wall_mfma<MT, KT, 9, 4, 0>);
+    default: return both(k_wall_mfma<MT, KT, 18, 2, 1>, k_wall_mfma<MT, KT, 18, 2, 0>);
+  }
+}
+
+// kappa blocks per wave of float64 plans: one wave per SIMD (4 waves, up to 36
+// blocks) or two (8), with equal shares -- whole lines of few blocks are bound
+// by one wave's chain of loads and MFMAs, and a workgroup by its longest wave.
+// us per launch against 9 blocks per wave (the others idle at the end): HD 32^3
+// (8 blocks) 1 x 8 waves 15.5, 2 x 4 19.6, 9 41; 16 x 64^3 (12) 219, 313; 96x120x77
+// (13) 45, 70; 128^3 d = 8 (20) 106, 142; z = 235 (30) 135, 152; z = 325 (41) 191,
+// 228.  Shares that leave 5 to 7 waves (two SIMDs of a CU with one more) are
+// slower than either neighbour: 128^3 with 4 blocks 137, 3 blocks 119.
+int wall_blocks_per_wave(int nbk) {
+  if (nbk <= kMaxWaves) return 1;
+  return nbk <= 36 ? (nbk + 3) / 4 : (nbk + 7) / 8;
+}
+
 }  // namespace
 
 // Tables of the plan's wall correction (float64 plans' and mixed plans' state
@@ -428,19 +462,22 @@ int build_wall_mfma(spx_plan* p) {
   const int mt = (2 * nq + 15) / 16, kt = (2 * nrho + 3) / 4;
   const int nbk = (2 * n + 15) / 16;
   if (!((mt == 5 || mt == 6) && kt <= 16 && np >= 2 * d)) return SPX_OK;
-  // waves per workgroup and kappa blocks per wave: the fewest registers that
-  // keep the workgroup within 8 waves
-  int kbw = 9;
-  if ((nbk + kbw - 1) / kbw > kMaxWaves) kbw = 18;
-  if ((nbk + kbw - 1) / kbw > kMaxWaves) return SPX_OK;
+  // kappa blocks per wave (at most 8 waves per workgroup).  Mixed plans keep 9:
+  // the partial sums of other shares differ in the last bit, which redraws the
+  // rounding of the float32 nonlinear term (see build_wave_fft)
+  int kbw = p->fp32 ? 9 : wall_blocks_per_wave(nbk);
+  auto fits = [&](int v) { return v >= 1 && (v <= 9 || v == 18) && (nbk + v - 1) / v <= kMaxWaves; };
+  if (!fits(kbw)) kbw = 18;
+  if (!fits(kbw)) return SPX_OK;
   WallTune tune;
   const bool tuned = get_wall_tune(n, &tune);
-  if (tuned && (tune.kbw == 9 || tune.kbw == 18) && (nbk + tune.kbw - 1) / tune.kbw <= kMaxWaves)
-    kbw = tune.kbw;
-  if (const char* e = std::getenv("SPX_WALL_KBW")) {
-    const int v = std::atoi(e);
-    if ((v == 9 || v == 18) && (nbk + v - 1) / v <= kMaxWaves) kbw = v;
-  }
+  if (tuned && (tune.kbw == 9 || tune.kbw == 18) && fits(tune.kbw)) kbw = tune.kbw;
+  if (const char* e = std::getenv("SPX_WALL_KBW"))
+    if (fits(std::atoi(e))) kbw = std::atoi(e);
+  w.tab = 1;
+  if (const char* e = std::getenv("SPX_WALL_TAB")) w.tab = std::atoi(e) == 0 ? 0 : 1;
+  // (the fragment tables are read by the kernels of 9 and 18 blocks)
+  if (w.tab == 0 && kbw < 9) kbw = 9;
   // register budget: 3 or 4 waves per SIMD for 9 blocks per wave (4: two
   // 8-wave workgroups per CU overlap their load and matrix phases; HD 512^3:
   // 3.64 ms per launch against 5.31 ms with 3), 2 for 18
@@ -450,10 +487,17 @@ int build_wall_mfma(spx_plan* p) {
     const int v = std::atoi(e);
     if (v == 3 || v == 4) wpe = v;
   }
-  w.wpe = kbw == 18 ? 2 : wpe;
+  w.wpe = kbw == 18 ? 2 : (kbw < 9 ? 4 : wpe);
   w.nbk = nbk;
   w.kbw = kbw;
   w.nw = (nbk + kbw - 1) / kbw;
+  // Slots of the waves' partial sums: the LDS of four slots (10 or 12 KB each)
+  // leaves room for two or three workgroups on a CU.  Up to four waves add onto
+  // two slots in float64 (16 x 64^3 277 -> 219 us per launch, HD 256^3 491 -> 422)
+  // and onto one in mixed plans, whose order of sums is that of four (192^3 264
+  // -> 235 us, 96x144x150 109 -> 97); more waves gain nothing (their registers
+  // bound the workgroups per CU).
+  w.ns = w.nw > 4 ? 4 : (p->fp32 ? 1 : std::min(w.nw, 2));
   w.mt = mt;
   w.kt = kt;
   // points of the partial inverse DFT and of the correction
@@ -506,8 +550,6 @@ int build_wall_mfma(spx_plan* p) {
     rt[2 * m + 1] = ci[m];
   }
   w.magic = unsigned((uint64_t(1) << 32) / uint64_t(n) + 1);
-  w.tab = 1;
-  if (const char* e = std::getenv("SPX_WALL_TAB")) w.tab = std::atoi(e) == 0 ? 0 : 1;
   double** dst[3] = {&w.winv, &w.wfwd, &w.roots};
   const std::vector<double>* src[3] = {&ta, &tc, &rt};
   for (int i = 0; i < 3; ++i) {
@@ -523,23 +565,13 @@ int build_wall_mfma(spx_plan* p) {
   return SPX_OK;
 }
 
-#define SPX_WALL_LAUNCH(MT, KT, KBW, WPE)                                                     \
-  if (w.tab) SPX_WALL_LAUNCH_T(MT, KT, KBW, WPE, 1) else SPX_WALL_LAUNCH_T(MT, KT, KBW, WPE, 0)
-#define SPX_WALL_LAUNCH_T(MT, KT, KBW, WPE, TAB)                                              \
-  hipLaunchKernelGGL((k_wall_mfma<MT, KT, KBW, WPE, TAB>), grid, dim3(64 * w.nw), lds, p->stream, \
-                     static_cast<double*>(vx), static_cast<double*>(vy),                      \
-                     static_cast<const Cd*>(pr), nlines, p->g.ny, p->g.nz, p->np, w.nbk,      \
-                     1.0 / double(p->g.nz), wp, p->d_kx, p->d_ky, p->d_dir, p->g.Cz, p->g.oz, \
-                     w.winv, w.wfwd, reinterpret_cast<const Cd*>(w.roots), w.magic, r,     \
-                     rk ? 1 : 0);
-
 int wall_mfma(spx_plan* p, void* vx, void* vy, const void* pr, const WallParams& wp, int ncomp,
               const RkLoad* rk) {
   const WallMfmaHost& w = p->wall;
   if (!w.on) return SPX_ERR_UNSUPPORTED;
   const long nlines = p->wlines();
   const dim3 grid(unsigned((nlines + 15) / 16), unsigned(ncomp));
-  const size_t lds = (size_t(std::min(w.nw, 4)) * w.mt * 256 + size_t(w.kt) * 64 + 64 +
+  const size_t lds = (size_t(w.ns) * w.mt * 256 + size_t(w.kt) * 64 + 64 +
                       (w.tab ? 2 * size_t(p->g.nz) : 0)) *
                      sizeof(double);
   RkLoad r;
@@ -550,16 +582,16 @@ int wall_mfma(spx_plan* p, void* vx, void* vy, const void* pr, const WallParams&
                 ncomp * double(p->wnc()) * (2.0 * 16.0 + extra));
   // the partial-IDFT tile count follows (d, C): 5 for d = 5, C = 25 (70 rows),
   // 6 for d = 8, C = 27 (86 rows); the correction steps 14 / 15
-  const int key = w.mt * 10000 + w.kt * 100 + w.kbw * 10 / 9 + w.wpe;  // kbw 9 -> 10, 18 -> 20
-  switch (key) {
-    case 51413: SPX_WALL_LAUNCH(5, 14, 9, 3); break;
-    case 51414: SPX_WALL_LAUNCH(5, 14, 9, 4); break;
-    case 51422: SPX_WALL_LAUNCH(5, 14, 18, 2); break;
-    case 61513: SPX_WALL_LAUNCH(6, 15, 9, 3); break;
-    case 61514: SPX_WALL_LAUNCH(6, 15, 9, 4); break;
-    case 61522: SPX_WALL_LAUNCH(6, 15, 18, 2); break;
-    default: return SPX_ERR_UNSUPPORTED;
-  }
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * w.nw), lds, p->stream, static_cast<double*>(vx),
+                       static_cast<double*>(vy), static_cast<const Cd*>(pr), nlines, p->g.ny,
+                       p->g.nz, p->np, w.nbk, 1.0 / double(p->g.nz), wp, p->d_kx, p->d_ky, p->d_dir,
+                       p->g.Cz, p->g.oz, w.winv, w.wfwd, reinterpret_cast<const Cd*>(w.roots),
+                       w.magic, w.ns, r, rk ? 1 : 0);
+  };
+  if (w.mt == 5 && w.kt == 14) wall_kernel<5, 14>(w, launch);
+  else if (w.mt == 6 && w.kt == 15) wall_kernel<6, 15>(w, launch);
+  else return SPX_ERR_UNSUPPORTED;
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
