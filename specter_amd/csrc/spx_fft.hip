@@ -944,7 +944,10 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cp
 // ((u Dx v_c + v Dy v_c) + w Dz v_c) tmp from the c2r of i kx YV_c, YY_c and
 // XZ_c, in k_xgrad_prod's operation order, and its r2c.  Neither the real
 // velocity nor the products go to memory.  A line is owned by its tpl threads, so
-// the transforms of a row pair synchronise with line_sync.
+// the transforms of a row pair synchronise with line_sync.  Launches of fewer
+// than kSpread tiles give each field a workgroup of its own (blockIdx.y), which
+// forms the velocity again: 7 transforms one after the other instead of 15 (HD
+// 32^3 38 -> 20 us, 64^3 45 -> 26 us); rv is then stored by the first.
 template <typename T>
 struct XGradArgs {
   const cpx<T>* yv[4];
@@ -986,7 +989,7 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
         const Cp z = xl[x];
         vel[c][0][q] = z.x;
         vel[c][1][q] = -z.y;
-        if (a.rv[c] && ok) {
+        if (a.rv[c] && ok && blockIdx.y == 0) {
           a.rv[c][ro + x] = z.x;
           a.rv[c][ro + x + nx] = -z.y;
         }
@@ -995,7 +998,7 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
     line_sync(f.tpl);
   }
 #pragma unroll 1
-  for (int c = 0; c < nf; ++c) {
+  for (int c = blockIdx.y; c < nf; c += gridDim.y) {
     T accA[KX], accB[KX];
     const Cp* srcs[3] = {a.yv[c], a.yy[c], a.xz[c]};
 #pragma unroll
@@ -2186,6 +2189,18 @@ template <int CS, typename F>
 static int with_xy(const LineFFTHost& f, F&& fn) {
   return f.wave >= 0 ? with_wave<CS, true>(f.wave, fn) : with_general(f, fn);
 }
+// f with fewer lines per workgroup where a launch of that many lines and
+// fields would leave CUs idle: down to one wave, and to rows of 64 bytes where a
+// workgroup's lines are neighbours in memory (least: lines of such a row).
+// Two workgroups per CU: one step's kernels at limits of 0 / 256 / 512 / 1024 take
+// 241 / 192 / 192 / 192 us for HD 32^3, 324 / 310 / 285 / 284 for 64^3, 572 / 565 / 559
+// / 554 for 96x120x77, 95 / 90 / 84 / 86 for the 160x120x103 transforms.
+constexpr long kSpread = 512;
+static inline LineFFTHost spread(const LineFFTHost& f, long lines, long fields, int least) {
+  int nl = f.nl;
+  while (nl > least && nl * f.tpl > 64 && (lines + nl - 1) / nl * fields < kSpread) nl >>= 1;
+  return f.with_lines(nl);
+}
 #define SPX_COMMA ,
 // launch the instance KER<TY, RS TARGS> of the dispatcher DISP(F, ...)
 #define SPX_LAUNCH(DISP, F, KER, TY, TARGS, GRID, BLOCK, LDS, STREAM, ...)                   \
@@ -2256,9 +2271,10 @@ struct ZForward {
 };
 template <typename T>
 int ZForward<T>::run(spx_plan* p, int ncomp, const void* const* X, void* const* S, int nofft,
-                      const LineFFTHost& f, const void* const* Xb) {
+                      const LineFFTHost& fp, const void* const* Xb) {
   // members: grid.z; X holds np planes per member (all nz with nofft)
   const long pl = long(p->nkx) * p->g.ny;
+  const LineFFTHost f = spread(fp, pl, long(ncomp) * p->mem, 64 / int(sizeof(cpx<T>)));
   dim3 grid(unsigned((pl + f.nl - 1) / f.nl), unsigned(ncomp), unsigned(p->mem));
   const long xstride = pl * (nofft ? p->g.nz : p->np);
   ZX2S<T> a;
@@ -2351,9 +2367,10 @@ struct ZBackward {
 };
 template <typename T>
 int ZBackward<T>::run(spx_plan* p, int ncomp, const void* const* S, void* const* X, int dirn,
-                      int nzout, int nofft, void* const* X2, const LineFFTHost& f) {
+                      int nzout, int nofft, void* const* X2, const LineFFTHost& fp) {
   // members: grid.z; X holds nzout planes per member
   const long pl = long(p->nkx) * p->g.ny;
+  const LineFFTHost f = spread(fp, pl, long(ncomp) * p->mem, 64 / int(sizeof(cpx<T>)));
   dim3 grid(unsigned((pl + f.nl - 1) / f.nl), unsigned(ncomp), unsigned(p->mem));
   const double line = double(p->wkx()) * p->g.ny * ncomp;
   ZS2X<T, double> a;
@@ -2403,9 +2420,10 @@ struct YPass {
 };
 template <typename T>
 int YPass<T>::run(spx_plan* p, int nf, const void* const* in, void* const* out, int forward,
-                  int nplanes, void* const* Y2, const LineFFTHost& f, bool cont) {
+                  int nplanes, void* const* Y2, const LineFFTHost& fp, bool cont) {
   // members are consecutive blocks of nplanes planes
   const long nlines = long(p->nkx) * nplanes * p->mem;
+  const LineFFTHost f = spread(fp, nlines, nf, 64 / int(sizeof(cpx<T>)));
   dim3 grid(unsigned((nlines + f.nl - 1) / f.nl), unsigned(nf));
   YFields<T> a;
   int nd = 0;
@@ -2471,8 +2489,9 @@ struct XForward {
 };
 template <typename T>
 int XForward<T>::run(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
-                  const LineFFTHost& f) {
+                  const LineFFTHost& fp) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
+  const LineFFTHost f = spread(fp, npairs, nf, 1);
   dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
   const XFields<T> a = x_fields<T>(nf, R, X);
   ProfScope ps_(p, "xr2c", double(p->g.ny) * nplanes * p->mem * nf *
@@ -2508,8 +2527,9 @@ struct XBackward {
 };
 template <typename T>
 int XBackward<T>::run(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes,
-                  int dirx, const LineFFTHost& f) {
+                  int dirx, const LineFFTHost& fp) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
+  const LineFFTHost f = spread(fp, npairs, nf, 1);
   dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
   const XFields<T> a = x_fields<T>(nf, X, R);
   ProfScope ps_(p, "xc2r", double(p->g.ny) * nplanes * p->mem * nf *
@@ -2548,8 +2568,9 @@ struct XGradProd {
 template <typename T>
 int XGradProd<T>::run(spx_plan* p, int nf, const void* const* YV, const void* const* YY,
                         const void* const* XZ, const void* const* vel, void* const* out,
-                        const LineFFTHost& f, int nplanes) {
+                        const LineFFTHost& fp, int nplanes) {
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
+  const LineFFTHost f = spread(fp, npairs, nf, 1);
   dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
   const double t = double(p->g.nx) * double(p->g.ny) * double(p->g.nz);
   const double rows = double(p->g.ny) * nplanes * p->mem * nf;
@@ -2585,9 +2606,10 @@ struct XGradFused {
 };
 template <typename T>
 int XGradFused<T>::run(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
-                         void* const* RV, void* const* out, const LineFFTHost& f) {
+                         void* const* RV, void* const* out, const LineFFTHost& fp) {
   const int nplanes = p->np;
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
+  const LineFFTHost f = spread(fp, npairs, 1, 1);
   const double t = double(p->g.nx) * double(p->g.ny) * double(p->g.nz);
   const double rows = double(p->g.ny) * nplanes * p->mem;
   XGradArgs<T> a;
@@ -2605,9 +2627,10 @@ int XGradFused<T>::run(spx_plan* p, int nf, void* const* YV, void* const* YY, vo
     if constexpr (xfused_ok<T, RS>()) {
       const size_t lds = f.lds_bytes(sizeof(cpx<T>));
       if (int lrc = lds_limit(k_xgrad_fused<T, RS>, lds)) return lrc;
-      hipLaunchKernelGGL((k_xgrad_fused<T, RS>), dim3(unsigned((npairs + f.nl - 1) / f.nl)),
-                         blk(f), lds, p->stream, a, f.dev<cpx<T>>(), p->nkx, npairs, nf,
-                         1.0 / (t * t), p->d_kx);
+      const unsigned tiles = unsigned((npairs + f.nl - 1) / f.nl);
+      hipLaunchKernelGGL((k_xgrad_fused<T, RS>), dim3(tiles, tiles < kSpread ? nf : 1), blk(f),
+                         lds, p->stream, a, f.dev<cpx<T>>(), p->nkx, npairs, nf, 1.0 / (t * t),
+                         p->d_kx);
       return SPX_OK;
     } else {
       return SPX_ERR_UNSUPPORTED;
