@@ -1993,7 +1993,7 @@ int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_blo
 struct WaveInfo {
   int n, m, lanes, mode, nmax, ldl, tab, twm, lines16, lines8, npass;
   const int* radix;
-  bool natural;
+  bool natural, xy;
   int lines(int csize) const { return csize == 16 ? lines16 : lines8; }
 };
 template <int W = 0>
@@ -2001,7 +2001,7 @@ static void wave_infos(WaveInfo* o) {
   using P = typename WavePlanN<W>::type;
   o[W] = WaveInfo{P::n,   P::m,   P::lanes,          P::mode,          P::nmax,  P::ldl,
                   P::tab, P::twm, wave_lines<W>(16), wave_lines<W>(8), P::npass, P::radix,
-                  P::natural};
+                  P::natural, P::xy};
   if constexpr (W + 1 < kWavePlans) wave_infos<W + 1>(o);
 }
 static const WaveInfo* wave_info() {
@@ -2106,7 +2106,7 @@ int attach_xy_wave(LineFFTHost& f, int csize) {
   if (f.mode != 0) return SPX_OK;
   for (int q = 0; q < kWavePlans; ++q) {
     const WaveInfo& i = wave_info()[q];
-    if (i.mode != 0 || i.m != f.n || !i.lines(csize)) continue;
+    if (!i.xy || i.m != f.n || !i.lines(csize)) continue;
     if (!i.natural) return set_wave(f, q, csize);
     if (f.n == 512 && f.tpl == 64) f.wave = q;  // the engine's launch shape
     return SPX_OK;
@@ -2167,7 +2167,7 @@ static int with_general(const LineFFTHost& f, F&& fn) {
 template <int CS, bool DIRECT, int W = 0, int END = kWavePlans, typename F>
 static int with_wave(int w, F&& fn) {
   if constexpr (W < END) {
-    if constexpr (wave_lines<W>(CS) > 0 && (!DIRECT || WavePlanN<W>::type::mode == 0)) {
+    if constexpr (wave_lines<W>(CS) > 0 && (!DIRECT || WavePlanN<W>::type::xy)) {
       if (w == W) return fn(std::integral_constant<int, RS_WAVE + W>{});
     }
     return with_wave<CS, DIRECT, W + 1, END>(w, fn);

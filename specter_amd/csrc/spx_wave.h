@@ -596,6 +596,7 @@ template <int M, int L, int MODE, int TWM, int PAD, int... Rs>
 struct WavePlan {
   static constexpr int n = 0, m = M, mode = MODE, lanes = L, twm = TWM;  // n: any
   static constexpr bool natural = false;
+  static constexpr bool xy = MODE == 0 && M % 2 == 0;  // compiled for x and y lines too
   static constexpr int nmax = MODE == 1 ? (M + 1) / 2 : (MODE == 2 ? M + 1 : M);
   static constexpr int ldl = M + (PAD ? M / RadixProduct<Rs...>::first : 0) + 1;
   static_assert(RadixProduct<Rs...>::value == M, "radices do not multiply to M");
@@ -743,7 +744,7 @@ template <int N, int M, int MODE, int TWM, int... Rs>
 struct FixedPlan {
   static constexpr int n = N, m = M, mode = MODE, lanes = 64, nmax = N, twm = TWM;
   static constexpr int ldl = M + 1, tab = M, npass = 0;
-  static constexpr bool natural = true;
+  static constexpr bool natural = true, xy = MODE == 0 && M % 2 == 0;
   static constexpr const int* radix = nullptr;
   static constexpr int lines(int csize) {
     return (size_t(M) + 8 * (size_t(M) + 1)) * csize <= 160 * 1024 ? 8 : 0;
@@ -853,9 +854,21 @@ SPX_WAVE_PLAN(35, 16, 640, 32, 1, 2, 1, 20, 8, 4)
 SPX_WAVE_PLAN(36, 16, 720, 64, 1, 2, 0, 10, 6, 12)
 SPX_WAVE_PLAN(37, 16, 900, 64, 1, 2, 0, 15, 15, 4)
 SPX_WAVE_PLAN(38, 16, 1080, 64, 1, 2, 0, 18, 6, 10)
+// odd direct lengths, z lines only: np + 25 of 80, 96, 100, 144, 150 and 200 planes,
+// np + 27 of 48 and 64, with the engine's radices (z stages of an RK stage on the
+// engine and compiled: 16 members of 64^2 x 91 float64 201 + 148 -> 147 + 85 us,
+// 96x144x175 mixed 68 + 46 -> 40 + 31 us)
+SPX_WAVE_PLAN(39, 0, 75, 16, 0, 0, 0, 3, 5, 5)
+SPX_WAVE_PLAN(40, 0, 91, 16, 0, 0, 0, 7, 13)
+SPX_WAVE_PLAN(41, 0, 105, 16, 0, 0, 0, 3, 5, 7)
+SPX_WAVE_PLAN(42, 0, 121, 16, 0, 0, 0, 11, 11)
+SPX_WAVE_PLAN(43, 0, 125, 32, 0, 0, 0, 5, 5, 5)
+SPX_WAVE_PLAN(44, 0, 169, 16, 0, 0, 0, 13, 13)
+SPX_WAVE_PLAN(45, 0, 175, 32, 0, 0, 0, 5, 5, 7)
+SPX_WAVE_PLAN(46, 0, 225, 32, 0, 0, 0, 9, 5, 5)
 #undef SPX_WAVE_PLAN
 #undef SPX_PLAN
-constexpr int kWavePlans = 39;
+constexpr int kWavePlans = 47;
 template <int RS>
 struct WavePlanOf {
   using type = typename WavePlanN<RS - RS_WAVE>::type;

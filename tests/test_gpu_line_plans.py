@@ -1,7 +1,7 @@
 """The compiled line plans at the edges of their ranges.
 
-Direct plans serve x, y and z lines of exactly their length, Rader plans z lines
-of M + 1, and a ladder of Bluestein lengths M every other z length with a prime
+Direct plans serve z lines (of even length: x and y lines too) of exactly their
+length, Rader plans z lines of M + 1, and a ladder of Bluestein lengths M every other z length with a prime
 factor above 13 up to n = (M + 1) / 2: each rung is run at the smallest and the
 largest n it serves.  Tolerances as for the other transform and gradre tests:
 1e-13 of the largest value in float64 (the transforms), 1e-12 (gradre, d = 5),
@@ -16,6 +16,7 @@ from conftest import TABLES, rel_err, rel_l2
 pytestmark = pytest.mark.gpu
 
 DIRECT = (32, 48, 64, 80, 96, 120, 128, 144, 160, 192, 240, 256, 288, 320, 384, 512, 1024)
+ODD = (75, 91, 105, 121, 125, 169, 175, 225)
 RUNGS = (120, 128, 192, 256, 315, 320, 375, 384, 441, 448, 512, 640, 700, 720, 840, 900, 1080)
 
 
@@ -106,7 +107,7 @@ def _same_as_engine(monkeypatch, shape, switch):
     monkeypatch.delenv(switch)
 
 
-@pytest.mark.parametrize("n", _edges() + [89, 281])
+@pytest.mark.parametrize("n", _edges() + [89, 281, *ODD])
 def test_z_lines(n):
     info = _transforms((6, 10, n))
     assert info.z_wave_plan >= 0
@@ -124,7 +125,7 @@ def test_direct_lines(n):
     _gradre((6, n, 41))
 
 
-@pytest.mark.parametrize("n", [n for n in DIRECT if n != 512] + [57, 59, 89, 153, 217, 281, 409])
+@pytest.mark.parametrize("n", [n for n in DIRECT if n != 512] + [*ODD, 57, 59, 89, 153, 217, 281, 409])
 def test_mixed_plans_keep_the_bits(monkeypatch, n):
     """compiled lines against the general engine (512 and 537 have passes of
     their own)"""
