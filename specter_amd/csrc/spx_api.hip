@@ -231,6 +231,31 @@ static int cross_spec(spx_plan* p, const void* const* A, const void* const* B, v
   return r2c3_n(p, 3, RO, out);
 }
 
+// W <- W x V, M <- V x B, L <- J x B through real space, each field's z and y
+// stages once: XZ holds V's planes until V x B replaces them, XV then B's
+static int mhd_products(spx_plan* p, void* const* W, void* const* V, void* const* J,
+                        void* const* B, void* const* L, void* const* M) {
+  const void* wv[6] = {W[0], W[1], W[2], V[0], V[1], V[2]};
+  const void* b[3] = {B[0], B[1], B[2]};
+  const void* j[3] = {J[0], J[1], J[2]};
+  void* x[6] = {p->XV[0], p->XV[1], p->XV[2], p->XZ[0], p->XZ[1], p->XZ[2]};
+  void* const* xz = x + 3;
+  int rc;
+  auto planes = [&](int nf, const void* const* in, void* const* xs) {
+    const int r = zfft_s2x(p, nf, in, xs, 0, p->np, 0);
+    return r ? r : yfft(p, nf, xs, xs, 0, p->np);
+  };
+  auto product = [&](void* const* xa, void* const* xb, void* const* xs, void* const* out) {
+    if (int r = xcross(p, xa, xb, xs)) return r;
+    if (int r = yfft(p, 3, xs, xs, 1, p->np, nullptr, false, p->Cy > 0)) return r;
+    return zfft_x2s(p, 3, xs, out, 0);
+  };
+  if ((rc = planes(6, wv, x)) || (rc = product(x, xz, x, W))) return rc;
+  if ((rc = planes(3, b, x)) || (rc = product(xz, x, xz, M))) return rc;
+  if ((rc = planes(3, j, xz))) return rc;
+  return product(xz, x, xz, L);
+}
+
 // sol_project with the condition on the potential (bctarget 0; wall kinds
 // k0, k1: 0 Dirichlet, 2 Robin; boundary_mod.fpp:197-402)
 static int sol_project_pot(spx_plan* p, void* a, void* b, void* c, void* d, int k0, int k1) {
@@ -1427,8 +1452,8 @@ int spx_rkstep1(spx_plan* p, spx_state* s) {
   return op_copy_fields(p, 3, asrc, s->C9);
 }
 
-// One RK stage of the MHD solver (include/mhd/mhd_rkstep2.f90:3-84).  Real
-// work fields: MR[0..2] curl v, then j; MR[3..5] v; MR[6..8] b; MR[9..11] products.
+// One RK stage of the MHD solver (include/mhd/mhd_rkstep2.f90:3-84).  Without
+// the fused x stage the real work fields are MR[0..2] curl v, then j; MR[3..5] v; MR[6..8] b; MR[9..11] products.
 static int mhd_substep(spx_plan* p, spx_state* s, int o) {
   const spx_params& q = s->prm;
   const double rmp = 1.0 / double(o);
@@ -1447,9 +1472,13 @@ static int mhd_substep(spx_plan* p, spx_state* s, int o) {
   // (curl v) x v (:28), j x b (:31), v x b (:45)
   void* W[3] = {s->N[0], s->N[1], s->N[2]};
   if ((rc = op_curl3(p, V, W))) return rc;
-  if ((rc = cross_spec(p, W, V, W, R, R + 3, R + 9, false, false))) return rc;
-  if ((rc = cross_spec(p, A, s->B, s->L, R, R + 6, R + 9, false, false))) return rc;
-  if ((rc = cross_spec(p, V, s->B, s->M, R + 3, R + 6, R + 9, true, true))) return rc;
+  if (xcross_fused(p)) {
+    if ((rc = mhd_products(p, W, V, A, s->B, s->L, s->M))) return rc;
+  } else {
+    if ((rc = cross_spec(p, W, V, W, R, R + 3, R + 9, false, false))) return rc;
+    if ((rc = cross_spec(p, A, s->B, s->L, R, R + 6, R + 9, false, false))) return rc;
+    if ((rc = cross_spec(p, V, s->B, s->M, R + 3, R + 6, R + 9, true, true))) return rc;
+  }
   // filters, laplak and the stage update (:33-76)
   const void* c1[3] = {s->C1, s->C2, s->C3};
   const void* f[3] = {s->fx, s->fy, s->fz};

@@ -354,9 +354,15 @@ int xgrad_prod(spx_plan* p, int nf, const void* const* YV, const void* const* YY
                int nplanes = -1);
 // the same on the np planes of three velocity components (and a scalar,
 // nf = 4) with vel = c2r(YV[0..2]) formed in the same launch and stored to RV
-// when given; x lengths of a power of two, SPX_ERR_UNSUPPORTED otherwise
+// when given; x lengths whose plan has it (plan flag xfused), SPX_ERR_UNSUPPORTED
+// otherwise
 int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
                 void* const* RV, void* const* out, bool lo);
+// the x stage of out = A x B on the np planes of float64 half spectra, tmp =
+// 1 / (nx ny nz)^2 as op_cross_real; out may be A or B.  xcross_fused: whether the
+// plan's x lines have it (else SPX_ERR_UNSUPPORTED) and its work arrays exist
+bool xcross_fused(const spx_plan* p);
+int xcross(spx_plan* p, void* const* A, void* const* B, void* const* out);
 // fused v_imposebc: goto_domain_w_boundaries + noslip_z + goto_3d_fourier on vx,vy
 // rk: the RK update of vx, vy (c[0], c[1]) is applied on load (null: none)
 // Launch-shape overrides set by an autotuner (spx_tune_*), consulted when a

@@ -1041,10 +1041,90 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
   }
 }
 
+using Cd = cpx<double>;
+// The x stage of a cross product A x B on a row pair (pseudospec_hd.f90:383-399,
+// pseudospec_mhd.f90 vector): the c2r of A's components, kept in registers,
+// then of B's one after the other with the partial products they enter, and the
+// r2c of the three results; neither the real fields nor the products go to
+// memory.  k_xc2r, k_cross_real and k_xr2c moved 69 field passes for the three
+// products of a stage (128^3, two stages: 460 us), this kernel 27 (277 us; one to
+// two waves per SIMD at 190 to 256 registers, 3.3 TB/s).  out may be
+// A's or B's buffers: the line that writes a row pair is the one that read it.
+struct XCross {
+  const cpx<double>* a[3];
+  const cpx<double>* b[3];
+  cpx<double>* out[3];
+};
+// five of the six components' values live at a time: up to 8 points per lane
+// stay within two waves per SIMD's registers
+template <int RS>
+constexpr bool xcross_ok() {
+  if constexpr (RS >= RS_WAVE) return keep_n<RS>() <= 8;
+  else return false;
+}
+
+template <int RS>
+__global__ void __launch_bounds__(kMaxBlock, 2) k_xcross(XCross a, LineFFT<Cd> f, int nkx,
+                                                   long npairs, double tmp) {
+#pragma clang fp contract(off)
+  SPX_PROLOGUE(Cd, f);
+  const int nx = f.n;
+  const long p = long(blockIdx.x) * f.nl + line;
+  const bool ok = p < npairs;
+  const long co = long(nkx) * (2 * (ok ? p : 0));
+  constexpr int KX = keep_n<RS>(), CH = KX >= 4 ? 4 : KX;
+  double A[3][2][KX], P1[2][KX], P2[2][KX], P3[2][KX];
+  // values of one field: use(q, row, value)
+  auto field = [&](const Cd* src, bool first, auto use) {
+    load_c2r_pair<double, KX, CH>(xl, src + co, nkx, nx, lane, f.tpl, ok, 0, nullptr);
+    if (first) __syncthreads();  // also publishes the staged twiddles
+    else line_sync(f.tpl);
+    line_fft_nosync<double, RS>(xl, f, tws, lane);
+    line_sync(f.tpl);
+#pragma unroll
+    for (int q = 0; q < KX; ++q) {
+      const int x = lane + q * f.tpl;
+      const Cd z = x < nx ? xl[x] : mkc<double>(0, 0);
+      use(q, 0, z.x);
+      use(q, 1, -z.y);
+    }
+    line_sync(f.tpl);
+  };
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    field(a.a[c], c == 0, [&](int q, int r, double v) { A[c][r][q] = v; });
+  field(a.b[0], false, [&](int q, int r, double v) {
+    P2[r][q] = A[2][r][q] * v;
+    P3[r][q] = v * A[1][r][q];
+  });
+  field(a.b[1], false, [&](int q, int r, double v) {
+    P1[r][q] = v * A[2][r][q];
+    P3[r][q] = (A[0][r][q] * v - P3[r][q]) * tmp;
+  });
+  field(a.b[2], false, [&](int q, int r, double v) {
+    P1[r][q] = (A[1][r][q] * v - P1[r][q]) * tmp;
+    P2[r][q] = (P2[r][q] - v * A[0][r][q]) * tmp;
+  });
+  auto result = [&](Cd* out, const double (&o)[2][KX]) {
+#pragma unroll
+    for (int q = 0; q < KX; ++q) {
+      const int x = lane + q * f.tpl;
+      if (x < nx) xl[x] = ok ? mkc<double>(o[0][q], o[1][q]) : mkc<double>(0, 0);
+    }
+    line_sync(f.tpl);
+    line_fft_nosync<double, RS>(xl, f, tws, lane);
+    line_sync(f.tpl);
+    if (ok) store_r2c_pair(xl, out + co, nkx, nx, lane, f.tpl);
+    line_sync(f.tpl);
+  };
+  result(a.out[0], P1);
+  result(a.out[1], P2);
+  result(a.out[2], P3);
+}
+
 // ---------------------------------------------------------------------------
 // float64 boundary kernels; TS is the storage type of the fields
 // ---------------------------------------------------------------------------
-using Cd = cpx<double>;
 using LFd = LineFFT<Cd>;
 
 // goto_domain_w_boundaries + noslip_z + goto_3d_fourier fused per line
@@ -2556,6 +2636,41 @@ int xc2r(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes,
   if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xc2r: bad field count");
   return lo ? XBackward<float>::run(p, nf, X, R, nplanes, dirx, p->fx32)
             : XBackward<double>::run(p, nf, X, R, nplanes, dirx, p->fx);
+}
+#endif
+
+#if !defined(SPX_PART) || SPX_PART == 10
+bool xcross_fused(const spx_plan* p) {
+  if (p->fp32 || !p->XV[0] || p->fx.wave < 0) return false;
+  return with_xy<16>(p->fx, [](auto rs) -> int { return xcross_ok<decltype(rs)::value>(); }) == 1;
+}
+
+int xcross(spx_plan* p, void* const* A, void* const* B, void* const* out) {
+  const long npairs = long(p->g.ny) * p->np * p->mem / 2;
+  const LineFFTHost f = spread(p->fx, npairs, 1, 1);
+  const double tmp = 1.0 / std::pow(double(p->g.nx) * double(p->g.ny) * double(p->g.nz), 2);
+  XCross a;
+  for (int c = 0; c < 3; ++c) {
+    a.a[c] = C_<double>(static_cast<const void*>(A[c]));
+    a.b[c] = C_<double>(static_cast<const void*>(B[c]));
+    a.out[c] = C_<double>(out[c]);
+  }
+  ProfScope ps_(p, "xcross", 18.0 * npairs * sizeof(Cd) * p->nkx);
+  const int rc = with_xy<16>(f, [&](auto rs) -> int {
+    constexpr int RS = decltype(rs)::value;
+    if constexpr (xcross_ok<RS>()) {
+      const size_t lds = f.lds_bytes(16);
+      if (int lrc = lds_limit(k_xcross<RS>, lds)) return lrc;
+      hipLaunchKernelGGL(k_xcross<RS>, dim3(unsigned((npairs + f.nl - 1) / f.nl)), blk(f), lds,
+                         p->stream, a, f.dev<Cd>(), p->nkx, npairs, tmp);
+      return SPX_OK;
+    } else {
+      return SPX_ERR_UNSUPPORTED;
+    }
+  });
+  if (rc) return rc;
+  SPX_CHECK_LAUNCH();
+  return SPX_OK;
 }
 #endif
 
