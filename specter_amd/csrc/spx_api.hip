@@ -299,21 +299,12 @@ static double diag_tmp(const spx_plan* p) {
   return 1.0 / (t * t) / double(p->g.nz - p->g.Cz);
 }
 
-static int fetch_parts(spx_plan* p, size_t count) {
+static int fetch_parts(spx_plan* p, size_t count, size_t from = 0) {
   if (p->h_part.size() < count) p->h_part.resize(count);
-  SPX_HIP(hipMemcpyAsync(p->h_part.data(), p->part, count * sizeof(double),
+  SPX_HIP(hipMemcpyAsync(p->h_part.data(), p->part + from, count * sizeof(double),
                          hipMemcpyDeviceToHost, p->stream));
   SPX_HIP(hipStreamSynchronize(p->stream));
   return SPX_OK;
-}
-
-// weighted sum over the (kx,ky) lines of member b: weight 1 for kx = 0, 2 otherwise
-static double weighted_sum(const spx_plan* p, const std::vector<double>& acc, int b = 0) {
-  const long ny = p->g.ny, nl = long(p->g.ny) * p->nkx, o = long(b) * nl;
-  double s0 = 0.0, s1 = 0.0;
-  for (long l = 0; l < ny; ++l) s0 += acc[o + l];
-  for (long l = ny; l < nl; ++l) s1 += acc[o + l];
-  return s0 + 2.0 * s1;
 }
 
 static inline void* coff(void* a, size_t elems, int b) {
@@ -577,8 +568,9 @@ static int plan_create(const spx_grid* g, const double* A, const double* Q, int 
   if ((rc = alloc_dev(p, &p->X, p->nc * nmembers * 16))) return bail(rc);
   if ((rc = alloc_dev(p, &p->bc, nlines * 2 * 16))) return bail(rc);
   if ((rc = alloc_dev(p, &p->pw, nlines * 2 * 16))) return bail(rc);
-  // per-line partials of the diagnostics (up to 4 per line), block maxima (64 per member)
-  const size_t nparts = std::max(nlines * 4, size_t(64) * nmembers);
+  // per-line partials of the diagnostics (up to 4 per line, then 2 sums per
+  // member), block maxima (64 per member)
+  const size_t nparts = std::max(nlines * 4 + 2 * size_t(nmembers), size_t(64) * nmembers);
   if ((rc = alloc_dev(p, reinterpret_cast<void**>(&p->part), nparts * sizeof(double))))
     return bail(rc);
   *out = p;
@@ -1066,15 +1058,34 @@ int spx_a_imposebc_and_project(spx_plan* p, void* ax, void* ay, void* az, void* 
 }
 
 // ---- diagnostics ------------------------------------------------------------------
-// (the diagnostics run in a view of all active members; acc holds one value
-// per line of every member)
-static int sumsq_lines(spx_plan* p, const LinComb& lc, std::vector<double>& acc, double w) {
-  const size_t nl = size_t(p->wlines());
+// (the diagnostics run in a view of all active members)
+// The terms' sums over the lines of each member, formed on the device: one
+// launch for the terms, one for the sums and one copy of the results (a copy of
+// every line and a host sum per term took half of hdcheck's and vdiagnostic's
+// time at 128^3).  out[value][member]; per values per line.
+static int member_sums(spx_plan* p, int nterm, const double* w, int per, double* out0,
+                       double* out1, double scale) {
+  const size_t from = 4 * size_t(p->wlines());
   int rc;
-  if ((rc = zline_sumsq(p, lc, p->part))) return rc;
-  if ((rc = fetch_parts(p, nl))) return rc;
-  for (size_t l = 0; l < nl; ++l) acc[l] += w * p->h_part[l];
+  if ((rc = line_sums(p, nterm, w, per, p->part, p->part + from))) return rc;
+  if ((rc = fetch_parts(p, size_t(per) * p->nact, from))) return rc;
+  for (int m = 0; m < p->nact; ++m) {
+    out0[m] = p->h_part[m] * scale;
+    if (per == 2) out1[m] = p->h_part[p->nact + m] * scale;
+  }
   return SPX_OK;
+}
+
+static const double kOnes[3] = {1.0, 1.0, 1.0};
+
+static int sumsq(spx_plan* p, int nterm, const LinComb* lc, const double* w, double* out) {
+  if (int rc = zline_sumsq(p, nterm, lc, p->part)) return rc;
+  return member_sums(p, nterm, w, 1, out, nullptr, diag_tmp(p));
+}
+
+static int dots(spx_plan* p, int nterm, const LinComb* lc, const void* const* b, double* out) {
+  if (int rc = zline_dot(p, nterm, lc, b, p->part)) return rc;
+  return member_sums(p, nterm, kOnes, 1, out, nullptr, diag_tmp(p));
 }
 
 static LinComb one(const void* a, int dir) {
@@ -1104,62 +1115,42 @@ int spx_energy(spx_plan* p, const void* a, const void* b, const void* c, int kin
     for (int q = 0; q < 6; ++q)
       if ((rc = alloc_dev(p, &p->MS[q], p->nc * p->nb * 16))) return rc;
   MemberView mv(p, p->nact);
-  std::vector<double> acc(size_t(p->wlines()), 0.0);
   if (kin == 1) {
-    for (const void* q : {a, b, c})
-      if ((rc = sumsq_lines(p, one(q, 0), acc, 1.0))) return rc;
-  } else if (kin == 2) {
+    const LinComb v[3] = {one(a, 0), one(b, 0), one(c, 0)};
+    return sumsq(p, 3, v, kOnes, out);
+  }
+  if (kin == 2) {
     // curl of curl by the reference's curlk calls (pseudospec_hd.f90:555-560)
     const void* v[3] = {a, b, c};
     const void* w[3] = {p->MS[0], p->MS[1], p->MS[2]};
     if ((rc = op_curl3(p, v, p->MS))) return rc;
     if ((rc = op_curl3(p, w, p->MS + 3))) return rc;
-    for (int q = 3; q < 6; ++q)
-      if ((rc = sumsq_lines(p, one(p->MS[q], 0), acc, 1.0))) return rc;
-  } else {
-    // curlk(b,c,1) = d_y c - d_z b ; curlk(a,c,2) = d_z a - d_x c, counted twice
-    // (pseudospec_hd.f90:527,540)
-    if ((rc = sumsq_lines(p, two(c, 2, b, 3, -1), acc, 1.0))) return rc;
-    if ((rc = sumsq_lines(p, two(a, 3, c, 1, -1), acc, 2.0))) return rc;
+    const LinComb cc[3] = {one(p->MS[3], 0), one(p->MS[4], 0), one(p->MS[5], 0)};
+    return sumsq(p, 3, cc, kOnes, out);
   }
-  for (int b = 0; b < p->nact; ++b) out[b] = weighted_sum(p, acc, b) * diag_tmp(p);
-  return SPX_OK;
+  // curlk(b,c,1) = d_y c - d_z b ; curlk(a,c,2) = d_z a - d_x c, counted twice
+  // (pseudospec_hd.f90:527,540)
+  const LinComb w[2] = {two(c, 2, b, 3, -1), two(a, 3, c, 1, -1)};
+  const double twice[2] = {1.0, 2.0};
+  return sumsq(p, 2, w, twice, out);
 }
 
 int spx_cross(spx_plan* p, const void* a, const void* b, const void* c, const void* d,
               const void* e, const void* f, double* out) {
   SPX_REQ(p && a && b && c && d && e && f && out, "spx_cross: null argument");
   MemberView mv(p, p->nact);
-  const size_t nl = size_t(p->wlines());
-  std::vector<double> acc(nl, 0.0);
-  const void* L[3] = {a, b, c};
-  const void* Rr[3] = {d, e, f};
-  int rc;
-  for (int t = 0; t < 3; ++t) {
-    if ((rc = zline_dot(p, L[t], Rr[t], p->part))) return rc;
-    if ((rc = fetch_parts(p, nl))) return rc;
-    for (size_t l = 0; l < nl; ++l) acc[l] += p->h_part[l];
-  }
-  for (int b = 0; b < p->nact; ++b) out[b] = weighted_sum(p, acc, b) * diag_tmp(p);
-  return SPX_OK;
+  const LinComb l[3] = {one(a, 0), one(b, 0), one(c, 0)};
+  const void* r[3] = {d, e, f};
+  return dots(p, 3, l, r, out);
 }
 
 int spx_helicity(spx_plan* p, const void* a, const void* b, const void* c, double* out) {
   SPX_REQ(p && a && b && c && out, "spx_helicity: null argument");
   MemberView mv(p, p->nact);
-  const size_t nl = size_t(p->wlines());
-  std::vector<double> acc(nl, 0.0);
   // curlk(b,c,1) = d_y c - d_z b ; curlk(a,c,2) = d_z a - d_x c ; curlk(a,b,3) = d_x b - d_y a
   const LinComb w[3] = {two(c, 2, b, 3, -1), two(a, 3, c, 1, -1), two(b, 1, a, 2, -1)};
   const void* v[3] = {a, b, c};
-  int rc;
-  for (int t = 0; t < 3; ++t) {
-    if ((rc = zline_dot_lc(p, w[t], v[t], p->part))) return rc;
-    if ((rc = fetch_parts(p, nl))) return rc;
-    for (size_t l = 0; l < nl; ++l) acc[l] += p->h_part[l];
-  }
-  for (int m = 0; m < p->nact; ++m) out[m] = weighted_sum(p, acc, m) * diag_tmp(p);
-  return SPX_OK;
+  return dots(p, 3, w, v, out);
 }
 
 int spx_divergence(spx_plan* p, const void* a, const void* b, const void* c, double* out) {
@@ -1169,34 +1160,16 @@ int spx_divergence(spx_plan* p, const void* a, const void* b, const void* c, dou
   lc.dir[2] = 3;
   lc.sgn[2] = 1;
   MemberView mv(p, p->nact);
-  std::vector<double> acc(size_t(p->wlines()), 0.0);
-  int rc = sumsq_lines(p, lc, acc, 1.0);
-  if (rc) return rc;
-  for (int m = 0; m < p->nact; ++m) out[m] = weighted_sum(p, acc, m) * diag_tmp(p);
-  return SPX_OK;
+  return sumsq(p, 1, &lc, kOnes, out);
 }
 
 int spx_bouncheck_z(spx_plan* p, const void* a, const void* b, double* bot, double* top) {
   SPX_REQ(p && a && bot && top, "spx_bouncheck_z: null argument");
   MemberView mv(p, p->nact);
-  const size_t nl = size_t(p->wlines());
-  std::vector<double> ab(nl, 0.0), at(nl, 0.0);
-  int rc;
-  for (const void* q : {a, b}) {
-    if (!q) continue;
-    if ((rc = zline_walls(p, q, p->part))) return rc;
-    if ((rc = fetch_parts(p, 2 * nl))) return rc;
-    for (size_t l = 0; l < nl; ++l) {
-      ab[l] += p->h_part[2 * l];
-      at[l] += p->h_part[2 * l + 1];
-    }
-  }
+  const LinComb v[2] = {one(a, 0), one(b, 0)};
+  if (int rc = zline_walls(p, b ? 2 : 1, v, p->part)) return rc;
   const double t = 1.0 / double(long(p->g.nx) * p->g.ny * p->g.nz);
-  for (int m = 0; m < p->nact; ++m) {
-    bot[m] = weighted_sum(p, ab, m) * (t * t);
-    top[m] = weighted_sum(p, at, m) * (t * t);
-  }
-  return SPX_OK;
+  return member_sums(p, b ? 2 : 1, kOnes, 2, bot, top, t * t);
 }
 
 // ---- scalar and wall diagnostics ---------------------------------------------------
@@ -1204,23 +1177,15 @@ int spx_variance(spx_plan* p, const void* a, int kin, double* out) {
   SPX_REQ(p && a && out, "spx_variance: null argument");
   SPX_REQ(kin == 0 || kin == 1, "spx_variance: kin must be 0 or 1");
   MemberView mv(p, p->nact);
-  std::vector<double> acc(size_t(p->wlines()), 0.0);
-  int rc = sumsq_lines(p, one(a, kin == 1 ? 0 : 4), acc, 1.0);
-  if (rc) return rc;
-  for (int m = 0; m < p->nact; ++m) out[m] = weighted_sum(p, acc, m) * diag_tmp(p);
-  return SPX_OK;
+  const LinComb v = one(a, kin == 1 ? 0 : 4);
+  return sumsq(p, 1, &v, kOnes, out);
 }
 
 int spx_product(spx_plan* p, const void* a, const void* b, double* out) {
   SPX_REQ(p && a && b && out, "spx_product: null argument");
   MemberView mv(p, p->nact);
-  const size_t nl = size_t(p->wlines());
-  int rc;
-  if ((rc = zline_dot(p, a, b, p->part))) return rc;
-  if ((rc = fetch_parts(p, nl))) return rc;
-  std::vector<double> acc(p->h_part.begin(), p->h_part.begin() + nl);
-  for (int m = 0; m < p->nact; ++m) out[m] = weighted_sum(p, acc, m) * diag_tmp(p);
-  return SPX_OK;
+  const LinComb l = one(a, 0);
+  return dots(p, 1, &l, &b, out);
 }
 
 // horizontal means of d a/dz at z = 0 and z = Lz (physical units), per member
@@ -1297,10 +1262,12 @@ int spx_energy_spectrum(spx_plan* p, const void* a, const void* b, const void* c
                         double* out) {
   SPX_REQ(p && a && b && c && out && nbins > 0, "spx_energy_spectrum: bad argument");
   MemberView mv(p, p->nact);
-  std::vector<double> acc(size_t(p->wlines()), 0.0);
+  const size_t all = size_t(p->wlines());
+  const LinComb v[3] = {one(a, 0), one(b, 0), one(c, 0)};
   int rc;
-  for (const void* q : {a, b, c})
-    if ((rc = sumsq_lines(p, one(q, 0), acc, 1.0))) return rc;
+  if ((rc = zline_sumsq(p, 3, v, p->part))) return rc;
+  if ((rc = fetch_parts(p, 3 * all))) return rc;
+  const std::vector<double>& part = p->h_part;
   const long ny = p->g.ny, nl = long(p->g.ny) * p->nkx;
   const double tmp = diag_tmp(p);
   for (int m = 0; m < p->nact; ++m) {
@@ -1310,7 +1277,9 @@ int spx_energy_spectrum(spx_plan* p, const void* a, const void* b, const void* c
       const long i = l / ny, j = l - i * ny;
       const double kh = std::sqrt(p->h_kx[i] * p->h_kx[i] + p->h_ky[j] * p->h_ky[j]) / p->Dkx;
       const long sh = long(std::floor(kh + 0.5));
-      if (sh < nbins) o[sh] += (i == 0 ? 1.0 : 2.0) * acc[size_t(m) * nl + l] * tmp;
+      const size_t at = size_t(m) * nl + l;
+      const double e = (part[at] + part[all + at]) + part[2 * all + at];
+      if (sh < nbins) o[sh] += (i == 0 ? 1.0 : 2.0) * e * tmp;
     }
   }
   return SPX_OK;

@@ -420,11 +420,14 @@ struct LinComb {
 // also advect (pseudospec_phd.f90:23-113) of th into out[3]
 int gradre_impl(spx_plan* p, const void* const v[3], const void* th, void* const* out);
 
-int zline_sumsq(spx_plan* p, const LinComb& lc, double* line_out);
-int zline_dot(spx_plan* p, const void* a, const void* b, double* line_out);
-// sum_k<np Re(IFFT(lincomb) conj IFFT(b)) per line
-int zline_dot_lc(spx_plan* p, const LinComb& lc, const void* b, double* line_out);
-int zline_walls(spx_plan* p, const void* a, double* line_out /*2 per line*/);
+// one value per line (walls: two) of up to three terms in one launch, term t's
+// lines from line_out + t wlines() on.  dot: sum_k<np Re(IFFT(lincomb) conj IFFT(b))
+int zline_sumsq(spx_plan* p, int nterm, const LinComb* lc, double* line_out);
+int zline_dot(spx_plan* p, int nterm, const LinComb* lc, const void* const* b, double* line_out);
+int zline_walls(spx_plan* p, int nterm, const LinComb* lc, double* line_out /*2 per line*/);
+// the weighted sum of the terms over each member's lines (kx > 0 twice) of each
+// of the per values: out[value][member]
+int line_sums(spx_plan* p, int nterm, const double* w, int per, const double* part, double* out);
 // IFFT_z(lincomb) at z = 0 and z = Lz: (re, im) bottom, (re, im) top per line
 int zline_wall_values(spx_plan* p, const LinComb& lc, double* line_out /*4 per line*/);
 

@@ -1688,12 +1688,20 @@ __device__ __forceinline__ Cd deriv_apply(Cd v, int dirn, double kxi, double kyj
   return v;
 }
 
+// The terms of one diagnostic (blockIdx.y): a field or combination each, with
+// its factor field of mode 1.
+template <typename TS>
+struct ZTerms {
+  LinCombDev<TS> lc[3];
+  const cpx<TS>* b[3];
+};
+
 // mode 0: sum_k<np |IFFT(lincomb)|^2 ; mode 1: Re(IFFT(a) conj IFFT(b)) ; mode 2: walls |.|^2 ;
-// mode 3: the wall values IFFT(lincomb) at z = 0 and z = Lz (4 doubles per line)
+// mode 3: the wall values IFFT(lincomb) at z = 0 and z = Lz (4 doubles per line).
+// Term t writes its lines' values at out + t nlines (1, 2 or 4 doubles).
 template <typename TS, int RS>
-__global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(LinCombDev<TS> lc,
-                                                      const cpx<TS>* __restrict__ bsrc, int mode,
-                                                      double* __restrict__ out, LFd f,
+__global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(ZTerms<TS> terms, int mode,
+                                                      double* __restrict__ outs, LFd f,
                                                       long nlines, int ny, int np,
                                                       const double* __restrict__ kx,
                                                       const double* __restrict__ ky,
@@ -1701,6 +1709,9 @@ __global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(LinCombDev<TS> lc,
 #pragma clang fp contract(off)
   SPX_PROLOGUE(Cd, f);
   const int n = f.n;
+  const LinCombDev<TS>& lc = terms.lc[blockIdx.y];
+  const cpx<TS>* __restrict__ bsrc = terms.b[blockIdx.y];
+  double* __restrict__ out = outs + blockIdx.y * nlines * (mode == 3 ? 4 : (mode == 2 ? 2 : 1));
   Cd* const ldsB = lds + f.nl * f.ldl;
   Cd* const xb = ldsB + line * f.ldl;
   double* red = reinterpret_cast<double*>(ldsB + (mode == 1 ? f.nl * f.ldl : 0));
@@ -1759,6 +1770,36 @@ __global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(LinCombDev<TS> lc,
   const double s = line_reduce(acc, red, line, lane, f.tpl);
   if (lane == 0 && ok) out[ln] = s;
 }
+
+#if !defined(SPX_PART) || SPX_PART == 8
+// The sum over a member's (kx, ky) lines of the weighted terms, lines of kx > 0
+// counted twice: blockIdx.x member, blockIdx.y which of the line's per values.
+// In a fixed order: a thread's lines upwards, then a tree over the threads.
+struct LineWeights {
+  double w[3];
+};
+__global__ void __launch_bounds__(1024) k_line_sum(const double* __restrict__ part, LineWeights w,
+                                             int nterm, int per, long nl, int ny,
+                                             double* __restrict__ out) {
+#pragma clang fp contract(off)
+  __shared__ double red[1024];
+  const long lines = nl * gridDim.x, l0 = nl * blockIdx.x;
+  double s = 0.0;
+  for (long l = threadIdx.x; l < nl; l += 1024) {
+    double a = 0.0;
+    for (int t = 0; t < nterm; ++t)
+      a += w.w[t] * part[(t * lines + l0 + l) * per + blockIdx.y];
+    s += l < ny ? a : 2.0 * a;
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int q = 512; q > 0; q >>= 1) {
+    if (threadIdx.x < q) red[threadIdx.x] += red[threadIdx.x + q];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+}
+#endif
 
 #if !defined(SPX_PART) || SPX_PART == 1
 // ---------------------------------------------------------------------------
@@ -3081,55 +3122,54 @@ int proj_pressure(spx_plan* p, void* d, int k0, int k1) {
 #endif  // SPX_PART 16 (magnetic walls, pressure)
 
 #if !defined(SPX_PART) || SPX_PART == 8
-static int zline_launch(spx_plan* p, const LinComb& lc, const void* b, int mode, double* out) {
+static int zline_launch(spx_plan* p, int nterm, const LinComb* lc, const void* const* b, int mode,
+                        double* out) {
+  if (nterm < 1 || nterm > 3) return fail(SPX_ERR_ARG, "zline_reduce: 1..3 terms");
   const LineFFTHost& fw = fzt(p, false);
   const LineFFTHost f = mode == 1 ? fw.with_lines(fw.nl / 2) : fw;
   const long nlines = p->wlines();
-  LinCombDev<double> d;
-  for (int t = 0; t < 3; ++t) {
-    d.in[t] = static_cast<const Cd*>(lc.in[t]);
-    d.dir[t] = lc.dir[t];
-    d.sgn[t] = lc.sgn[t];
+  ZTerms<double> d;
+  for (int q = 0; q < 3; ++q) {
+    const LinComb& c = lc[q < nterm ? q : 0];
+    for (int t = 0; t < 3; ++t) {
+      d.lc[q].in[t] = static_cast<const Cd*>(c.in[t]);
+      d.lc[q].dir[t] = c.dir[t];
+      d.lc[q].sgn[t] = c.sgn[t];
+    }
+    d.b[q] = b ? C_<double>(b[q < nterm ? q : 0]) : nullptr;
   }
   const size_t lds = f.lds_bytes(16, mode == 1 ? 2 : 1) + size_t(f.nl) * f.tpl * sizeof(double);
-  ProfScope ps_(p, "zline_reduce", double(p->wnc()) * 16.0 * (mode == 1 ? 2 : 1));
-  SPX_LAUNCH(with_z<16>, f, k_zline_reduce, double, , dim3(unsigned((nlines + f.nl - 1) / f.nl)), blk(f),
-                lds, p->stream, d, C_<double>(b), mode, out, f.dev<Cd>(), nlines, p->g.ny, p->np,
-                p->d_kx, p->d_ky, p->d_kz);
+  ProfScope ps_(p, "zline_reduce", nterm * double(p->wnc()) * 16.0 * (mode == 1 ? 2 : 1));
+  SPX_LAUNCH(with_z<16>, f, k_zline_reduce, double, ,
+             dim3(unsigned((nlines + f.nl - 1) / f.nl), unsigned(nterm)), blk(f), lds, p->stream, d,
+             mode, out, f.dev<Cd>(), nlines, p->g.ny, p->np, p->d_kx, p->d_ky, p->d_kz);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }
 
-int zline_sumsq(spx_plan* p, const LinComb& lc, double* line_out) {
-  return zline_launch(p, lc, nullptr, 0, line_out);
+int zline_sumsq(spx_plan* p, int nterm, const LinComb* lc, double* line_out) {
+  return zline_launch(p, nterm, lc, nullptr, 0, line_out);
 }
 
-int zline_dot(spx_plan* p, const void* a, const void* b, double* line_out) {
-  LinComb lc;
-  lc.in[0] = a;
-  lc.in[1] = lc.in[2] = nullptr;
-  lc.dir[0] = lc.dir[1] = lc.dir[2] = 0;
-  lc.sgn[0] = 1;
-  lc.sgn[1] = lc.sgn[2] = 0;
-  return zline_launch(p, lc, b, 1, line_out);
-}
-
-int zline_dot_lc(spx_plan* p, const LinComb& lc, const void* b, double* line_out) {
-  return zline_launch(p, lc, b, 1, line_out);
+int zline_dot(spx_plan* p, int nterm, const LinComb* lc, const void* const* b, double* line_out) {
+  return zline_launch(p, nterm, lc, b, 1, line_out);
 }
 
 int zline_wall_values(spx_plan* p, const LinComb& lc, double* line_out) {
-  return zline_launch(p, lc, nullptr, 3, line_out);
+  return zline_launch(p, 1, &lc, nullptr, 3, line_out);
 }
 
-int zline_walls(spx_plan* p, const void* a, double* line_out) {
-  LinComb lc;
-  lc.in[0] = a;
-  lc.in[1] = lc.in[2] = nullptr;
-  lc.dir[0] = lc.dir[1] = lc.dir[2] = 0;
-  lc.sgn[0] = 1;
-  lc.sgn[1] = lc.sgn[2] = 0;
-  return zline_launch(p, lc, nullptr, 2, line_out);
+int zline_walls(spx_plan* p, int nterm, const LinComb* lc, double* line_out) {
+  return zline_launch(p, nterm, lc, nullptr, 2, line_out);
+}
+
+int line_sums(spx_plan* p, int nterm, const double* w, int per, const double* part, double* out) {
+  LineWeights lw;
+  for (int t = 0; t < 3; ++t) lw.w[t] = t < nterm ? w[t] : 0.0;
+  hipLaunchKernelGGL(k_line_sum, dim3(unsigned(p->mem), unsigned(per)), dim3(1024), 0, p->stream,
+                     part, lw, nterm, per, p->wlines() / p->mem, p->g.ny, out);
+  SPX_CHECK_LAUNCH();
+  return SPX_OK;
 }
 #endif  // SPX_PART 8 (diagnostics)
 
