@@ -77,7 +77,7 @@ static int upload(spx_plan* p, double** dst, const V& host) {
 // the boundary-plane buffers of mixed plans) and the advect additions
 static void work_sizes(const spx_plan* p, size_t* hd, size_t* bouss) {
   const size_t cb = p->nc * p->nb * p->csize, rb = p->nr * p->nb * p->rsize;
-  size_t h = 3 * (3 * cb + rb) + p->nr * p->nb * 8;
+  size_t h = 3 * (3 * cb + rb);
   if (p->fp32 && p->g.Cz > 0) {
     const size_t d2 = 2 * size_t(p->g.oz), nbm = size_t(p->nb);
     const size_t bc = size_t(p->nkx) * p->g.ny * d2 * nbm * 16;
@@ -108,7 +108,6 @@ static int ensure_work(spx_plan* p, bool bouss) {
           (rc = alloc_dev(p, &p->XY[c], cb)) || (rc = alloc_dev(p, &p->RV[c], rb)))
         return rc;
     }
-    if ((rc = alloc_dev(p, &p->R0, p->nr * p->nb * 8))) return rc;
   }
   if (bouss && !p->work_bouss) {
     if ((rc = alloc_dev(p, &p->XV[3], cb)) || (rc = alloc_dev(p, &p->XZ[3], cb)) ||
@@ -1538,10 +1537,13 @@ static int substep_impl(spx_plan* p, spx_state* s, int o, bool full_pressure) {
   if (rot) return SPX_OK;
   if ((rc = op_filter(p, s->th))) return rc;
   // round trip of th through real space (include/bouss/bouss_rkstep2.f90:56-59)
-  if ((rc = c2r3(p, s->th, p->R0, 0, p->np))) return rc;
-  if ((rc = op_real_div3(p, p->R0, double(p->g.nx), double(p->g.ny), double(p->g.nz))))
-    return rc;
-  return r2c3(p, p->R0, s->th);
+  const void* th = s->th;
+  const void* x = p->X;
+  if ((rc = zfft_s2x(p, 1, &th, &p->X, 0, p->np, 0))) return rc;
+  if ((rc = yfft(p, 1, &x, &p->X, 0, p->np))) return rc;
+  if ((rc = xround(p, p->X))) return rc;
+  if ((rc = yfft(p, 1, &x, &p->X, 1, p->np, nullptr, false, p->Cy > 0))) return rc;
+  return zfft_x2s(p, 1, &x, &s->th, 0);
 }
 
 int spx_substep(spx_plan* p, spx_state* s, int o) { return substep_impl(p, s, o, true); }

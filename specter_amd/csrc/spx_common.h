@@ -186,7 +186,6 @@ struct spx_plan {
   void* XZ[4] = {nullptr};
   void* XY[4] = {nullptr};
   void* RV[3] = {nullptr};
-  void* R0 = nullptr;       // general real scratch (Boussinesq round trip)
   // MHD: real work fields (physical planes of every member), allocated on
   // first use by prodre / vector / the MHD stage; Neumann vectors neu
   // (order 1) and neu2 (order 2) of the z walls (fcgram_mod.f90:347-355)
@@ -358,6 +357,9 @@ int xgrad_prod(spx_plan* p, int nf, const void* const* YV, const void* const* YY
 // otherwise
 int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
                 void* const* RV, void* const* out, bool lo);
+// the x stage of a round trip through real space with the division by nx ny nz,
+// in place on the np planes of float64 half spectra
+int xround(spx_plan* p, void* X);
 // the x stage of out = A x B on the np planes of float64 half spectra, tmp =
 // 1 / (nx ny nz)^2 as op_cross_real; out may be A or B.  xcross_fused: whether the
 // plan's x lines have it (else SPX_ERR_UNSUPPORTED) and its work arrays exist
@@ -471,6 +473,5 @@ int op_coriolis(spx_plan* p, void* const* nl, const void* const* v, const double
 int op_div_spec(spx_plan* p, const void* a, const void* b, const void* c, void* d);
 // per member: block maxima of |r| over n values at member stride ms -> out[member][block]
 int op_absmax(spx_plan* p, const void* r, long n, long ms, double* out, int* nblocks);
-int op_real_div3(spx_plan* p, void* r, double nx, double ny, double nz);
 
 }  // namespace spx

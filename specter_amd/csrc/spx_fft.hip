@@ -857,6 +857,34 @@ __global__ void __launch_bounds__(kMaxBlock) k_xc2r(XFields<T> a, LineFFT<cpx<T>
   }
 }
 
+// The x stage of a field's round trip through real space: c2r, ((r/nx)/ny)/nz
+// (include/bouss/bouss_rkstep2.f90:57) and r2c of a row pair in LDS, in place on
+// its half spectra.  Two field passes instead of the six of k_xc2r, a division
+// pass and k_xr2c: 128^3 float64 36 us in three launches, 23 here, bound by the
+// three divisions a value.
+template <int RS>
+__global__ void __launch_bounds__(kMaxBlock) k_xround(cpx<double>* __restrict__ X,
+                                                LineFFT<cpx<double>> f, int nkx, long npairs,
+                                                double ny, double nz) {
+#pragma clang fp contract(off)
+  using Cp = cpx<double>;
+  SPX_PROLOGUE(Cp, f);
+  const int nx = f.n;
+  const long p = long(blockIdx.x) * f.nl + line;
+  const bool ok = p < npairs;
+  Cp* xs = X + long(nkx) * (2 * (ok ? p : 0));
+  load_c2r_pair<double, batch_n<RS>()>(xl, xs, nkx, nx, lane, f.tpl, ok, 0, nullptr);
+  __syncthreads();
+  zline_dft<double, RS>(xl, f, tws, lane);
+  for (int x = lane; x < nx; x += f.tpl) {
+    const Cp z = xl[x];
+    xl[x] = mkc<double>(((z.x / double(nx)) / ny) / nz, ((-z.y / double(nx)) / ny) / nz);
+  }
+  __syncthreads();
+  zline_dft<double, RS>(xl, f, tws, lane);
+  if (ok) store_r2c_pair(xl, xs, nkx, nx, lane, f.tpl);
+}
+
 // ((u*Dx + v*Dy) + w*Dz)*tmp on a row pair, the three derivatives c2r'd in
 // LDS one after the other and accumulated in registers
 // (pseudospec_hd.f90:254-312, pseudospec_phd.f90:63-108), then the r2c of the
@@ -2681,6 +2709,24 @@ int xc2r(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes,
 #endif
 
 #if !defined(SPX_PART) || SPX_PART == 10
+int xround(spx_plan* p, void* X) {
+  const long npairs = long(p->g.ny) * p->np * p->mem / 2;
+  const LineFFTHost f = spread(p->fx, npairs, 1, 1);
+  ProfScope ps_(p, "xround", 4.0 * npairs * sizeof(Cd) * p->nkx);
+  const int rc = with_xy<16>(f, [&](auto rs) -> int {
+    constexpr int RS = decltype(rs)::value;
+    const size_t lds = f.lds_bytes(16);
+    if (int lrc = lds_limit(k_xround<RS>, lds)) return lrc;
+    hipLaunchKernelGGL(k_xround<RS>, dim3(unsigned((npairs + f.nl - 1) / f.nl)), blk(f), lds,
+                       p->stream, C_<double>(X), f.dev<Cd>(), p->nkx, npairs, double(p->g.ny),
+                       double(p->g.nz));
+    return SPX_OK;
+  });
+  if (rc) return rc;
+  SPX_CHECK_LAUNCH();
+  return SPX_OK;
+}
+
 bool xcross_fused(const spx_plan* p) {
   if (p->fp32 || !p->XV[0] || p->fx.wave < 0) return false;
   return with_xy<16>(p->fx, [](auto rs) -> int { return xcross_ok<decltype(rs)::value>(); }) == 1;

@@ -87,14 +87,6 @@ __global__ void k_scale(TR* __restrict__ a, long n, double s) {
   if (e < n) a[e] = TR(double(a[e]) * s);
 }
 
-// real r <- ((r/nx)/ny)/nz  (include/bouss/bouss_rkstep2.f90:57)
-template <typename TR>
-__global__ void k_div3(TR* __restrict__ r, long n, double a, double b, double c) {
-#pragma clang fp contract(off)
-  const long e = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e < n) r[e] = TR(((double(r[e]) / a) / b) / c);
-}
-
 // Fused fc_filter(N) + laplak(v) + RK stage update (include/hd/hd_rkstep2.f90:11-32):
 //   v = C0 + dt*(nu*(-kk2 v) - ((N*fx)*fy)*fz + F)*rmp
 // with the Boussinesq source N <- N - coef*src applied first
@@ -550,15 +542,6 @@ int op_scale(spx_plan* p, void* a, size_t n, double s) {
   ProfScope ps_(p, "scale", 16.0 * double(n));
   hipLaunchKernelGGL(k_scale<double>, dim3(nblk(long(n))), dim3(256), 0, p->stream,
                      static_cast<double*>(a), long(n), s);
-  SPX_CHECK_LAUNCH();
-  return SPX_OK;
-}
-
-int op_real_div3(spx_plan* p, void* r, double a, double b, double c) {
-  const long n = long(p->g.nx) * p->g.ny * p->np * p->mem;
-  ProfScope ps_(p, "real_div3", 16.0 * double(n));
-  hipLaunchKernelGGL(k_div3<double>, dim3(nblk(n)), dim3(256), 0, p->stream,
-                     static_cast<double*>(r), n, a, b, c);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
 }

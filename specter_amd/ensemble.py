@@ -125,7 +125,7 @@ def member_bytes(req: RunRequest) -> int:
     nc, nr = nz * ny * nkx, nx * ny * nz
     c = 8 if req.precision == _l.SPX_FP32_MIXED else 16
     r = c // 2
-    return 13 * nc * 16 + 12 * nc * c + 3 * nr * r + nr * 8 + 2 * nc * 16
+    return 13 * nc * 16 + 12 * nc * c + 3 * nr * r + 2 * nc * 16
 
 
 class _Class:
