@@ -866,9 +866,22 @@ SPX_WAVE_PLAN(43, 0, 125, 32, 0, 0, 0, 5, 5, 5)
 SPX_WAVE_PLAN(44, 0, 169, 16, 0, 0, 0, 13, 13)
 SPX_WAVE_PLAN(45, 0, 175, 32, 0, 0, 0, 5, 5, 7)
 SPX_WAVE_PLAN(46, 0, 225, 32, 0, 0, 0, 9, 5, 5)
+// further even direct lengths, with the engine's radices (transforms of
+// 180x24x88 both ways on the engine 45.2 us, here 32.8; HD step of 108x34x49
+// float64 253 -> 233 us)
+SPX_WAVE_PLAN(47, 0, 24, 4, 0, 0, 1, 8, 3)
+SPX_WAVE_PLAN(48, 0, 40, 8, 0, 0, 1, 8, 5)
+SPX_WAVE_PLAN(49, 0, 60, 16, 0, 0, 1, 4, 3, 5)
+SPX_WAVE_PLAN(50, 0, 72, 8, 0, 0, 1, 8, 9)
+SPX_WAVE_PLAN(51, 0, 88, 16, 0, 0, 1, 8, 11)
+SPX_WAVE_PLAN(52, 0, 90, 16, 0, 0, 0, 2, 9, 5)
+SPX_WAVE_PLAN(53, 0, 100, 32, 0, 0, 1, 4, 5, 5)
+SPX_WAVE_PLAN(54, 0, 108, 16, 0, 0, 1, 4, 9, 3)
+SPX_WAVE_PLAN(55, 0, 180, 32, 0, 0, 1, 4, 9, 5)
+SPX_WAVE_PLAN(56, 0, 200, 32, 0, 0, 1, 8, 5, 5)
 #undef SPX_WAVE_PLAN
 #undef SPX_PLAN
-constexpr int kWavePlans = 47;
+constexpr int kWavePlans = 57;
 template <int RS>
 struct WavePlanOf {
   using type = typename WavePlanN<RS - RS_WAVE>::type;

@@ -15,7 +15,8 @@ from conftest import TABLES, rel_err, rel_l2
 
 pytestmark = pytest.mark.gpu
 
-DIRECT = (32, 48, 64, 80, 96, 120, 128, 144, 160, 192, 240, 256, 288, 320, 384, 512, 1024)
+DIRECT = (24, 32, 40, 48, 60, 64, 72, 80, 88, 90, 96, 100, 108, 120, 128, 144, 160, 180, 192, 200,
+          240, 256, 288, 320, 384, 512, 1024)
 ODD = (75, 91, 105, 121, 125, 169, 175, 225)
 RUNGS = (120, 128, 192, 256, 315, 320, 375, 384, 441, 448, 512, 640, 700, 720, 840, 900, 1080)
 
