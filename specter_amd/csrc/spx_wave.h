@@ -596,7 +596,12 @@ template <int M, int L, int MODE, int TWM, int PAD, int... Rs>
 struct WavePlan {
   static constexpr int n = 0, m = M, mode = MODE, lanes = L, twm = TWM;  // n: any
   static constexpr bool natural = false;
-  static constexpr bool xy = MODE == 0 && M % 2 == 0;  // compiled for x and y lines too
+  static constexpr bool y = MODE == 0 && M % 2 == 0;  // compiled for y lines too
+  // and for x lines, whose fused stages hold a row pair's fields in registers: on
+  // 64 lanes 1024 points (16 a lane) spill 291 registers in float32 and more than the
+  // float64 stage can hold, so they stay on the engine's 128 threads (gradre of
+  // 1024 x 1024 x 64: 6.93 / 6.92 ms mixed / float64 there, 9.14 / 11.67 here)
+  static constexpr bool x = y && (M + L - 1) / L <= 10;
   static constexpr int nmax = MODE == 1 ? (M + 1) / 2 : (MODE == 2 ? M + 1 : M);
   static constexpr int ldl = M + (PAD ? M / RadixProduct<Rs...>::first : 0) + 1;
   static_assert(RadixProduct<Rs...>::value == M, "radices do not multiply to M");
@@ -744,7 +749,7 @@ template <int N, int M, int MODE, int TWM, int... Rs>
 struct FixedPlan {
   static constexpr int n = N, m = M, mode = MODE, lanes = 64, nmax = N, twm = TWM;
   static constexpr int ldl = M + 1, tab = M, npass = 0;
-  static constexpr bool natural = true, xy = MODE == 0 && M % 2 == 0;
+  static constexpr bool natural = true, y = MODE == 0 && M % 2 == 0, x = y;
   static constexpr const int* radix = nullptr;
   static constexpr int lines(int csize) {
     return (size_t(M) + 8 * (size_t(M) + 1)) * csize <= 160 * 1024 ? 8 : 0;
