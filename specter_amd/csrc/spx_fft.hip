@@ -144,6 +144,10 @@ __device__ __forceinline__ unsigned xcd_tile() {
 // in the x stage (24 launches per HD stage before, 9 now) an RK2 step of 32^3
 // takes 318 us instead of 529, Boussinesq 128^3 RK4 4.01 ms instead of 4.98,
 // MHD 128^3 RK2 3.42 ms instead of 4.21, HD 256^3 RK4 14.6 ms instead of 15.4.
+// The kernels read their field's pointers ahead of the prologue, together with its
+// own arguments: after it, their cold reads were two to four percent of a small
+// launch (transforms both ways on the engine's lines, us: 36x30x65 38.4 -> 36.9,
+// 54x56x71 47.8 -> 46.2, 28x26x49 41.7 -> 39.6, 110x98x110 79.3 -> 77.1).
 constexpr int kMaxComp = 8;
 
 // ---------------------------------------------------------------------------
@@ -232,11 +236,12 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_z_x2s(ZX2S<
                                                const double* __restrict__ dir, int C, int d,
                                                long xstride) {
   using Cp = cpx<T>;
+  const Cp* __restrict__ X = a.x[blockIdx.y] + blockIdx.z * xstride;
+  Cp* __restrict__ S = a.s[blockIdx.y];
   SPX_PROLOGUE(Cp, f);
   const int n = f.n;
   const long pl = long(nkx) * ny;
-  const Cp* __restrict__ X = a.x[blockIdx.y] + blockIdx.z * xstride;
-  Cp* __restrict__ S = a.s[blockIdx.y] + blockIdx.z * (pl * n);
+  S += blockIdx.z * (pl * n);
   const int e0 = int(xcd_tile()) * f.nl;
   const int nlines = int(pl);
   const int nload = nofft ? n : np;
@@ -436,10 +441,12 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_z_s2x(ZS2X<
                                                const double* __restrict__ ky,
                                                const double* __restrict__ kz) {
   using Cp = cpx<T>;
+  const cpx<TI>* __restrict__ S = a.s[blockIdx.y];
+  Cp* __restrict__ X = a.x[blockIdx.y];
   SPX_PROLOGUE(Cp, f);
   const int n = f.n;
   const long pl = long(nkx) * ny;
-  const cpx<TI>* __restrict__ S = a.s[blockIdx.y] + blockIdx.z * (pl * n);
+  S += blockIdx.z * (pl * n);
   const int e0 = int(xcd_tile()) * f.nl;
   const int nlines = int(pl);
   const bool ok = e0 + line < nlines;
@@ -505,7 +512,7 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_z_s2x(ZS2X<
   // (batched stores measured slower here: the z line kernels are VALU-bound)
   constexpr int KB = 0;
   if (e < nlines) {
-    Cp* __restrict__ xo = a.x[blockIdx.y] + blockIdx.z * (pl * nzout) + e;
+    Cp* __restrict__ xo = X + blockIdx.z * (pl * nzout) + e;
     lds_to_global<KB, Cp>(
         tid >> f.lgnl, f.tpl, nzout, [&](int k) { return cconj(lds[l * f.ldl + k]); },
         [&](int k, Cp v) { xo[pl * k] = v; });
@@ -553,13 +560,14 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_y(YFields<T
                                            const double* __restrict__ ky, int npy, int Cy, int oy,
                                            const double* __restrict__ diry) {
   using Cp = cpx<T>;
+  const Cp* const Xin = a.in[blockIdx.y];
+  Cp* const Xout = a.out[blockIdx.y];
   SPX_PROLOGUE(Cp, f);
   const int l = tid & (f.nl - 1);
   const long e = long(xcd_tile()) * f.nl + l;
   const bool in = e < nlines;
   const long plane = in ? e / nkx : 0;
   const long base = plane * nkx * ny + (in ? e - plane * nkx : 0);
-  const Cp* const Xin = a.in[blockIdx.y];
   const bool cont = forward && Cy > 0;
   const int nload = cont ? npy : ny;
   if constexpr (RS >= RS_WAVE) {
@@ -604,7 +612,7 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_y(YFields<T
   zline_dft<T, RS>(xl, f, tws, lane);
   constexpr int KB = RS >= RS_WAVE ? keep_n<RS>() : 0;
   if (in) {
-    Cp* xo = a.out[blockIdx.y] + base;
+    Cp* xo = Xout + base;
     lds_to_global<KB, Cp>(
         tid >> f.lgnl, f.tpl, ny,
         [&](int jy) {
@@ -660,9 +668,9 @@ template <typename T, int RS>
 __global__ void __launch_bounds__(kMaxBlock) k_xr2c(XFields<T> a, LineFFT<cpx<T>> f, int nkx,
                                               long npairs) {
   using Cp = cpx<T>;
-  SPX_PROLOGUE(Cp, f);
   const T* __restrict__ R = static_cast<const T*>(a.in[blockIdx.y]);
   Cp* __restrict__ X = static_cast<Cp*>(a.out[blockIdx.y]);
+  SPX_PROLOGUE(Cp, f);
   const int nx = f.n;
   const long p = long(blockIdx.x) * f.nl + line;
   const bool ok = p < npairs;
@@ -837,9 +845,9 @@ __global__ void __launch_bounds__(kMaxBlock) k_xc2r(XFields<T> a, LineFFT<cpx<T>
                                               long npairs, int dirx,
                                               const double* __restrict__ kx) {
   using Cp = cpx<T>;
-  SPX_PROLOGUE(Cp, f);
   const Cp* __restrict__ X = static_cast<const Cp*>(a.in[blockIdx.y]);
   T* __restrict__ R = static_cast<T*>(a.out[blockIdx.y]);
+  SPX_PROLOGUE(Cp, f);
   const int nx = f.n;
   const long p = long(blockIdx.x) * f.nl + line;
   const bool ok = p < npairs;
