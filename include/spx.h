@@ -103,8 +103,9 @@ int spx_plan_get_info(const spx_plan* p, spx_plan_info* info);
  * lines per workgroup and threads per line (powers of two; 0 = default) and
  * the Rader / Bluestein tables in global memory (1), LDS (0) or default (-1);
  * values the engine cannot run (LDS, 512 threads, fewer threads than the
- * length needs) are ignored.  spx_tune_wall: kappa blocks per wave (9, 18)
- * and waves per SIMD (3, 4) of the wall kernel for lines of length n. */
+ * length needs) are ignored.  spx_tune_wall: kappa blocks per wave (9, 18;
+ * 0 = default) and waves per SIMD (3, 4) of the wall kernel for lines of
+ * length n. */
 int spx_tune_line(int n, int csize, int lines, int threads, int tables_global);
 int spx_tune_wall(int n, int blocks_per_wave, int waves_per_simd);
 int spx_tune_clear(void);

@@ -7,8 +7,9 @@ searches, coordinate by coordinate,
   boundary planes) and, in mixed plans, the float32 z lines of the nonlinear
   term: threads per line, lines per workgroup, and whether the Rader /
   Bluestein tables sit in global memory or LDS;
-* the wall kernel on the matrix cores: kappa blocks per wave and waves per
-  SIMD of its register budget,
+* the wall kernel on the matrix cores: waves per SIMD of its register budget
+  and kappa blocks per wave (0: the library's share, which float64 plans of the
+  same length then keep),
 
 timing each candidate as whole RK steps of a batched solver on the GPU (HIP
 events on the solver's stream) and keeping the fastest.  The choices are
@@ -52,7 +53,7 @@ def apply_tuning(path: str = DEFAULT_PATH) -> int:
     return n
 
 
-def _time_steps(grid, precision, members, nsteps=4, warmup=2, seed=7):
+def _time_steps(grid, precision, members, nsteps=20, warmup=4, seed=7):
     """ms per RK2 step of a batched HD solver of the grid (plans are created
     with the overrides registered at call time)."""
     import torch
@@ -122,7 +123,7 @@ def tune_grid(n: int, d: int, precision: int, members: int, log=print) -> dict:
                     best = ms
                 else:
                     state[cs] = keep
-    for kbw, wpe in ((9, 3), (18, 2), (9, 4)):
+    for kbw, wpe in ((0, 3), (9, 3), (18, 2), (9, 4)):
         keep = list(wall)
         wall[:] = [kbw, wpe]
         register()
