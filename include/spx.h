@@ -75,7 +75,7 @@ typedef struct {
   size_t work_bytes_bouss; /* and on first use of advect (Boussinesq), beyond work_bytes     */
   size_t state_bytes;      /* device memory of one spx_state (all members): HD              */
   size_t state_bytes_bouss;/* ... Boussinesq                                                 */
-  int z_threads_per_line;  /* launch shape of the float64 z line kernels                      */
+  int z_threads_per_line;  /* launch shape of the float64 z transforms                        */
   int z_lines_per_block;
   int z_tables_global;     /* 1: Rader / Bluestein tables read from global memory, 0: LDS    */
   int z_wave_plan;         /* compiled one-wavefront-per-line plan of the z transforms, -1: none */
@@ -103,9 +103,10 @@ int spx_plan_get_info(const spx_plan* p, spx_plan_info* info);
  * lines per workgroup and threads per line (powers of two; 0 = default) and
  * the Rader / Bluestein tables in global memory (1), LDS (0) or default (-1);
  * values the engine cannot run (LDS, 512 threads, fewer threads than the
- * length needs) are ignored.  spx_tune_wall: kappa blocks per wave (9, 18;
- * 0 = default) and waves per SIMD (3, 4) of the wall kernel for lines of
- * length n. */
+ * length needs) are ignored.  Lines that a compiled plan transforms take the
+ * lines per workgroup only: their threads and table places belong to the plan.
+ * spx_tune_wall: kappa blocks per wave (9, 18; 0 = default) and waves per SIMD
+ * (3, 4) of the wall kernel for lines of length n. */
 int spx_tune_line(int n, int csize, int lines, int threads, int tables_global);
 int spx_tune_wall(int n, int blocks_per_wave, int waves_per_simd);
 int spx_tune_clear(void);

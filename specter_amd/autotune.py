@@ -5,8 +5,8 @@ searches, coordinate by coordinate,
 
 * the float64 z lines (state transforms, projection, harmonic correction,
   boundary planes) and, in mixed plans, the float32 z lines of the nonlinear
-  term: threads per line, lines per workgroup, and whether the Rader /
-  Bluestein tables sit in global memory or LDS;
+  term: lines per workgroup and, where no compiled plan transforms them, threads
+  per line and whether the Rader / Bluestein tables sit in global memory or LDS;
 * the wall kernel on the matrix cores: waves per SIMD of its register budget
   and kappa blocks per wave (0: the library's share, which float64 plans of the
   same length then keep),
@@ -55,7 +55,8 @@ def apply_tuning(path: str = DEFAULT_PATH) -> int:
 
 def _time_steps(grid, precision, members, nsteps=20, warmup=4, seed=7):
     """ms per RK2 step of a batched HD solver of the grid (plans are created
-    with the overrides registered at call time)."""
+    with the overrides registered at call time), and the z lines' threads, lines
+    per workgroup, table place and whether a plan is compiled per element size."""
     import torch
     from . import FCPlan, Solver, SolverParams, ic
     nx, ny, nz, C, d = grid
@@ -74,7 +75,8 @@ def _time_steps(grid, precision, members, nsteps=20, warmup=4, seed=7):
     torch.cuda.synchronize()
     ms = e0.elapsed_time(e1) / nsteps
     info = plan.info()
-    shape = (info.z_threads_per_line, info.z_lines_per_block, info.z_tables_global)
+    shape = (info.z_threads_per_line, info.z_lines_per_block, info.z_tables_global,
+             {16: info.z_wave_plan >= 0, 8: info.z_wave_plan_lo >= 0})
     sol.close()
     plan.close()
     return ms, shape
@@ -97,14 +99,16 @@ def tune_grid(n: int, d: int, precision: int, members: int, log=print) -> dict:
         _l.check(lib.spx_tune_wall(nz, wall[0], wall[1]))
 
     register()
-    best, (t0, l0, g0) = _time_steps(grid, precision, members)
+    best, (t0, l0, g0, compiled) = _time_steps(grid, precision, members)
     ms_default = best
     log(f"  {grid} precision {precision} x{members}: default {best:.3f} ms/step "
         f"(z: {t0} threads/line, {l0} lines/block, global tables {g0})")
     csizes = [16, 8] if precision == _l.SPX_FP32_MIXED else [16]
     for cs in csizes:
-        for field, values in ((1, (t0, 2 * t0, 4 * t0)), (0, (l0, max(1, l0 // 2), 2 * l0)),
-                              (2, (0, 1))):
+        sweep = [(0, (l0, max(1, l0 // 2), 2 * l0))]
+        if not compiled[cs]:
+            sweep = [(1, (t0, 2 * t0, 4 * t0))] + sweep + [(2, (0, 1))]
+        for field, values in sweep:
             for v in values:
                 trial = list(state[cs])
                 trial[field] = v

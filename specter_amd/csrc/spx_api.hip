@@ -604,8 +604,10 @@ int spx_plan_get_info(const spx_plan* p, spx_plan_info* info) {
   info->n_real = p->nr;
   info->bytes_spectral = p->nc * 16;
   info->bytes_real = p->nr * 8;
-  info->z_fft_len = p->fz.M;
-  info->z_algorithm = p->fz.mode;
+  // the lines of the z transforms: compiled where there is a plan, else the engine's
+  const spx::LineFFTHost& z = p->fzw.wave >= 0 ? p->fzw : p->fz;
+  info->z_fft_len = z.M;
+  info->z_algorithm = z.mode;
   size_t tab = 0;
   for (const spx::LineFFTHost* f :
        {&p->fx, &p->fy, &p->fz, &p->fx32, &p->fy32, &p->fz32, &p->fzw, &p->fzw32})
@@ -617,9 +619,9 @@ int spx_plan_get_info(const spx_plan* p, spx_plan_info* info) {
   info->work_bytes_bouss = p->work_bouss ? 0 : wb;
   info->state_bytes = state_size(p, false);
   info->state_bytes_bouss = state_size(p, true);
-  info->z_threads_per_line = p->fz.tpl;
-  info->z_lines_per_block = p->fz.nl;
-  info->z_tables_global = (p->fz.mode != 0 && p->fz.tab == p->fz.M) ? 1 : 0;
+  info->z_threads_per_line = z.tpl;
+  info->z_lines_per_block = z.nl;
+  info->z_tables_global = z.mode != 0 && (z.wave >= 0 || z.tab == z.M) ? 1 : 0;
   info->z_wave_plan = p->fzw.wave;
   info->z_wave_plan_lo = p->fp32 ? p->fzw32.wave : -1;
   return SPX_OK;

@@ -371,6 +371,7 @@ int xcross(spx_plan* p, void* const* A, void* const* B, void* const* out);
 // plan builds its line FFTs and wall tables; 0 / -1 fields keep the default.
 struct LineTune {
   int lines = 0;     // lines per workgroup (power of two)
+  // the engine's lines only:
   int threads = 0;   // threads per line (power of two, >= the minimum for n)
   int gtab = -1;     // Rader / Bluestein tables: 1 global memory, 0 LDS
 };

@@ -2179,6 +2179,15 @@ static int set_wave(LineFFTHost& h, int w, int csize) {
   for (h.lgnl = 0; (1 << h.lgnl) < h.nl;) ++h.lgnl;
   h.ldl = i.ldl;
   h.tab = i.tab;  // staged in LDS; filter, chirp and indices in global memory
+  // a tuned line count that fits beside what the kernels stage behind the lines:
+  // float32 boundary planes (two times eight float64 values a line) and a sum per thread
+  LineTune tune;
+  if (get_line_tune(h.n, csize, &tune) && tune.lines > 0 && (tune.lines & (tune.lines - 1)) == 0 &&
+      tune.lines * h.tpl >= 64 && tune.lines * h.tpl <= kMaxBlock) {
+    const LineFFTHost t = h.with_lines(tune.lines);
+    const size_t behind = csize == 8 ? size_t(t.nl) * 16 * 16 + 16 : size_t(t.nl) * t.tpl * 8;
+    if (t.lds_bytes(size_t(csize)) + behind <= 160 * 1024) h = t;
+  }
   if (i.natural) return SPX_OK;  // the engine's own table
   const long double PI2 = 6.283185307179586476925286766559005768L;
   const int M = h.M;

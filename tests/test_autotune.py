@@ -1,8 +1,10 @@
 """The autotuner's search, with the timing replaced by a formula (no GPU)."""
 import json
 
+import pytest
+
 from specter_amd import autotune
-from specter_amd.lib import SPX_FP32_MIXED
+from specter_amd.lib import SPX_FP32_MIXED, SPX_FP64
 
 
 class _Lib:
@@ -27,7 +29,7 @@ class _Lib:
         return 0
 
 
-def _tune(monkeypatch, cost, precision):
+def _tune(monkeypatch, cost, precision, compiled):
     lib, seen = _Lib(), []
 
     def time_steps(grid, prec, members):
@@ -35,7 +37,7 @@ def _tune(monkeypatch, cost, precision):
         line = {cs: lib.line.get((n, cs), (0, 0, -1)) for cs in (16, 8)}
         wall = lib.wall.get(n, (0, 0))
         seen.append((line, wall))
-        return cost(line, wall), (16, 8, 0)
+        return cost(line, wall), (16, 8, 0, compiled)
 
     monkeypatch.setattr(autotune._l, "load_library", lambda: lib)
     monkeypatch.setattr(autotune, "_time_steps", time_steps)
@@ -45,8 +47,22 @@ def _tune(monkeypatch, cost, precision):
 def test_register_budget_leaves_the_blocks_to_the_library(monkeypatch):
     """a mixed class faster with three waves per SIMD must not fix the blocks per wave
     of the float64 plans of the same z length"""
-    r, _ = _tune(monkeypatch, lambda line, wall: 1.0 - 0.05 * (wall[1] == 3), SPX_FP32_MIXED)
+    r, _ = _tune(monkeypatch, lambda line, wall: 1.0 - 0.05 * (wall[1] == 3), SPX_FP32_MIXED,
+                 {16: True, 8: True})
     assert r["wall"] == [{"n": 89, "blocks_per_wave": 0, "waves_per_simd": 3}]
+
+
+@pytest.mark.parametrize("compiled", [True, False])
+def test_compiled_lines_are_swept_over_lines_only(monkeypatch, compiled):
+    """threads and table places belong to a compiled plan: no time is spent on them and
+    no noise in them is kept"""
+    r, seen = _tune(monkeypatch,
+                    lambda line, wall: 1.0 - 0.1 * (line[16][0] == 4) - 0.1 * (line[16][1] == 32),
+                    SPX_FP64, {16: compiled, 8: False})
+    swept = any(line[16][1:] != (0, -1) for line, _ in seen)
+    assert swept != compiled
+    assert r["line"] == [{"n": 89, "csize": 16, "lines": 4, "threads": 0 if compiled else 32,
+                          "tables_global": -1}]
 
 
 def test_shipped_choices_leave_the_blocks_to_the_library():
