@@ -845,7 +845,7 @@ int gradre_impl(spx_plan* p, const void* const v[3], const void* th, void* const
     y2[nf + c] = nullptr;
   }
   if ((rc = yfft(p, 2 * nf, yf, yf, 0, np, y2, lo))) return rc;
-  rc = p->xfused ? xgrad_fused(p, nf, p->XV, p->XY, p->XZ, nullptr, p->XY, lo)
+  rc = p->xfused ? xgrad_fused(p, nf, p->XV, p->XY, p->XZ, p->XY, lo)
                  : SPX_ERR_UNSUPPORTED;
   if (rc == SPX_ERR_UNSUPPORTED) {
     if ((rc = xc2r(p, 3, p->XV, p->RV, np, 0, lo))) return rc;

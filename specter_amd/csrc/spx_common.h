@@ -340,8 +340,8 @@ int zfft_s2x(spx_plan* p, int nf, const void* const* S, void* const* X, int dir,
 // before the FFT (rows ny-Cy.. from the first and last oy physical rows).
 int yfft(spx_plan* p, int nf, const void* const* in, void* const* out, int forward, int nplanes,
          void* const* Y2 = nullptr, bool lo = false, bool cont = false);
-int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
-         bool lo = false);
+// x real -> half complex, float64
+int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes);
 // x half complex -> real of planes < nplanes; dirx = 1 multiplies by i kx first.
 int xc2r(spx_plan* p, int nf, const void* const* X, void* const* R, int nplanes, int dirx = 0,
          bool lo = false);
@@ -352,11 +352,10 @@ int xgrad_prod(spx_plan* p, int nf, const void* const* YV, const void* const* YY
                const void* const* XZ, const void* const* vel, void* const* out, bool lo = false,
                int nplanes = -1);
 // the same on the np planes of three velocity components (and a scalar,
-// nf = 4) with vel = c2r(YV[0..2]) formed in the same launch and stored to RV
-// when given; x lengths whose plan has it (plan flag xfused), SPX_ERR_UNSUPPORTED
-// otherwise
+// nf = 4) with vel = c2r(YV[0..2]) formed in the same launch; x lengths whose plan
+// has it (plan flag xfused), SPX_ERR_UNSUPPORTED otherwise
 int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
-                void* const* RV, void* const* out, bool lo);
+                void* const* out, bool lo);
 // the x stage of a round trip through real space with the division by nx ny nz,
 // in place on the np planes of float64 half spectra
 int xround(spx_plan* p, void* X);

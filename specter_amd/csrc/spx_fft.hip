@@ -571,7 +571,7 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_y(YFields<T
   const bool cont = forward && Cy > 0;
   const int nload = cont ? npy : ny;
   if constexpr (RS >= RS_WAVE) {
-    // compiled plans (tpl 64, ny <= KN*tpl): all of a thread's loads in
+    // compiled plans (ny <= KN*tpl): all of a thread's loads in
     // flight at once instead of one load-wait-store round trip per element
     constexpr int KN = keep_n<RS>();
     Cp v[KN];
@@ -664,9 +664,10 @@ struct XFields {
   void* out[kMaxComp];
 };
 
-template <typename T, int RS>
-__global__ void __launch_bounds__(kMaxBlock) k_xr2c(XFields<T> a, LineFFT<cpx<T>> f, int nkx,
-                                              long npairs) {
+template <int RS>
+__global__ void __launch_bounds__(kMaxBlock) k_xr2c(XFields<double> a, LineFFT<cpx<double>> f,
+                                              int nkx, long npairs) {
+  using T = double;
   using Cp = cpx<T>;
   const T* __restrict__ R = static_cast<const T*>(a.in[blockIdx.y]);
   Cp* __restrict__ X = static_cast<Cp*>(a.out[blockIdx.y]);
@@ -675,9 +676,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_xr2c(XFields<T> a, LineFFT<cpx<T>
   const long p = long(blockIdx.x) * f.nl + line;
   const bool ok = p < npairs;
   const T* r0 = R + long(nx) * (2 * (ok ? p : 0));
-  // float64 rows: batched loads; float32 rows keep the loop (batching them
-  // tripled the register count and halved the occupancy)
-  if constexpr (RS >= RS_WAVE && sizeof(T) == 8) {
+  if constexpr (RS >= RS_WAVE) {  // batched loads
     constexpr int KN = keep_n<RS>();
     T a[KN], b[KN];
 #pragma unroll
@@ -808,12 +807,6 @@ constexpr int batch_n() {
   if constexpr (RS >= RS_WAVE) return keep_n<RS>();
   else return 0;
 }
-// the fused x stage holds the velocity of its row pair in registers, so its
-// loads are batched in chunks
-template <typename T, int RS>
-constexpr int xg_batch() {
-  return batch_n<RS>();
-}
 // x lines of a plan whose fused x stage keeps its row pair's velocity in
 // registers: powers of two of the general engine (its other radix families
 // spill) and the compiled plans of x lines
@@ -832,7 +825,9 @@ constexpr bool xprod_fma() {
   if constexpr (RS >= RS_WAVE) return WavePlanOf<RS>::type::natural;
   else return false;
 }
-template <typename T, int RS>
+// The fused x stage holds the velocity of its row pair in registers, so its loads
+// are batched in chunks.
+template <int RS>
 constexpr int xg_chunk() {
   // four elements in flight at a time: at 512^3 the x stage takes 2.2 ms
   // (float32) / 4.2 ms (float64) per RK stage against 2.9 / 5.5 with one
@@ -974,7 +969,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cp
 
 // gradre's whole x stage on a row pair (pseudospec_hd.f90:254-312): the
 // velocity components u, v, w = c2r(YV_c) are formed first and kept in
-// registers (and stored to rv[c] when given: advect reuses them), then for
+// registers, then for
 // each field c (the three components, and a scalar when nf = 4)
 // ((u Dx v_c + v Dy v_c) + w Dz v_c) tmp from the c2r of i kx YV_c, YY_c and
 // XZ_c, in k_xgrad_prod's operation order, and its r2c.  Neither the real
@@ -982,13 +977,12 @@ __global__ void __launch_bounds__(kMaxBlock) k_xgrad_prod(XProd<T> a, LineFFT<cp
 // the transforms of a row pair synchronise with line_sync.  Launches of fewer
 // than kSpread tiles give each field a workgroup of its own (blockIdx.y), which
 // forms the velocity again: 7 transforms one after the other instead of 15 (HD
-// 32^3 38 -> 20 us, 64^3 45 -> 26 us); rv is then stored by the first.
+// 32^3 38 -> 20 us, 64^3 45 -> 26 us).
 template <typename T>
 struct XGradArgs {
   const cpx<T>* yv[4];
   const cpx<T>* yy[4];
   const cpx<T>* xz[4];
-  T* rv[3];   // may be null
   cpx<T>* out[4];
 };
 
@@ -1003,14 +997,13 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
   const T tmp = T(tmpd);
   const long p = long(blockIdx.x) * f.nl + line;
   const bool ok = p < npairs;
-  const long ro = long(nx) * (2 * (ok ? p : 0));
   const long co = long(nkx) * (2 * (ok ? p : 0));
   constexpr int KX = keep_n<RS>();
   constexpr bool pow2 = xline_pow2<RS>();
   T vel[3][2][KX];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>()>(xl, a.yv[c] + co, nkx, nx, lane, f.tpl, ok, 0, kx);
+    load_c2r_pair<T, batch_n<RS>(), xg_chunk<RS>()>(xl, a.yv[c] + co, nkx, nx, lane, f.tpl, ok, 0, kx);
     // the first barrier also publishes the staged twiddles
     if (c == 0) __syncthreads();
     else line_sync(f.tpl);
@@ -1024,10 +1017,6 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
         const Cp z = xl[x];
         vel[c][0][q] = z.x;
         vel[c][1][q] = -z.y;
-        if (a.rv[c] && ok && blockIdx.y == 0) {
-          a.rv[c][ro + x] = z.x;
-          a.rv[c][ro + x + nx] = -z.y;
-        }
       }
     }
     line_sync(f.tpl);
@@ -1040,10 +1029,10 @@ __global__ void __launch_bounds__(kMaxBlock, sizeof(T) == 4 ? 4 : 2) k_xgrad_fus
     for (int r = 0; r < 3; ++r) {
       // (the scalar's and other lengths' d/dx are k_xgrad_prod's to the bit)
       if (r == 0 && (!pow2 || c == 3))
-        load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>(), false>(
+        load_c2r_pair<T, batch_n<RS>(), xg_chunk<RS>(), false>(
             xl, srcs[r] + co, nkx, nx, lane, f.tpl, ok, 1, kx);
       else
-        load_c2r_pair<T, xg_batch<T, RS>(), xg_chunk<T, RS>()>(xl, srcs[r] + co, nkx, nx, lane,
+        load_c2r_pair<T, batch_n<RS>(), xg_chunk<RS>()>(xl, srcs[r] + co, nkx, nx, lane,
                                                               f.tpl, ok, r == 0 ? 1 : 0, kx);
       line_sync(f.tpl);
       line_fft_nosync<T, RS>(xl, f, tws, lane);
@@ -2396,9 +2385,6 @@ static inline const cpx<T>* C_(const void* p) { return static_cast<const cpx<T>*
 
 // ---- transforms ----
 // lo selects the float32 kernels and tables of a mixed plan.
-static inline const LineFFTHost& fxp(const spx_plan* p, bool lo) { return lo ? p->fx32 : p->fx; }
-static inline const LineFFTHost& fyp(const spx_plan* p, bool lo) { return lo ? p->fy32 : p->fy; }
-static inline const LineFFTHost& fzp(const spx_plan* p, bool lo) { return lo ? p->fz32 : p->fz; }
 // the z-transform plan: the wave variant where one is compiled
 static inline const LineFFTHost& fzt(const spx_plan* p, bool lo) {
   if (lo) return p->fzw32.wave >= 0 ? p->fzw32 : p->fz32;
@@ -2657,41 +2643,25 @@ static XFields<T> x_fields(int nf, const void* const* in, void* const* out) {
   return a;
 }
 
-template <typename T>
-struct XForward {
-  static int run(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes, const
-                 LineFFTHost& f);
-};
-template <typename T>
-int XForward<T>::run(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes,
-                  const LineFFTHost& fp) {
+#if !defined(SPX_PART) || SPX_PART == 10
+int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes) {
+  if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xr2c: bad field count");
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
-  const LineFFTHost f = spread(fp, npairs, nf, 1);
-  dim3 grid(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf));
-  const XFields<T> a = x_fields<T>(nf, R, X);
+  const LineFFTHost f = spread(p->fx, npairs, nf, 1);
+  const XFields<double> a = x_fields<double>(nf, R, X);
   ProfScope ps_(p, "xr2c", double(p->g.ny) * nplanes * p->mem * nf *
-                               (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
-  SPX_LAUNCH(with_x<sizeof(cpx<T>)>, f, k_xr2c, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
-                f.dev<cpx<T>>(), p->nkx, npairs);
+                               (8.0 * p->g.nx + 16.0 * p->nkx));
+  const int rc = with_x<16>(f, [&](auto rs) -> int {
+    constexpr int RS = decltype(rs)::value;
+    const size_t lds = f.lds_bytes(16);
+    if (int lrc = lds_limit(k_xr2c<RS>, lds)) return lrc;
+    hipLaunchKernelGGL(k_xr2c<RS>, dim3(unsigned((npairs + f.nl - 1) / f.nl), unsigned(nf)),
+                       blk(f), lds, p->stream, a, f.dev<Cd>(), p->nkx, npairs);
+    return SPX_OK;
+  });
+  if (rc) return rc;
   SPX_CHECK_LAUNCH();
   return SPX_OK;
-}
-#if !defined(SPX_PART) || SPX_PART == 10
-template struct XForward<double>;
-#else
-extern template struct XForward<double>;
-#endif
-#if !defined(SPX_PART) || SPX_PART == 11
-template struct XForward<float>;
-#else
-extern template struct XForward<float>;
-#endif
-#if !defined(SPX_PART) || SPX_PART == 1
-int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes, bool lo) {
-  if (int rc = check_lo(p, lo)) return rc;
-  if (nf < 1 || nf > kMaxComp) return fail(SPX_ERR_ARG, "xr2c: bad field count");
-  return lo ? XForward<float>::run(p, nf, R, X, nplanes, p->fx32)
-            : XForward<double>::run(p, nf, R, X, nplanes, p->fx);
 }
 #endif
 
@@ -2829,12 +2799,12 @@ extern template struct XGradProd<float>;
 #endif
 template <typename T>
 struct XGradFused {
-  static int run(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ, void*
-                 const* RV, void* const* out, const LineFFTHost& f);
+  static int run(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
+                 void* const* out, const LineFFTHost& f);
 };
 template <typename T>
 int XGradFused<T>::run(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
-                         void* const* RV, void* const* out, const LineFFTHost& fp) {
+                         void* const* out, const LineFFTHost& fp) {
   const int nplanes = p->np;
   const long npairs = long(p->g.ny) * nplanes * p->mem / 2;
   const LineFFTHost f = spread(fp, npairs, 1, 1);
@@ -2846,10 +2816,8 @@ int XGradFused<T>::run(spx_plan* p, int nf, void* const* YV, void* const* YY, vo
     a.yy[c] = c < nf ? C_<T>(static_cast<const void*>(YY[c])) : nullptr;
     a.xz[c] = c < nf ? C_<T>(static_cast<const void*>(XZ[c])) : nullptr;
     a.out[c] = c < nf ? C_<T>(out[c]) : nullptr;
-    if (c < 3) a.rv[c] = RV ? static_cast<T*>(RV[c]) : nullptr;
   }
-  ProfScope ps_(p, "xgrad_fused", rows * (4.0 * nf * sizeof(cpx<T>) * p->nkx +
-                                          (RV ? 3.0 : 0.0) * sizeof(T) * p->g.nx));
+  ProfScope ps_(p, "xgrad_fused", rows * 4.0 * nf * sizeof(cpx<T>) * p->nkx);
   const int rc = with_x<sizeof(cpx<T>)>(f, [&](auto rs) -> int {
     constexpr int RS = decltype(rs)::value;
     if constexpr (xfused_ok<RS>()) {
@@ -2880,11 +2848,11 @@ extern template struct XGradFused<float>;
 #endif
 #if !defined(SPX_PART) || SPX_PART == 1
 int xgrad_fused(spx_plan* p, int nf, void* const* YV, void* const* YY, void* const* XZ,
-                void* const* RV, void* const* out, bool lo) {
+                void* const* out, bool lo) {
   if (int rc = check_lo(p, lo)) return rc;
   if (nf < 3 || nf > 4) return fail(SPX_ERR_ARG, "xgrad_fused: 3 or 4 fields");
-  return lo ? XGradFused<float>::run(p, nf, YV, YY, XZ, RV, out, p->fx32)
-            : XGradFused<double>::run(p, nf, YV, YY, XZ, RV, out, p->fx);
+  return lo ? XGradFused<float>::run(p, nf, YV, YY, XZ, out, p->fx32)
+            : XGradFused<double>::run(p, nf, YV, YY, XZ, out, p->fx);
 }
 #endif
 

@@ -47,22 +47,24 @@ static int scratch_address(int dev, unsigned char** out) {
 
 // the gradre work set carved out of the scratch, each array on a 256-byte
 // boundary: XV, XZ, XY, RV (3 each), and in mixed plans with walls the float64
-// boundary-plane buffers.  The reserve also counts real products of the size
-// of RV and of the boundary planes, which the x stage no longer stores: the
-// limit on the grid stays where callers know it
-// (in the order of the pointer slots of spx_gradre_noalloc); returns the count
+// boundary-plane buffers (in the order of the pointer slots of
+// spx_gradre_noalloc); returns the count.  spare: bytes of the real products that
+// the x stage does not store, still counted: the limit on the grid stays where
+// callers know it
 static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
-static int noalloc_sizes(const spx_plan* p, size_t sz[21]) {
+static int noalloc_sizes(const spx_plan* p, size_t sz[17], size_t* spare) {
   const size_t cb = p->nc * p->nb * p->csize, rb = p->nr * p->nb * p->rsize;
   for (int i = 0; i < 9; ++i) sz[i] = cb;
-  for (int i = 9; i < 15; ++i) sz[i] = rb;
-  if (!(p->fp32 && p->g.Cz > 0)) return 15;
+  for (int i = 9; i < 12; ++i) sz[i] = rb;
+  *spare = 3 * round256(rb);
+  if (!(p->fp32 && p->g.Cz > 0)) return 12;
   const size_t d2 = 2 * size_t(p->g.oz), nbm = size_t(p->nb);
   const size_t bcb = size_t(p->nkx) * p->g.ny * d2 * nbm * 16;
   const size_t brb = size_t(p->g.nx) * p->g.ny * d2 * nbm * 8;
-  const size_t bsz[6] = {4 * bcb, 4 * bcb, 4 * bcb, 3 * brb, 4 * brb, 4 * bcb};
-  for (int i = 0; i < 6; ++i) sz[15 + i] = bsz[i];
-  return 21;
+  const size_t bsz[5] = {4 * bcb, 4 * bcb, 4 * bcb, 3 * brb, 4 * bcb};
+  for (int i = 0; i < 5; ++i) sz[12 + i] = bsz[i];
+  *spare += round256(4 * brb);
+  return 17;
 }
 
 }  // namespace
@@ -71,9 +73,8 @@ extern "C" {
 
 int spx_gradre_scratch_bytes(const spx_plan* p, size_t* need, size_t* limit) {
   SPX_REQ(p && need && limit, "spx_gradre_scratch_bytes: null argument");
-  size_t sz[21];
-  const int nset = noalloc_sizes(p, sz);
-  size_t n = 0;
+  size_t sz[17], n = 0;
+  const int nset = noalloc_sizes(p, sz, &n);
   for (int i = 0; i < nset; ++i) n += round256(sz[i]);
   *need = n;
   *limit = kScratchBytes;
@@ -100,15 +101,13 @@ int spx_gradre_noalloc(spx_plan* p, const void* a, const void* b, const void* c,
   // carve the work set out of the scratch (every array is written before it
   // is read, as with the allocated set, so nothing is cleared); the plan's
   // own work pointers are swapped for the call and restored after it
-  void* unused = nullptr;
-  void** slots[21] = {&p->XV[0], &p->XV[1], &p->XV[2], &p->XZ[0], &p->XZ[1], &p->XZ[2],
+  void** slots[17] = {&p->XV[0], &p->XV[1], &p->XV[2], &p->XZ[0], &p->XZ[1], &p->XZ[2],
                       &p->XY[0], &p->XY[1], &p->XY[2], &p->RV[0], &p->RV[1], &p->RV[2],
-                      &unused,   &unused,   &unused,   &p->XVb, &p->XZb, &p->XYb,
-                      &p->RVb,   &unused,   &p->XFb};
-  void* sv[21];
-  for (int i = 0; i < 21; ++i) sv[i] = *slots[i];
-  size_t sz[21];
-  const int nset = noalloc_sizes(p, sz);
+                      &p->XVb,   &p->XZb,   &p->XYb,   &p->RVb,   &p->XFb};
+  void* sv[17];
+  for (int i = 0; i < 17; ++i) sv[i] = *slots[i];
+  size_t sz[17], spare;
+  const int nset = noalloc_sizes(p, sz, &spare);
   size_t off = 0;
   for (int i = 0; i < nset; ++i) {
     *slots[i] = base + off;
@@ -120,7 +119,7 @@ int spx_gradre_noalloc(spx_plan* p, const void* a, const void* b, const void* c,
     void* o[3] = {d, e, f};
     rc = gradre_impl(p, v, nullptr, o);
   }
-  for (int i = 0; i < 21; ++i) *slots[i] = sv[i];
+  for (int i = 0; i < 17; ++i) *slots[i] = sv[i];
   return rc;
 }
 

@@ -151,172 +151,6 @@ struct RootTab<20> {
       -1.000000000000000000000000, -0.951056516295153572116439, -0.809016994374947424102293,
       -0.587785252292473129168706, -0.309016994374947424102293};
 };
-template <>
-struct RootTab<24> {
-  static constexpr double c[24] = {
-      1.000000000000000000000000, 0.965925826289068286749743, 0.866025403784438646763723,
-      0.707106781186547524400844, 0.500000000000000000000000, 0.258819045102520762348899,
-      0.0, -0.258819045102520762348899, -0.500000000000000000000000,
-      -0.707106781186547524400844, -0.866025403784438646763723, -0.965925826289068286749743,
-      -1.000000000000000000000000, -0.965925826289068286749743, -0.866025403784438646763723,
-      -0.707106781186547524400844, -0.500000000000000000000000, -0.258819045102520762348899,
-      0.0, 0.258819045102520762348899, 0.500000000000000000000000,
-      0.707106781186547524400844, 0.866025403784438646763723, 0.965925826289068286749743};
-  static constexpr double s[24] = {
-      0.0, 0.258819045102520762348899, 0.500000000000000000000000,
-      0.707106781186547524400844, 0.866025403784438646763723, 0.965925826289068286749743,
-      1.000000000000000000000000, 0.965925826289068286749743, 0.866025403784438646763723,
-      0.707106781186547524400844, 0.500000000000000000000000, 0.258819045102520762348899,
-      0.0, -0.258819045102520762348899, -0.500000000000000000000000,
-      -0.707106781186547524400844, -0.866025403784438646763723, -0.965925826289068286749743,
-      -1.000000000000000000000000, -0.965925826289068286749743, -0.866025403784438646763723,
-      -0.707106781186547524400844, -0.500000000000000000000000, -0.258819045102520762348899};
-};
-template <>
-struct RootTab<27> {
-  static constexpr double c[27] = {
-      1.000000000000000000000000, 0.973044870579823838832885, 0.893632640323412248192574,
-      0.766044443118978035202393, 0.597158591702786164851852, 0.396079766039156823696043,
-      0.173648177666930348851717, -0.058144828910475828538748, -0.286803232711090253103280,
-      -0.500000000000000000000000, -0.686241637868733585729605, -0.835487811412936419653826,
-      -0.939692620785908384054109, -0.993238357741942988547896, -0.993238357741942988547896,
-      -0.939692620785908384054109, -0.835487811412936419653826, -0.686241637868733585729605,
-      -0.500000000000000000000000, -0.286803232711090253103280, -0.058144828910475828538748,
-      0.173648177666930348851717, 0.396079766039156823696043, 0.597158591702786164851852,
-      0.766044443118978035202393, 0.893632640323412248192574, 0.973044870579823838832885};
-  static constexpr double s[27] = {
-      0.0, 0.230615870742440178450198, 0.448799180200462172785040,
-      0.642787609686539326322643, 0.802123192755043785083295, 0.918216106880274014758961,
-      0.984807753012208059366743, 0.998308158271268208047821, 0.957989512315488874437375,
-      0.866025403784438646763723, 0.727373641573048695987176, 0.549508978070806035262780,
-      0.342020143325668733044100, 0.116092914125230229675667, -0.116092914125230229675667,
-      -0.342020143325668733044100, -0.549508978070806035262780, -0.727373641573048695987176,
-      -0.866025403784438646763723, -0.957989512315488874437375, -0.998308158271268208047821,
-      -0.984807753012208059366743, -0.918216106880274014758961, -0.802123192755043785083295,
-      -0.642787609686539326322643, -0.448799180200462172785040, -0.230615870742440178450198};
-};
-template <>
-struct RootTab<30> {
-  static constexpr double c[30] = {
-      1.000000000000000000000000, 0.978147600733805637928567, 0.913545457642600895502128,
-      0.809016994374947424102293, 0.669130606358858213826273, 0.500000000000000000000000,
-      0.309016994374947424102293, 0.104528463267653471399834, -0.104528463267653471399834,
-      -0.309016994374947424102293, -0.500000000000000000000000, -0.669130606358858213826273,
-      -0.809016994374947424102293, -0.913545457642600895502128, -0.978147600733805637928567,
-      -1.000000000000000000000000, -0.978147600733805637928567, -0.913545457642600895502128,
-      -0.809016994374947424102293, -0.669130606358858213826273, -0.500000000000000000000000,
-      -0.309016994374947424102293, -0.104528463267653471399834, 0.104528463267653471399834,
-      0.309016994374947424102293, 0.500000000000000000000000, 0.669130606358858213826273,
-      0.809016994374947424102293, 0.913545457642600895502128, 0.978147600733805637928567};
-  static constexpr double s[30] = {
-      0.0, 0.207911690817759337101742, 0.406736643075800207753986,
-      0.587785252292473129168706, 0.743144825477394235014697, 0.866025403784438646763723,
-      0.951056516295153572116439, 0.994521895368273336922692, 0.994521895368273336922692,
-      0.951056516295153572116439, 0.866025403784438646763723, 0.743144825477394235014697,
-      0.587785252292473129168706, 0.406736643075800207753986, 0.207911690817759337101742,
-      0.0, -0.207911690817759337101742, -0.406736643075800207753986,
-      -0.587785252292473129168706, -0.743144825477394235014697, -0.866025403784438646763723,
-      -0.951056516295153572116439, -0.994521895368273336922692, -0.994521895368273336922692,
-      -0.951056516295153572116439, -0.866025403784438646763723, -0.743144825477394235014697,
-      -0.587785252292473129168706, -0.406736643075800207753986, -0.207911690817759337101742};
-};
-template <>
-struct RootTab<36> {
-  static constexpr double c[36] = {
-      1.000000000000000000000000, 0.984807753012208059366743, 0.939692620785908384054109,
-      0.866025403784438646763723, 0.766044443118978035202393, 0.642787609686539326322643,
-      0.500000000000000000000000, 0.342020143325668733044100, 0.173648177666930348851717,
-      0.0, -0.173648177666930348851717, -0.342020143325668733044100,
-      -0.500000000000000000000000, -0.642787609686539326322643, -0.766044443118978035202393,
-      -0.866025403784438646763723, -0.939692620785908384054109, -0.984807753012208059366743,
-      -1.000000000000000000000000, -0.984807753012208059366743, -0.939692620785908384054109,
-      -0.866025403784438646763723, -0.766044443118978035202393, -0.642787609686539326322643,
-      -0.500000000000000000000000, -0.342020143325668733044100, -0.173648177666930348851717,
-      0.0, 0.173648177666930348851717, 0.342020143325668733044100,
-      0.500000000000000000000000, 0.642787609686539326322643, 0.766044443118978035202393,
-      0.866025403784438646763723, 0.939692620785908384054109, 0.984807753012208059366743};
-  static constexpr double s[36] = {
-      0.0, 0.173648177666930348851717, 0.342020143325668733044100,
-      0.500000000000000000000000, 0.642787609686539326322643, 0.766044443118978035202393,
-      0.866025403784438646763723, 0.939692620785908384054109, 0.984807753012208059366743,
-      1.000000000000000000000000, 0.984807753012208059366743, 0.939692620785908384054109,
-      0.866025403784438646763723, 0.766044443118978035202393, 0.642787609686539326322643,
-      0.500000000000000000000000, 0.342020143325668733044100, 0.173648177666930348851717,
-      0.0, -0.173648177666930348851717, -0.342020143325668733044100,
-      -0.500000000000000000000000, -0.642787609686539326322643, -0.766044443118978035202393,
-      -0.866025403784438646763723, -0.939692620785908384054109, -0.984807753012208059366743,
-      -1.000000000000000000000000, -0.984807753012208059366743, -0.939692620785908384054109,
-      -0.866025403784438646763723, -0.766044443118978035202393, -0.642787609686539326322643,
-      -0.500000000000000000000000, -0.342020143325668733044100, -0.173648177666930348851717};
-};
-template <>
-struct RootTab<40> {
-  static constexpr double c[40] = {
-      1.000000000000000000000000, 0.987688340595137726190040, 0.951056516295153572116439,
-      0.891006524188367862359710, 0.809016994374947424102293, 0.707106781186547524400844,
-      0.587785252292473129168706, 0.453990499739546791560408, 0.309016994374947424102293,
-      0.156434465040230869010105, 0.0, -0.156434465040230869010105,
-      -0.309016994374947424102293, -0.453990499739546791560408, -0.587785252292473129168706,
-      -0.707106781186547524400844, -0.809016994374947424102293, -0.891006524188367862359710,
-      -0.951056516295153572116439, -0.987688340595137726190040, -1.000000000000000000000000,
-      -0.987688340595137726190040, -0.951056516295153572116439, -0.891006524188367862359710,
-      -0.809016994374947424102293, -0.707106781186547524400844, -0.587785252292473129168706,
-      -0.453990499739546791560408, -0.309016994374947424102293, -0.156434465040230869010105,
-      0.0, 0.156434465040230869010105, 0.309016994374947424102293,
-      0.453990499739546791560408, 0.587785252292473129168706, 0.707106781186547524400844,
-      0.809016994374947424102293, 0.891006524188367862359710, 0.951056516295153572116439,
-      0.987688340595137726190040};
-  static constexpr double s[40] = {
-      0.0, 0.156434465040230869010105, 0.309016994374947424102293,
-      0.453990499739546791560408, 0.587785252292473129168706, 0.707106781186547524400844,
-      0.809016994374947424102293, 0.891006524188367862359710, 0.951056516295153572116439,
-      0.987688340595137726190040, 1.000000000000000000000000, 0.987688340595137726190040,
-      0.951056516295153572116439, 0.891006524188367862359710, 0.809016994374947424102293,
-      0.707106781186547524400844, 0.587785252292473129168706, 0.453990499739546791560408,
-      0.309016994374947424102293, 0.156434465040230869010105, 0.0,
-      -0.156434465040230869010105, -0.309016994374947424102293, -0.453990499739546791560408,
-      -0.587785252292473129168706, -0.707106781186547524400844, -0.809016994374947424102293,
-      -0.891006524188367862359710, -0.951056516295153572116439, -0.987688340595137726190040,
-      -1.000000000000000000000000, -0.987688340595137726190040, -0.951056516295153572116439,
-      -0.891006524188367862359710, -0.809016994374947424102293, -0.707106781186547524400844,
-      -0.587785252292473129168706, -0.453990499739546791560408, -0.309016994374947424102293,
-      -0.156434465040230869010105};
-};
-template <>
-struct RootTab<45> {
-  static constexpr double c[45] = {
-      1.000000000000000000000000, 0.990268068741570315083775, 0.961261695938318861916497,
-      0.913545457642600895502128, 0.848048096156425970386176, 0.766044443118978035202393,
-      0.669130606358858213826273, 0.559192903470746830160428, 0.438371146789077417452735,
-      0.309016994374947424102293, 0.173648177666930348851717, 0.034899496702500971645995,
-      -0.104528463267653471399834, -0.241921895599667722560442, -0.374606593415912035414964,
-      -0.500000000000000000000000, -0.615661475325658279668811, -0.719339800338651139356055,
-      -0.809016994374947424102293, -0.882947592858926942032171, -0.939692620785908384054109,
-      -0.978147600733805637928567, -0.997564050259824247613163, -0.997564050259824247613163,
-      -0.978147600733805637928567, -0.939692620785908384054109, -0.882947592858926942032171,
-      -0.809016994374947424102293, -0.719339800338651139356055, -0.615661475325658279668811,
-      -0.500000000000000000000000, -0.374606593415912035414964, -0.241921895599667722560442,
-      -0.104528463267653471399834, 0.034899496702500971645995, 0.173648177666930348851717,
-      0.309016994374947424102293, 0.438371146789077417452735, 0.559192903470746830160428,
-      0.669130606358858213826273, 0.766044443118978035202393, 0.848048096156425970386176,
-      0.913545457642600895502128, 0.961261695938318861916497, 0.990268068741570315083775};
-  static constexpr double s[45] = {
-      0.0, 0.139173100960065444112497, 0.275637355816999185649972,
-      0.406736643075800207753986, 0.529919264233204954046781, 0.642787609686539326322643,
-      0.743144825477394235014697, 0.829037572555041692006337, 0.898794046299166992782296,
-      0.951056516295153572116439, 0.984807753012208059366743, 0.999390827019095730006243,
-      0.994521895368273336922692, 0.970295726275996472306378, 0.927183854566787400806474,
-      0.866025403784438646763723, 0.788010753606721956693978, 0.694658370458997286656406,
-      0.587785252292473129168706, 0.469471562785890775959462, 0.342020143325668733044100,
-      0.207911690817759337101742, 0.069756473744125300775959, -0.069756473744125300775959,
-      -0.207911690817759337101742, -0.342020143325668733044100, -0.469471562785890775959462,
-      -0.587785252292473129168706, -0.694658370458997286656406, -0.788010753606721956693978,
-      -0.866025403784438646763723, -0.927183854566787400806474, -0.970295726275996472306378,
-      -0.994521895368273336922692, -0.999390827019095730006243, -0.984807753012208059366743,
-      -0.951056516295153572116439, -0.898794046299166992782296, -0.829037572555041692006337,
-      -0.743144825477394235014697, -0.642787609686539326322643, -0.529919264233204954046781,
-      -0.406736643075800207753986, -0.275637355816999185649972, -0.139173100960065444112497};
-};
 
 // v * exp(-2 pi i k / R); k is a constant after unrolling, so the table
 // entries become immediates.  Exact for multiples of pi/2.
@@ -386,18 +220,6 @@ template <typename T>
 struct WDft<T, 18> : DftPQ<T, 2, 9> {};
 template <typename T>
 struct WDft<T, 20> : DftPQ<T, 4, 5> {};
-template <typename T>
-struct WDft<T, 24> : DftPQ<T, 8, 3> {};
-template <typename T>
-struct WDft<T, 27> : DftPQ<T, 3, 9> {};
-template <typename T>
-struct WDft<T, 30> : DftPQ<T, 2, 15> {};
-template <typename T>
-struct WDft<T, 36> : DftPQ<T, 4, 9> {};
-template <typename T>
-struct WDft<T, 40> : DftPQ<T, 8, 5> {};
-template <typename T>
-struct WDft<T, 45> : DftPQ<T, 5, 9> {};
 
 constexpr int ceil_sqrt(int r) {
   int q = 1;
@@ -412,8 +234,7 @@ constexpr int ceil_sqrt(int r) {
 // M-entry table of W_M at r jm M/(Ns R) met on few LDS banks (the dual y pass of
 // 256-point lines 307 us instead of 248, of 512-point lines 2.57 ms instead of
 // 2.25).  TWM 0: every factor read from the table.  TWM 2: those of r = a < q
-// and r = q b, q = ceil(sqrt(R)), are read and the others formed as products
-// (TWM 1: the powers of r = 1 and q too).  Direct lines are bound by memory
+// and r = q b, q = ceil(sqrt(R)), are read and the others formed as products.  Direct lines are bound by memory
 // either way and take TWM 0, the engine's accuracy; Bluestein lines, whose
 // error the chirp convolution sets, are 4-14 % faster with fewer reads.
 template <typename T, int R, int TWM, int Ns>
@@ -422,21 +243,6 @@ __device__ __forceinline__ void stage_twiddle(cpx<T>* v, const cpx<T>* tw, int j
   if constexpr (TWM == 0 || R <= 4) {
 #pragma unroll
     for (int r = 1; r < R; ++r) v[r] = cmul(v[r], t[r * Ns]);
-  } else if constexpr (TWM == 1) {
-    constexpr int q = ceil_sqrt(R);
-    cpx<T> w[R];
-    w[1] = t[Ns];
-    if constexpr (q < R) w[q] = t[q * Ns];
-#pragma unroll
-    for (int r = 2; r < R; ++r) {
-      if (r == q) continue;
-      const int a = r % q, b = r / q;
-      if (b == 0) w[r] = cmul(w[r - 1], w[1]);
-      else if (a == 0) w[r] = cmul(w[r - q], w[q]);
-      else w[r] = cmul(w[b * q], w[a]);
-    }
-#pragma unroll
-    for (int r = 1; r < R; ++r) v[r] = cmul(v[r], w[r]);
   } else {
     constexpr int q = ceil_sqrt(R), nb = (R + q - 1) / q;
     cpx<T> wa[q], wb[nb];
