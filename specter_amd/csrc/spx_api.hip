@@ -517,8 +517,7 @@ static int plan_create(const spx_grid* g, const double* A, const double* Q, int 
   // y lines (stride nkx in memory): up to 512 threads per workgroup, so a row
   // of a workgroup's load spans 8 consecutive kx at ny = 512
   if ((rc = build_line_fft(p->fy, ny, 16, 16, 512, 80 * 1024))) return bail(rc);
-  if ((rc = attach_xy_wave(p->fx, 16, true)) || (rc = attach_xy_wave(p->fy, 16, false)))
-    return bail(rc);
+  if ((rc = attach_xy_wave(p->fx, 16)) || (rc = attach_xy_wave(p->fy, 16))) return bail(rc);
   if ((rc = build_line_fft(p->fz, nz, 16, 16))) return bail(rc);
   p->fz2 = p->fz.with_lines(p->fz.nl / 2);
   if ((rc = build_wave_fft(p->fzw, nz, 16, p->fp32))) return bail(rc);
@@ -543,8 +542,7 @@ static int plan_create(const spx_grid* g, const double* A, const double* Q, int 
   if (p->fp32) {
     if ((rc = build_line_fft(p->fx32, nx, 8, 0))) return bail(rc);
     if ((rc = build_line_fft(p->fy32, ny, 8, 16, 512, 80 * 1024))) return bail(rc);
-    if ((rc = attach_xy_wave(p->fx32, 8, true)) || (rc = attach_xy_wave(p->fy32, 8, false)))
-      return bail(rc);
+    if ((rc = attach_xy_wave(p->fx32, 8)) || (rc = attach_xy_wave(p->fy32, 8))) return bail(rc);
     if ((rc = build_line_fft(p->fz32, nz, 8, 16))) return bail(rc);
     if ((rc = build_wave_fft(p->fzw32, nz, 8, true))) return bail(rc);
     if (C > 0) {

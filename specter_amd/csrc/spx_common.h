@@ -309,8 +309,8 @@ int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_blo
 // the compiled plan of z lines of length n (f.wave < 0 if there is none);
 // same_bits: only those that give the engine's results to the bit
 int build_wave_fft(LineFFTHost& f, int n, int csize, bool same_bits);
-// run an x (or y) line plan by the compiled plan of its length, where there is one
-int attach_xy_wave(LineFFTHost& f, int csize, bool x);
+// run an x / y line plan by the compiled plan of its length, where there is one
+int attach_xy_wave(LineFFTHost& f, int csize);
 void free_line_fft(LineFFTHost& f);
 
 // z transforms in place on S (contiguous lines).

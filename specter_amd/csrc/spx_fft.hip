@@ -2138,7 +2138,7 @@ int build_line_fft(LineFFTHost& f, int n, int csize, int want_lines, int max_blo
 struct WaveInfo {
   int n, m, lanes, mode, nmax, ldl, tab, twm, lines16, lines8, npass;
   const int* radix;
-  bool natural, x, y;
+  bool natural, xy;
   int lines(int csize) const { return csize == 16 ? lines16 : lines8; }
 };
 template <int W = 0>
@@ -2146,7 +2146,7 @@ static void wave_infos(WaveInfo* o) {
   using P = typename WavePlanN<W>::type;
   o[W] = WaveInfo{P::n,   P::m,   P::lanes,          P::mode,          P::nmax,  P::ldl,
                   P::tab, P::twm, wave_lines<W>(16), wave_lines<W>(8), P::npass, P::radix,
-                  P::natural, P::x, P::y};
+                  P::natural, P::xy};
   if constexpr (W + 1 < kWavePlans) wave_infos<W + 1>(o);
 }
 static const WaveInfo* wave_info() {
@@ -2253,14 +2253,14 @@ int build_wave_fft(LineFFTHost& f, int n, int csize, bool same_bits) {
   return SPX_OK;
 }
 
-int attach_xy_wave(LineFFTHost& f, int csize, bool x) {
+int attach_xy_wave(LineFFTHost& f, int csize) {
   for (const char* v : {"SPX_WAVE", "SPX_WAVE_XY"})
     if (const char* e = std::getenv(v))
       if (e[0] == '0') return SPX_OK;
   if (f.mode != 0) return SPX_OK;
   for (int q = 0; q < kWavePlans; ++q) {
     const WaveInfo& i = wave_info()[q];
-    if (!(x ? i.x : i.y) || i.m != f.n || !i.lines(csize)) continue;
+    if (!i.xy || i.m != f.n || !i.lines(csize)) continue;
     if (!i.natural) return set_wave(f, q, csize);
     if (f.n == 512 && f.tpl == 64) f.wave = q;  // the engine's launch shape
     return SPX_OK;
@@ -2318,40 +2318,30 @@ static int with_general(const LineFFTHost& f, F&& fn) {
   }
 }
 // the same for any plan, compiled ones included, with csize-byte elements
-enum { AX_X, AX_Y, AX_Z };
-template <int AX, int W>
-constexpr bool wave_on_axis() {
-  using P = typename WavePlanN<W>::type;
-  return AX == AX_Z || (AX == AX_X ? P::x : P::y);
-}
-template <int CS, int AX, int W = 0, int END = kWavePlans, typename F>
+template <int CS, bool XY, int W = 0, int END = kWavePlans, typename F>
 static int with_wave(int w, F&& fn) {
   if constexpr (W < END) {
-    if constexpr (wave_lines<W>(CS) > 0 && wave_on_axis<AX, W>()) {
+    if constexpr (wave_lines<W>(CS) > 0 && (!XY || WavePlanN<W>::type::xy)) {
       if (w == W) return fn(std::integral_constant<int, RS_WAVE + W>{});
     }
-    return with_wave<CS, AX, W + 1, END>(w, fn);
+    return with_wave<CS, XY, W + 1, END>(w, fn);
   } else {
     return fail(SPX_ERR_STATE, "line plan without a compiled kernel family");
   }
 }
 template <int CS, typename F>
 static int with_z(const LineFFTHost& f, F&& fn) {
-  return f.wave >= 0 ? with_wave<CS, AX_Z>(f.wave, fn) : with_general(f, fn);
+  return f.wave >= 0 ? with_wave<CS, false>(f.wave, fn) : with_general(f, fn);
 }
 constexpr int kInplacePlans = 2;  // 1080 and 539
 template <typename F>
 [[maybe_unused]] static int with_inplace(const LineFFTHost& f, F&& fn) {
-  return f.wave >= 0 ? with_wave<16, AX_Z, 0, kInplacePlans>(f.wave, fn) : with_general(f, fn);
+  return f.wave >= 0 ? with_wave<16, false, 0, kInplacePlans>(f.wave, fn) : with_general(f, fn);
 }
-// x lines and y lines: compiled plans of direct lengths
+// x / y lines: compiled plans of direct lengths
 template <int CS, typename F>
-static int with_x(const LineFFTHost& f, F&& fn) {
-  return f.wave >= 0 ? with_wave<CS, AX_X>(f.wave, fn) : with_general(f, fn);
-}
-template <int CS, typename F>
-static int with_y(const LineFFTHost& f, F&& fn) {
-  return f.wave >= 0 ? with_wave<CS, AX_Y>(f.wave, fn) : with_general(f, fn);
+static int with_xy(const LineFFTHost& f, F&& fn) {
+  return f.wave >= 0 ? with_wave<CS, true>(f.wave, fn) : with_general(f, fn);
 }
 // f with fewer lines per workgroup where a launch of that many lines and
 // fields would leave CUs idle: down to one wave, and to rows of 64 bytes where a
@@ -2598,12 +2588,12 @@ int YPass<T>::run(spx_plan* p, int nf, const void* const* in, void* const* out, 
   if (nd > 0) {
     if (forward) return fail(SPX_ERR_ARG, "dual y transform is backward only");
     ProfScope ps_(p, "y_dual", io * (2.0 * nf + nd));
-    SPX_LAUNCH(with_y<sizeof(cpx<T>)>, f, k_y, T, SPX_COMMA true, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
+    SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_y, T, SPX_COMMA true, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
                   p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, nlines, forward, p->d_ky,
                   p->npy, 0, 0, static_cast<const double*>(nullptr));
   } else {
     ProfScope ps_(p, "y", io * 2.0 * nf);
-    SPX_LAUNCH(with_y<sizeof(cpx<T>)>, f, k_y, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
+    SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_y, T, SPX_COMMA false, grid, blk(f), f.lds_bytes(sizeof(cpx<T>)),
                   p->stream, a, f.dev<cpx<T>>(), p->nkx, p->g.ny, nlines, forward, p->d_ky,
                   p->npy, cont ? p->Cy : 0, p->oy, p->d_diry);
   }
@@ -2651,7 +2641,7 @@ int xr2c(spx_plan* p, int nf, const void* const* R, void* const* X, int nplanes)
   const XFields<double> a = x_fields<double>(nf, R, X);
   ProfScope ps_(p, "xr2c", double(p->g.ny) * nplanes * p->mem * nf *
                                (8.0 * p->g.nx + 16.0 * p->nkx));
-  const int rc = with_x<16>(f, [&](auto rs) -> int {
+  const int rc = with_xy<16>(f, [&](auto rs) -> int {
     constexpr int RS = decltype(rs)::value;
     const size_t lds = f.lds_bytes(16);
     if (int lrc = lds_limit(k_xr2c<RS>, lds)) return lrc;
@@ -2679,7 +2669,7 @@ int XBackward<T>::run(spx_plan* p, int nf, const void* const* X, void* const* R,
   const XFields<T> a = x_fields<T>(nf, X, R);
   ProfScope ps_(p, "xc2r", double(p->g.ny) * nplanes * p->mem * nf *
                                (double(sizeof(T)) * p->g.nx + double(sizeof(cpx<T>)) * p->nkx));
-  SPX_LAUNCH(with_x<sizeof(cpx<T>)>, f, k_xc2r, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+  SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_xc2r, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
                 f.dev<cpx<T>>(), p->nkx, npairs, dirx, p->d_kx);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
@@ -2709,7 +2699,7 @@ int xround(spx_plan* p, void* X) {
   const long npairs = long(p->g.ny) * p->np * p->mem / 2;
   const LineFFTHost f = spread(p->fx, npairs, 1, 1);
   ProfScope ps_(p, "xround", 4.0 * npairs * sizeof(Cd) * p->nkx);
-  const int rc = with_x<16>(f, [&](auto rs) -> int {
+  const int rc = with_xy<16>(f, [&](auto rs) -> int {
     constexpr int RS = decltype(rs)::value;
     const size_t lds = f.lds_bytes(16);
     if (int lrc = lds_limit(k_xround<RS>, lds)) return lrc;
@@ -2725,7 +2715,7 @@ int xround(spx_plan* p, void* X) {
 
 bool xcross_fused(const spx_plan* p) {
   if (p->fp32 || !p->XV[0] || p->fx.wave < 0) return false;
-  return with_x<16>(p->fx, [](auto rs) -> int { return xcross_ok<decltype(rs)::value>(); }) == 1;
+  return with_xy<16>(p->fx, [](auto rs) -> int { return xcross_ok<decltype(rs)::value>(); }) == 1;
 }
 
 int xcross(spx_plan* p, void* const* A, void* const* B, void* const* out) {
@@ -2739,7 +2729,7 @@ int xcross(spx_plan* p, void* const* A, void* const* B, void* const* out) {
     a.out[c] = C_<double>(out[c]);
   }
   ProfScope ps_(p, "xcross", 18.0 * npairs * sizeof(Cd) * p->nkx);
-  const int rc = with_x<16>(f, [&](auto rs) -> int {
+  const int rc = with_xy<16>(f, [&](auto rs) -> int {
     constexpr int RS = decltype(rs)::value;
     if constexpr (xcross_ok<RS>()) {
       const size_t lds = f.lds_bytes(16);
@@ -2782,7 +2772,7 @@ int XGradProd<T>::run(spx_plan* p, int nf, const void* const* YV, const void* co
   for (int c = 0; c < 3; ++c) a.vel[c] = static_cast<const T*>(vel[c]);
   ProfScope ps_(p, "xgrad_prod", rows * (4.0 * sizeof(cpx<T>) * p->nkx +
                                          3.0 * sizeof(T) * p->g.nx));
-  SPX_LAUNCH(with_x<sizeof(cpx<T>)>, f, k_xgrad_prod, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
+  SPX_LAUNCH(with_xy<sizeof(cpx<T>)>, f, k_xgrad_prod, T, , grid, blk(f), f.lds_bytes(sizeof(cpx<T>)), p->stream, a,
                 f.dev<cpx<T>>(), p->nkx, npairs, 1.0 / (t * t), p->d_kx);
   SPX_CHECK_LAUNCH();
   return SPX_OK;
@@ -2818,7 +2808,7 @@ int XGradFused<T>::run(spx_plan* p, int nf, void* const* YV, void* const* YY, vo
     a.out[c] = c < nf ? C_<T>(out[c]) : nullptr;
   }
   ProfScope ps_(p, "xgrad_fused", rows * 4.0 * nf * sizeof(cpx<T>) * p->nkx);
-  const int rc = with_x<sizeof(cpx<T>)>(f, [&](auto rs) -> int {
+  const int rc = with_xy<sizeof(cpx<T>)>(f, [&](auto rs) -> int {
     constexpr int RS = decltype(rs)::value;
     if constexpr (xfused_ok<RS>()) {
       const size_t lds = f.lds_bytes(sizeof(cpx<T>));

@@ -402,12 +402,14 @@ template <int M, int L, int MODE, int TWM, int PAD, int... Rs>
 struct WavePlan {
   static constexpr int n = 0, m = M, mode = MODE, lanes = L, twm = TWM;  // n: any
   static constexpr bool natural = false;
-  static constexpr bool y = MODE == 0 && M % 2 == 0;  // compiled for y lines too
-  // and for x lines, whose fused stages hold a row pair's fields in registers: on
-  // 64 lanes 1024 points (16 a lane) spill 291 registers in float32 and more than the
-  // float64 stage can hold, so they stay on the engine's 128 threads (gradre of
-  // 1024 x 1024 x 64: 6.93 / 6.92 ms mixed / float64 there, 9.14 / 11.67 here)
-  static constexpr bool x = y && (M + L - 1) / L <= 10;
+  // compiled for x and y lines too, up to 10 points a lane.  1024 points on 64 lanes (16
+  // a lane) are slower than the engine's 128 threads: its fused x stage spills 291
+  // registers in float32 and does not fit in float64 (gradre of 1024 x 1024 x 64: 6.93 /
+  // 6.92 ms mixed / float64 on the engine, 9.14 / 11.67 here), and its 8 or 4 lines of
+  // a y workgroup leave one workgroup on a CU (dual y pass of 1024 x 1024 x 100: 2.37 /
+  // 4.97 against 2.96 / 6.19 ms).  In z it gains (128 x 128 x 1024, float64 step: 7.50 ->
+  // 6.50 ms).
+  static constexpr bool xy = MODE == 0 && M % 2 == 0 && (M + L - 1) / L <= 10;
   static constexpr int nmax = MODE == 1 ? (M + 1) / 2 : (MODE == 2 ? M + 1 : M);
   static constexpr int ldl = M + (PAD ? M / RadixProduct<Rs...>::first : 0) + 1;
   static_assert(RadixProduct<Rs...>::value == M, "radices do not multiply to M");
@@ -555,7 +557,7 @@ template <int N, int M, int MODE, int TWM, int... Rs>
 struct FixedPlan {
   static constexpr int n = N, m = M, mode = MODE, lanes = 64, nmax = N, twm = TWM;
   static constexpr int ldl = M + 1, tab = M, npass = 0;
-  static constexpr bool natural = true, y = MODE == 0 && M % 2 == 0, x = y;
+  static constexpr bool natural = true, xy = MODE == 0 && M % 2 == 0;
   static constexpr const int* radix = nullptr;
   static constexpr int lines(int csize) {
     return (size_t(M) + 8 * (size_t(M) + 1)) * csize <= 160 * 1024 ? 8 : 0;
