@@ -566,7 +566,8 @@ __global__ void __launch_bounds__(kMaxBlock, (min_waves<T, RS>())) k_y(YFields<T
   const int l = tid & (f.nl - 1);
   const long e = long(xcd_tile()) * f.nl + l;
   const bool in = e < nlines;
-  const long plane = in ? e / nkx : 0;
+  // (a 64-bit division only where the count needs it)
+  const long plane = !in ? 0 : (nlines >> 32 ? e / nkx : long(unsigned(e) / unsigned(nkx)));
   const long base = plane * nkx * ny + (in ? e - plane * nkx : 0);
   const bool cont = forward && Cy > 0;
   const int nload = cont ? npy : ny;
@@ -2349,9 +2350,13 @@ static int with_xy(const LineFFTHost& f, F&& fn) {
 // Two workgroups per CU: one step's kernels at limits of 0 / 256 / 512 / 1024 take
 // 241 / 192 / 192 / 192 us for HD 32^3, 324 / 310 / 285 / 284 for 64^3, 572 / 565 / 559
 // / 554 for 96x120x77, 95 / 90 / 84 / 86 for the 160x120x103 transforms.
+// The engine's Rader and Bluestein lines keep theirs: a workgroup stages their filter
+// and index tables too, which fewer threads do more slowly (x transforms of
+// 54x50x71 10.3 -> 9.9 us back, 10.6 -> 10.4 forward, without this).
 constexpr long kSpread = 512;
 static inline LineFFTHost spread(const LineFFTHost& f, long lines, long fields, int least) {
   int nl = f.nl;
+  if (f.wave < 0 && f.mode != 0) return f;
   while (nl > least && nl * f.tpl > 64 && (lines + nl - 1) / nl * fields < kSpread) nl >>= 1;
   return f.with_lines(nl);
 }
