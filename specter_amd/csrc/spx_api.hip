@@ -1064,16 +1064,46 @@ int spx_a_imposebc_and_project(spx_plan* p, void* ax, void* ay, void* az, void* 
 // launch for the terms, one for the sums and one copy of the results (a copy of
 // every line and a host sum per term took half of hdcheck's and vdiagnostic's
 // time at 128^3).  out[value][member]; per values per line.
+// Few values are added on the host, in k_line_sum's order (the same bits): a third
+// kernel costs more than their copy (divergence of 32 x 32 x 57, 544 values: 35.3 us
+// with the kernel, 32.8 so; enstrophy with 3920 values 37.4 and 38.9).
+constexpr size_t kHostSums = 2048;
+// what one workgroup of k_line_sum makes of a member's nl lines
+static double line_sum_host(const double* part, const double* w, int nterm, int per,
+                            size_t term, size_t nl, size_t ny) {
+#pragma clang fp contract(off)
+  double a[kHostSums], red[1024];
+  for (size_t l = 0; l < nl; ++l) a[l] = 0.0 + w[0] * part[l * per];
+  for (int t = 1; t < nterm; ++t)
+    for (size_t l = 0; l < nl; ++l) a[l] += w[t] * part[(t * term + l) * per];
+  for (size_t l = std::min(nl, ny); l < nl; ++l) a[l] = 2.0 * a[l];
+  // (the threads without a line add zeros)
+  size_t n = 1;
+  while (n < nl && n < 1024) n *= 2;
+  for (size_t i = 0; i < n; ++i) red[i] = i < nl ? 0.0 + a[i] : 0.0;
+  for (size_t l = 1024; l < nl; ++l) red[l & 1023] += a[l];
+  for (size_t q = n / 2; q > 0; q /= 2)
+    for (size_t i = 0; i < q; ++i) red[i] += red[i + q];
+  return red[0];
+}
 static int member_sums(spx_plan* p, int nterm, const double* w, int per, double* out0,
                        double* out1, double scale) {
-  const size_t from = 4 * size_t(p->wlines());
+  const size_t lines = size_t(p->wlines()), nl = lines / p->nact, ny = p->g.ny;
+  double* const out[2] = {out0, out1};
   int rc;
-  if ((rc = line_sums(p, nterm, w, per, p->part, p->part + from))) return rc;
-  if ((rc = fetch_parts(p, size_t(per) * p->nact, from))) return rc;
-  for (int m = 0; m < p->nact; ++m) {
-    out0[m] = p->h_part[m] * scale;
-    if (per == 2) out1[m] = p->h_part[p->nact + m] * scale;
+  if (nterm * per * lines > kHostSums) {
+    const size_t from = 4 * lines;
+    if ((rc = line_sums(p, nterm, w, per, p->part, p->part + from))) return rc;
+    if ((rc = fetch_parts(p, size_t(per) * p->nact, from))) return rc;
+    for (int v = 0; v < per; ++v)
+      for (int m = 0; m < p->nact; ++m) out[v][m] = p->h_part[v * p->nact + m] * scale;
+    return SPX_OK;
   }
+  if ((rc = fetch_parts(p, nterm * per * lines))) return rc;
+  for (int v = 0; v < per; ++v)
+    for (int m = 0; m < p->nact; ++m)
+      out[v][m] = scale * line_sum_host(p->h_part.data() + m * nl * per + v, w, nterm, per, lines,
+                                        nl, ny);
   return SPX_OK;
 }
 

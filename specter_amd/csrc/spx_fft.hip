@@ -1732,10 +1732,10 @@ __global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(ZTerms<TS> terms, in
                                                       const double* __restrict__ ky,
                                                       const double* __restrict__ kz) {
 #pragma clang fp contract(off)
+  const LinCombDev<TS> lc = terms.lc[blockIdx.y];
+  const cpx<TS>* __restrict__ bsrc = terms.b[blockIdx.y];
   SPX_PROLOGUE(Cd, f);
   const int n = f.n;
-  const LinCombDev<TS>& lc = terms.lc[blockIdx.y];
-  const cpx<TS>* __restrict__ bsrc = terms.b[blockIdx.y];
   double* __restrict__ out = outs + blockIdx.y * nlines * (mode == 3 ? 4 : (mode == 2 ? 2 : 1));
   Cd* const ldsB = lds + f.nl * f.ldl;
   Cd* const xb = ldsB + line * f.ldl;
@@ -1749,6 +1749,7 @@ __global__ void __launch_bounds__(kMaxBlock) k_zline_reduce(ZTerms<TS> terms, in
     if (ok) {
       const double kxi = kx[i], kyj = ky[j], kzk = kz[k];
       v = deriv_apply(ccast<double>(lc.in[0][ln * n + k]), lc.dir[0], kxi, kyj, kzk);
+#pragma unroll
       for (int t = 1; t < 3; ++t) {
         if (lc.sgn[t] == 0) continue;
         const Cd u = deriv_apply(ccast<double>(lc.in[t][ln * n + k]), lc.dir[t], kxi, kyj, kzk);
@@ -3161,8 +3162,8 @@ static int zline_launch(spx_plan* p, int nterm, const LinComb* lc, const void* c
                         double* out) {
   if (nterm < 1 || nterm > 3) return fail(SPX_ERR_ARG, "zline_reduce: 1..3 terms");
   const LineFFTHost& fw = fzt(p, false);
-  const LineFFTHost f = mode == 1 ? fw.with_lines(fw.nl / 2) : fw;
   const long nlines = p->wlines();
+  const LineFFTHost f = spread(mode == 1 ? fw.with_lines(fw.nl / 2) : fw, nlines, nterm, 1);
   ZTerms<double> d;
   for (int q = 0; q < 3; ++q) {
     const LinComb& c = lc[q < nterm ? q : 0];
