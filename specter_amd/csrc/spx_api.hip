@@ -1065,8 +1065,8 @@ int spx_a_imposebc_and_project(spx_plan* p, void* ax, void* ay, void* az, void* 
 // every line and a host sum per term took half of hdcheck's and vdiagnostic's
 // time at 128^3).  out[value][member]; per values per line.
 // Few values are added on the host, in k_line_sum's order (the same bits): a third
-// kernel costs more than their copy (divergence of 32 x 32 x 57, 544 values: 35.3 us
-// with the kernel, 32.8 so; enstrophy with 3920 values 37.4 and 38.9).
+// kernel costs more than their copy (544 values, divergence of 32 x 32 x 57: 2 us of
+// 35 more; 4000 values, wall checks of 48 x 40 x 57: 1 us less).
 constexpr size_t kHostSums = 2048;
 // what one workgroup of k_line_sum makes of a member's nl lines
 static double line_sum_host(const double* part, const double* w, int nterm, int per,
